@@ -68,22 +68,25 @@ typedef struct qesmc_fields {
 } qesmc_fields;
 
 /* Kernel path selection (qesmc_params.path). */
-#define QESMC_PATH_AUTO 0     /* fastest available: FUSED where the colour
-                                 arrays exceed the 256 MB Infinity Cache and
-                                 the run allows it (wall mask, below 2^31
-                                 half-cells, its
-                                 buffers already allocated in a
-                                 qesmc_run_static call), SPLIT otherwise        */
+#define QESMC_PATH_AUTO 0     /* fastest available.  On a wall mask: whole
+                                 iterations per launch, as FUSED, unless the
+                                 tile fields or qesmc_autotune tile the colour
+                                 passes, or its second lambda buffer cannot be
+                                 had (no memory, or not yet allocated in a
+                                 qesmc_run_static call); else SPLIT.  Reported
+                                 as FUSED where the colour arrays exceed the
+                                 256 MB Infinity Cache, as SPLIT otherwise     */
 #define QESMC_PATH_PLAIN 1    /* in-place red/black launches on the x-fastest
                                  layout, full fp32 coefficients: the classic
                                  GPU red-black SOR (baseline)                   */
-#define QESMC_PATH_SPLIT 2    /* colour-split (checkerboard) layout, per-cell
-                                 6-bit wall mask when the coefficients are
-                                 stair-step, full coefficients otherwise        */
-#define QESMC_PATH_FUSED 3    /* colour-split layout and wall mask, both colour
-                                 passes of an iteration in one launch (two
-                                 lambda buffers); stair-step coefficients only,
-                                 else QESMC_ERR_UNSUPPORTED                     */
+#define QESMC_PATH_SPLIT 2    /* colour-split (checkerboard) layout, a launch
+                                 per colour, per-cell 6-bit wall mask when the
+                                 coefficients are stair-step, full
+                                 coefficients otherwise                         */
+#define QESMC_PATH_FUSED 3    /* wall mask, both colours of two iterations in
+                                 one launch (two lambda buffers); stair-step
+                                 coefficients only, else
+                                 QESMC_ERR_UNSUPPORTED                          */
 
 typedef struct qesmc_params {
   float omega;      /* over-relaxation, reference 1.78f (Solver.h:83)          */
@@ -95,8 +98,8 @@ typedef struct qesmc_params {
   int check_every;  /* host polls convergence every this many iterations (>=1);
                        results never depend on it                             */
   int flags;        /* QESMC_RUN_* bits                                        */
-  int tile_k;       /* k planes marched by one SOR wave tile (0 = library's
-                       choice)                                                */
+  int tile_k;       /* split path: k planes marched by one SOR wave tile; fused
+                       path: planes per segment (0 = library's choice)        */
   int tile_v;       /* split path: half-cells per lane, 1, 2 or 4 (0 = choice) */
   int wg_per_cu;    /* split path: resident work-groups per CU (0 = choice)    */
   int slab_planes;  /* split path: k-slab of the interleaved red/black schedule

@@ -18,19 +18,25 @@
 
 #include "qesmc_internal.h"
 
-hipError_t qesmc_launch_divergence(qesmc_ctx *x, bool split, int alpha1);
+hipError_t qesmc_launch_divergence(qesmc_ctx *x, int layout, int alpha1);
 hipError_t qesmc_launch_stencil_encode(qesmc_ctx *x);
 hipError_t qesmc_launch_split_coefs(qesmc_ctx *x);
 hipError_t qesmc_launch_pack(qesmc_ctx *x, bool to_split);
-hipError_t qesmc_launch_unpack_selected(qesmc_ctx *x);
+hipError_t qesmc_launch_pack_pairs(qesmc_ctx *x, bool to_pairs);
+hipError_t qesmc_launch_march(qesmc_ctx *x, int t, int iters, int itermax, const float *om, float tol, int src,
+                              bool fix);
+hipError_t qesmc_march_settle(qesmc_ctx *x, int lo, int hi, float tol);
 hipError_t qesmc_launch_iteration(qesmc_ctx *x, int path, bool masked, int t, int itermax, float omega_red,
                                   float omega_black, float tol);
 hipError_t qesmc_launch_finish(qesmc_ctx *x, bool mirror, int alpha1, int alpha2);
 hipError_t qesmc_launch_div_linf(qesmc_ctx *x, int physical);
 hipError_t qesmc_launch_set_u32(qesmc_ctx *x, unsigned *p, unsigned v);
+hipError_t qesmc_launch_run_init(qesmc_ctx *x, long long rows, unsigned extend);
 hipError_t qesmc_launch_fill_u32(qesmc_ctx *x, unsigned *p, long long count, unsigned v);
 hipError_t qesmc_launch_rows_summary(qesmc_ctx *x, int launched, float tol);
 hipError_t qesmc_fused_prepare(qesmc_ctx *x);
+long long qesmc_march_top_words(const qesmc::Dims &d);
+void qesmc_march_choose(qesmc_ctx *x, int tile_k, const int *top);
 
 namespace {
 
@@ -66,6 +72,21 @@ void dfree(T *&p)
   p = nullptr;
 }
 
+// Both colours' arrays in one allocation: p[1] = p[0] + count.
+hipError_t dalloc2(float **p, long long count)
+{
+  p[1] = nullptr;
+  const hipError_t e = dalloc(&p[0], 2 * count);
+  if (e == hipSuccess && p[0]) p[1] = p[0] + count;
+  return e;
+}
+
+void dfree2(float **p)
+{
+  dfree(p[0]);
+  p[1] = nullptr;
+}
+
 void free_geometry(qesmc_ctx *x)
 {
   for (auto &p : x->d_coef) dfree(p);
@@ -81,15 +102,18 @@ void free_geometry(qesmc_ctx *x)
   dfree(x->d_lam);
   dfree(x->d_grad);
   x->have_velocity = false;
+  dfree2(x->d_lc);
+  dfree2(x->d_Rc);
+  dfree2(x->d_lc2);
+  dfree2(x->d_R0);
+  dfree2(x->d_base);
   for (int c = 0; c < 2; ++c) {
-    dfree(x->d_lc[c]);
-    dfree(x->d_Rc[c]);
     dfree(x->d_mask[c]);
-    dfree(x->d_lc2[c]);
-    dfree(x->d_R0[c]);
-    dfree(x->d_base[c]);
     for (auto &p : x->d_cc[c]) dfree(p);
   }
+  dfree(x->d_mask2);
+  dfree(x->d_top);
+  x->pair_masks = false;
   dfree(x->d_canon);
   dfree(x->d_canon8);
   x->have_geom = x->have_inflow = false;
@@ -132,11 +156,9 @@ int alloc_geometry(qesmc_ctx *x, int nx, int ny, int nz)
   HIPCHK(dalloc(&x->d_w, x->nface));
   HIPCHK(dalloc(&x->d_R, x->ncell));
   HIPCHK(dalloc(&x->d_lam, x->ncell));
-  for (int c = 0; c < 2; ++c) {
-    HIPCHK(dalloc(&x->d_lc[c], x->nsplit));
-    HIPCHK(dalloc(&x->d_Rc[c], x->nsplit));
-    HIPCHK(dalloc(&x->d_mask[c], x->nsplit));
-  }
+  HIPCHK(dalloc2(x->d_lc, x->nsplit));
+  HIPCHK(dalloc2(x->d_Rc, x->nsplit));
+  for (int c = 0; c < 2; ++c) HIPCHK(dalloc(&x->d_mask[c], x->nsplit));
   HIPCHK(dalloc(&x->d_canon, 6LL * d.NZ));
   HIPCHK(hipMemsetAsync(x->d_lam, 0, sizeof(float) * x->ncell, x->stream));
   return QESMC_OK;
@@ -148,6 +170,7 @@ int encode_stencil(qesmc_ctx *x)
 {
   HIPCHK(hipMemsetAsync(x->d_status, 0, sizeof(unsigned), x->stream));
   HIPCHK(hipMemsetAsync(x->d_canon, 0, sizeof(unsigned) * 6 * x->d.NZ, x->stream));
+  x->pair_masks = false;
   HIPCHK(qesmc_launch_stencil_encode(x));
   unsigned *hst = x->h_poll + 2 * qesmc::kErrSlots;
   HIPCHK(hipMemcpyAsync(hst, x->d_status, sizeof(unsigned), hipMemcpyDeviceToHost, x->stream));
@@ -359,7 +382,7 @@ float row_max(const unsigned *row)
 
 // Validation, optional re-encoding, tiling, convergence rows, lambda packing
 // and R, on the context's current stream (ev[0] .. ev[1]).
-int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st)
+int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, bool batch)
 {
   if (!x || !pp) return QESMC_ERR_ARG;
   if (!x->have_geom || !x->have_inflow) return QESMC_ERR_STATE;
@@ -384,20 +407,39 @@ int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st)
     if (rc != QESMC_OK) return rc;
   }
   st.masked = x->compressible;
-  // QESMC_PATH_AUTO: the two-colour march where the colour arrays (lambda and
-  // R of both colours, the masks) exceed MI355X's 256 MB Infinity Cache, so
-  // that each iteration streams them from HBM, and where it applies (wall
-  // mask, 32-bit offsets, its buffers available without allocating in a
-  // no-allocation run); the split kernel otherwise.
-  // Measured: 568 against 626 us per iteration on 1000 x 1000 x 150; 64
-  // against 58 us on 400 x 400 x 120, whose arrays stay in the cache.
+  const bool march_ready = x->d_lc2[0] && x->d_cur && x->d_canon8 && x->d_mask2 && x->d_top;
+  // QESMC_PATH_AUTO is reported as FUSED where the colour arrays (lambda and
+  // R of both colours, the masks) exceed MI355X's 256 MB Infinity Cache, as
+  // SPLIT otherwise
   if (p.path == QESMC_PATH_AUTO && st.masked &&
       x->nsplit < (1LL << 31) && (double)x->nsplit * 2.0 * (4.0 + 4.0 + 1.0) > 256.0 * (1 << 20) &&
-      (!x->no_alloc_run || (x->d_lc2[0] && x->d_lc2[1] && x->d_cur && x->d_canon8)))
+      (!x->no_alloc_run || march_ready))
     st.path = QESMC_PATH_FUSED;
   if (st.path == QESMC_PATH_FUSED && !st.masked) return QESMC_ERR_UNSUPPORTED;
-  // the fused march addresses its arrays with 32-bit element offsets
+  // the fused path addresses its arrays with 32-bit element offsets
   if (st.path == QESMC_PATH_FUSED && x->nsplit >= (1LL << 31)) return QESMC_ERR_UNSUPPORTED;
+  // The march (two iterations per launch) runs wherever it can: on every wall
+  // mask, unless the caller or the autotuner tiles the colour passes, a
+  // no-allocation run finds its buffers missing, or a plane is beyond its
+  // 32-bit byte offsets.
+  st.march = !batch && x->d.splane < (1LL << 28) && x->d.NZ < 32768 &&
+             (st.path == QESMC_PATH_FUSED ||
+              (p.path == QESMC_PATH_AUTO && st.masked && x->nsplit < (1LL << 31) && p.tile_k == 0 &&
+               p.tile_v == 0 && p.wg_per_cu == 0 && p.slab_planes == 0 && x->kplanes_auto == 0 &&
+               x->tile_v_auto == 0 && x->wg_per_cu_auto == 0 && (!x->no_alloc_run || march_ready)));
+  if (st.march && !march_ready) {
+    hipError_t e = hipSuccess;
+    if (!x->d_lc2[0]) e = dalloc2(x->d_lc2, x->nsplit);
+    if (e == hipSuccess && !x->d_cur) e = dalloc(&x->d_cur, 1);
+    if (e == hipSuccess && !x->d_canon8) e = dalloc(&x->d_canon8, (8LL + 64LL) * x->d.NZ);
+    if (e == hipSuccess && !x->d_mask2) e = dalloc(&x->d_mask2, (long long)((x->d.NY + 1) / 2) * x->d.HP * x->d.NZ);
+    if (e == hipSuccess && !x->d_top) e = dalloc(&x->d_top, qesmc_march_top_words(x->d));
+    if (e != hipSuccess) {
+      if (st.path == QESMC_PATH_FUSED) return map_hip(e);
+      (void)hipGetLastError();
+      st.march = false;  // no room for a second lambda: the colour passes need none
+    }
+  }
   x->kplanes = p.tile_k > 0 ? p.tile_k : x->kplanes_auto;
   x->tile_v = p.tile_v > 0 ? p.tile_v : x->tile_v_auto;
   if (x->kplanes == 0 || x->tile_v == 0) {
@@ -447,18 +489,11 @@ int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st)
     x->kplanes = p.tile_k > 0 ? p.tile_k : 8;
     x->tile_v = 1;
     x->wg_per_cu = 0;
-    for (int c = 0; c < 2; ++c)
-      if (!x->d_lc2[c]) HIPCHK(dalloc(&x->d_lc2[c], x->nsplit));
-    if (!x->d_cur) HIPCHK(dalloc(&x->d_cur, 1));
-    if (!x->d_canon8) HIPCHK(dalloc(&x->d_canon8, 8LL * x->d.NZ));
-    HIPCHK(qesmc_fused_prepare(x));
   }
   if (p.refine_every > 0) {
     // base lambda and the run's R, besides the correction and the residual
-    for (int c = 0; c < 2; ++c) {
-      if (!x->d_base[c]) HIPCHK(dalloc(&x->d_base[c], x->nsplit));
-      if (!x->d_R0[c]) HIPCHK(dalloc(&x->d_R0[c], x->nsplit));
-    }
+    if (!x->d_base[0]) HIPCHK(dalloc2(x->d_base, x->nsplit));
+    if (!x->d_R0[0]) HIPCHK(dalloc2(x->d_R0, x->nsplit));
   }
 
   const long long rows = (long long)p.itermax + 1;
@@ -471,27 +506,34 @@ int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st)
   }
   hipStream_t s = x->stream;
   HIPCHK(hipEventRecord(x->ev[0], s));
-  HIPCHK(qesmc_launch_fill_u32(x, x->d_status, 1, 0u));
-  // the stop rule: no end recorded yet, and the extension factor (0 for the
-  // reference's rule) that every kernel's gate reads
+  // status words and convergence rows: no end recorded yet, the extension
+  // factor (0 for the reference's rule) that every kernel's gate reads, and
+  // row 0 at 1.0f
   {
     unsigned ext;
     std::memcpy(&ext, &p.stop_extend, 4);
-    HIPCHK(qesmc_launch_fill_u32(x, x->d_status + kStopAt, 1, 0xffffffffu));
-    HIPCHK(qesmc_launch_fill_u32(x, x->d_status + kStopExtend, 1, ext));
+    HIPCHK(qesmc_launch_run_init(x, rows, ext));
   }
-  HIPCHK(qesmc_launch_fill_u32(x, x->d_err, rows * kErrSlots, 0u));
-  HIPCHK(qesmc_launch_set_u32(x, x->d_err, 0x3f800000u));  // row 0: 1.0f
-  if (st.path != QESMC_PATH_PLAIN) HIPCHK(qesmc_launch_pack(x, true));
-  if (st.path == QESMC_PATH_FUSED) {
-    // both buffer sets start equal: cells that are never relaxed keep their
-    // values in both, and iteration 0 reads set 0
-    for (int c = 0; c < 2; ++c)
-      HIPCHK(hipMemcpyAsync(x->d_lc2[c], x->d_lc[c], sizeof(float) * (size_t)x->nsplit, hipMemcpyDeviceToDevice, s));
+  if (st.march) {
+    if (!x->pair_masks) {
+      HIPCHK(qesmc_fused_prepare(x));
+      x->pair_masks = true;
+      x->march_tile_k = -1;
+    }
+    if (x->march_tile_k != p.tile_k) {
+      std::vector<int> top((size_t)qesmc_march_top_words(x->d));
+      HIPCHK(hipMemcpyAsync(top.data(), x->d_top, sizeof(int) * top.size(), hipMemcpyDeviceToHost, s));
+      HIPCHK(hipStreamSynchronize(s));
+      qesmc_march_choose(x, p.tile_k, top.data());
+      x->march_tile_k = p.tile_k;
+    }
+    HIPCHK(qesmc_launch_pack_pairs(x, true));
     HIPCHK(qesmc_launch_set_u32(x, x->d_cur, 0u));
+  } else if (st.path != QESMC_PATH_PLAIN) {
+    HIPCHK(qesmc_launch_pack(x, true));
   }
-  HIPCHK(qesmc_launch_divergence(x, st.path != QESMC_PATH_PLAIN, p.alpha1));
-  if (p.refine_every > 0) HIPCHK(refine_setup(x, st.masked, st.path == QESMC_PATH_FUSED));
+  HIPCHK(qesmc_launch_divergence(x, st.march ? 2 : st.path != QESMC_PATH_PLAIN ? 1 : 0, p.alpha1));
+  if (p.refine_every > 0) HIPCHK(refine_setup(x, st.masked, st.march));
   HIPCHK(hipEventRecord(x->ev[1], s));
   st.first_runs = p.itermax > 0 && (1.0f > p.tol);
   return QESMC_OK;
@@ -504,8 +546,8 @@ int run_finish(qesmc_ctx *x, const RunState &st, int launched, qesmc_result *res
   const qesmc_params &p = st.p;
   hipStream_t s = x->stream;
   HIPCHK(hipEventRecord(x->ev[2], s));
-  if (st.path == QESMC_PATH_SPLIT) HIPCHK(qesmc_launch_pack(x, false));
-  if (st.path == QESMC_PATH_FUSED) HIPCHK(qesmc_launch_unpack_selected(x));
+  if (st.march) HIPCHK(qesmc_launch_pack_pairs(x, false));
+  else if (st.path != QESMC_PATH_PLAIN) HIPCHK(qesmc_launch_pack(x, false));
   HIPCHK(qesmc_launch_finish(x, st.first_runs, p.alpha1, p.alpha2));
   HIPCHK(hipEventRecord(x->ev[3], s));
   // iteration t ran iff max(row t) > tol: the count and the last residual are
@@ -585,28 +627,44 @@ int run_loop(qesmc_ctx *x, const RunState &st, int *launched_out)
     };
     if (p.chebyshev_rho > 0.0)
       for (long long h = 0; h < 2LL * p.chebyshev_start && !fixed; ++h) (void)next_omega();
-    for (int t = 0; t < p.itermax && !stop; ++t) {
-      float w_red = p.omega, w_black = p.omega;
-      if (p.chebyshev_rho > 0.0) {
-        w_red = next_omega();
-        w_black = next_omega();
+    int src = 0;      // the march's buffer set that holds lambda
+    int settled = 0;  // rows the march's end has been looked for in
+    for (int t = 0; t < p.itermax && !stop;) {
+      // the march takes two iterations per launch, up to the next refresh
+      int iters = 1;
+      if (st.march && t + 2 <= p.itermax && !(p.refine_every > 0 && (t + 1) % p.refine_every == 0)) iters = 2;
+      float om[4];
+      for (int h = 0; h < 2 * iters; ++h) om[h] = p.chebyshev_rho > 0.0 ? next_omega() : p.omega;
+      hipError_t e;
+      if (st.march) {
+        e = qesmc_launch_march(x, t, iters, p.itermax, om, p.tol, src, false);
+        src ^= 1;
+      } else {
+        e = qesmc_launch_iteration(x, st.path, st.masked, t, p.itermax, om[0], om[1], p.tol);
       }
-      hipError_t e = qesmc_launch_iteration(x, st.path, st.masked, t, p.itermax, w_red, w_black, p.tol);
       if (e != hipSuccess) {
         rc = map_hip(e);
         break;
       }
-      ++launched;
-      if (p.refine_every > 0 && (t + 1) % p.refine_every == 0 && t + 1 < p.itermax &&
-          (e = refine_refresh(x, st.masked, st.path == QESMC_PATH_FUSED)) != hipSuccess) {
-        rc = map_hip(e);
-        break;
+      const int before = t;
+      t += iters;
+      launched = t;
+      if (p.refine_every > 0 && t % p.refine_every == 0 && t < p.itermax) {
+        if (st.march) {
+          e = qesmc_march_settle(x, settled, t, p.tol);
+          settled = t;
+        }
+        if (e == hipSuccess) e = refine_refresh(x, st.masked, st.march);
+        if (e != hipSuccess) {
+          rc = map_hip(e);
+          break;
+        }
       }
-      if ((t + 1) % p.check_every == 0 && t + 1 < p.itermax) {
+      if (t / p.check_every != before / p.check_every && t < p.itermax) {
         const int slot = chunk & 1;
         unsigned *dst = x->h_poll + slot * qesmc::kErrSlots;
         if (chunk >= 2 && (e = hipEventSynchronize(x->ev[4 + slot])) != hipSuccess) { rc = map_hip(e); break; }
-        e = hipMemcpyAsync(dst, x->d_err + (long long)(t + 1) * qesmc::kErrSlots,
+        e = hipMemcpyAsync(dst, x->d_err + (long long)t * qesmc::kErrSlots,
                            sizeof(unsigned) * qesmc::kErrSlots, hipMemcpyDeviceToHost, s);
         // the production rule's recorded end (all ones until fixed)
         unsigned *end_h = x->h_poll + 2 * qesmc::kErrSlots + 4 + slot;
@@ -619,13 +677,17 @@ int run_loop(qesmc_ctx *x, const RunState &st, int *launched_out)
           if ((e = hipEventSynchronize(x->ev[4 + prev])) != hipSuccess) { rc = map_hip(e); break; }
           if (p.stop_extend > 0.f) {
             // every iteration from the recorded end on is a no-op
-            if (x->h_poll[2 * qesmc::kErrSlots + 4 + prev] <= (unsigned)(t + 1)) stop = true;
+            if (x->h_poll[2 * qesmc::kErrSlots + 4 + prev] <= (unsigned)t) stop = true;
           } else if (!(qesmc::row_max(x->h_poll + prev * qesmc::kErrSlots) > p.tol)) {
             stop = true;
           }
         }
         ++chunk;
       }
+    }
+    if (rc == QESMC_OK && st.march) {
+      const hipError_t e = qesmc_march_settle(x, settled, launched, p.tol);
+      if (e != hipSuccess) rc = map_hip(e);
     }
     if (rc != QESMC_OK) (void)hipStreamSynchronize(s);
   }
@@ -644,7 +706,7 @@ int run_solve(qesmc_ctx *x, const qesmc_params *pp, qesmc_result *res)
   rc = run_loop(x, st, &launched);
   if (rc != QESMC_OK) return rc;
   if (st.p.refine_every > 0) {
-    hipError_t e = refine_fold_final(x, st.path == QESMC_PATH_FUSED);
+    hipError_t e = refine_fold_final(x, st.march);
     if (e != hipSuccess) return map_hip(e);
   }
   return qesmc::run_finish(x, st, launched, res);

@@ -296,7 +296,7 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
   };
   std::vector<RunState> st(n);
   int rc = QESMC_OK;
-  for (int i = 0; i < n && rc == QESMC_OK; ++i) rc = run_prepare(ctxs[i], params, st[i]);
+  for (int i = 0; i < n && rc == QESMC_OK; ++i) rc = run_prepare(ctxs[i], params, st[i], true);
   if (rc != QESMC_OK) {
     (void)hipStreamSynchronize(bs);
     restore();

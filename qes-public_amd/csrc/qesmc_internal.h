@@ -40,10 +40,21 @@ enum : unsigned {
 
 // Words of ctx->d_status: [0] status bits, [1..3] convergence-row summary
 // of the last run, [4] the production stop rule's end iteration (all ones
-// until fixed), [5] its extension factor (float bits, 0 = reference rule).
-constexpr int kStatusWords = 8;
+// until fixed), [5] its extension factor (float bits, 0 = reference rule),
+// [6] the march: earliest launch that left a non-finite lambda, as the last
+// iteration it covers (all ones: none); [7] the iteration the run ended at,
+// as far as it has been looked for (all ones: open), [8..9] first iteration
+// and iterations of the last launch that ran, [10] its first iteration is to
+// be redone alone, [11..12] that iteration's omega, red and black.
+constexpr int kStatusWords = 16;
 constexpr int kStopAt = 4;
 constexpr int kStopExtend = 5;
+constexpr int kBadAt = 6;
+constexpr int kEnd = 7;
+constexpr int kLastT = 8;
+constexpr int kLastIters = 9;
+constexpr int kFixGo = 10;
+constexpr int kLastOmega = 11;
 
 // Iteration gate, decided identically by every wave of a launch.  g is the
 // max of convergence row t (the previous iteration's max|dlambda|, 1.0 for
@@ -76,6 +87,32 @@ __device__ inline bool gate_pass(float g, int t, float tol, unsigned *status)
 // XCD on one address serialise at the memory side, so they are spread.
 constexpr int kErrSlots = 64;
 
+// The gate of a launch of several iterations starting at t, decided
+// identically by every wave: t runs iff every iteration before it did and
+// row t passes.  The launch before held at most two iterations, so rows t-1
+// and t are looked at (an earlier stop leaves both at zero).  With the
+// production rule the recorded end is either unset or what this wave finds
+// from the same rows, so the decision cannot differ between waves.
+__device__ inline bool gate_pass_multi(const unsigned *err, int t, float tol, unsigned *status, int lane)
+{
+  const float ext = __uint_as_float(status[kStopExtend]);
+  const unsigned recorded = *(volatile unsigned *)(status + kStopAt);
+  unsigned end = recorded;
+  for (int r = t > 0 ? t - 1 : 0; r <= t; ++r) {
+    float g = __uint_as_float(err[(long long)r * kErrSlots + lane]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) g = fmaxf(g, __shfl_xor(g, off, 64));
+    if (!(ext > 0.f)) {
+      if (!(g > tol)) return false;
+    } else if ((unsigned)r < end && !(g > tol)) {
+      end = min(end, (unsigned)r + (unsigned)ceilf(ext * (float)r));
+    }
+  }
+  if (!(ext > 0.f)) return true;
+  if (end < recorded && lane == 0 && threadIdx.x < 64) atomicMin(status + kStopAt, end);
+  return (unsigned)t < end;
+}
+
 // Grid constants passed by value to every kernel.
 //   nx, ny, nz : staggered sizes (qes::Domain)
 //   NX, NY, NZ : cell counts per axis = nx-1, ny-1, nz-1
@@ -87,6 +124,14 @@ struct Dims {
   long long sy, sz;    // cell strides (NX, NX*NY)
   long long fy, fz;    // face strides (nx, nx*ny)
   long long splane;    // split-layout plane stride NY*HP
+};
+
+// Tiling of the march: a shape of its table, the columns of tiles and the
+// segments of planes.
+constexpr int kMarchMaxSegments = 127;
+struct MarchPlan {
+  int shape = 0, nq = 1, nyt = 1, nseg = 0;
+  short begin[kMarchMaxSegments + 1] = {};  // first plane of each segment (odd), then the end
 };
 
 }  // namespace qesmc
@@ -119,15 +164,20 @@ struct qesmc_ctx {
   float *d_probe_val = nullptr; // gathered u, v, w of the probes (3 x n_probe)
   long long n_probe = 0, probe_cap = 0, probe_nface = 0;
 
-  // colour-split arrays (index = colour)
+  // colour-split arrays (index = colour).  Both colours' arrays are one
+  // allocation ([1] = [0] + nsplit); the march reads the same memory in the
+  // pair layout, 2 * nsplit floats from [0].
   float *d_lc[2] = {};
   float *d_Rc[2] = {};
   unsigned char *d_mask[2] = {};
+  unsigned *d_mask2 = nullptr; // march: both colours' masks in the pair layout, two rows a word (allocated on first use)
+  int *d_top = nullptr;        // march: highest plane with a wall, per two rows and 32 pairs
+  bool pair_masks = false;           // d_mask2, d_top and d_canon8 hold the resident geometry's
   float *d_cc[2][6] = {};     // full coefficients, split (only if not compressible)
   unsigned *d_canon = nullptr; // 6*NZ wall values per layer (float bits)
-  unsigned *d_canon8 = nullptr; // fused path: the same, 8 words per layer (6 used), layer-major
-  float *d_lc2[2] = {};       // second lambda buffer set of the fused path (allocated on first use)
-  unsigned *d_cur = nullptr;   // fused path: buffer set holding the latest iterate (0: d_lc, 1: d_lc2)
+  unsigned *d_canon8 = nullptr; // march: the same, 8 words per layer (6 used), layer-major, then 64 sums per layer
+  float *d_lc2[2] = {};       // second lambda buffer set of the march (allocated on first use)
+  unsigned *d_cur = nullptr;   // march: buffer set holding the latest iterate (0: d_lc, 1: d_lc2)
   float *d_R0[2] = {};        // refine_every: R of the run (d_Rc then holds the residual of the base)
   float *d_base[2] = {};      // refine_every: the base lambda (the iterates hold the correction)
 
@@ -146,6 +196,8 @@ struct qesmc_ctx {
   int wg_per_cu_auto = 0;      // 0: chosen per run from tile_v
   int slab_planes = 0;         // split path: k-slab of the interleaved red/black schedule (this run; 0: whole passes)
   int slab_planes_auto = 0;    // default when qesmc_params.slab_planes == 0
+  qesmc::MarchPlan march[2];   // tiling of the march's launches of one and of two iterations
+  int march_tile_k = -1;       // the tile_k they were chosen for (-1: not chosen)
   int n_cu = 256;              // compute units of the device
 };
 
@@ -156,20 +208,23 @@ struct RunState {
   qesmc_params p{};
   int path = QESMC_PATH_SPLIT;
   bool masked = false;
+  bool march = false;       // whole iterations per launch on the pair layout
   bool first_runs = false;
 };
-int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st);
+// batch: prepared for qesmc_run_batch, which relaxes a colour per launch
+int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, bool batch = false);
 int run_finish(qesmc_ctx *x, const RunState &st, int launched, qesmc_result *res);
 int run_solve(qesmc_ctx *x, const qesmc_params *pp, qesmc_result *res);
 int run_loop(qesmc_ctx *x, const RunState &st, int *launched);
 // refine_every: set up base = lambda, R0 = R, R = residual of base, delta
 // = 0 (refine_setup); fold delta into base and re-form the residual
 // (refine_refresh); lambda = base + delta at the end (refine_fold_final).
-// With `fused` the correction lives in whichever buffer set the march wrote
-// last (d_cur, read on the device); otherwise in d_lc.
-hipError_t refine_setup(qesmc_ctx *x, bool masked, bool fused);
-hipError_t refine_refresh(qesmc_ctx *x, bool masked, bool fused);
-hipError_t refine_fold_final(qesmc_ctx *x, bool fused);
+// With `march` the arrays are in the pair layout and the correction lives in
+// whichever buffer set the march wrote last (d_cur, read on the device);
+// otherwise in d_lc.
+hipError_t refine_setup(qesmc_ctx *x, bool masked, bool march);
+hipError_t refine_refresh(qesmc_ctx *x, bool masked, bool march);
+hipError_t refine_fold_final(qesmc_ctx *x, bool march);
 // Whether the resident flags hold a cut cell (7 or 8).
 hipError_t find_cut_cells(qesmc_ctx *x, bool *cut);
 int static_scratch_init(int device);

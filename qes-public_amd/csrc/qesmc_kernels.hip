@@ -67,7 +67,8 @@ __device__ inline void publish_delta(unsigned *err, int t, float bm)
 // ---------------------------------------------------------------------------
 // R: divergence of u0 (Solver_CPU_RB.cpp:56-80), k in [1, nz-3]
 // ---------------------------------------------------------------------------
-template <bool SPLIT>
+// LAYOUT 0: x-fastest R; 1: colour-split R0, R1; 2: pair layout (R0).
+template <int LAYOUT>
 __global__ __launch_bounds__(256) void k_divergence(Dims d, float dx, float dy,
                                                     const float *__restrict__ dz,
                                                     const float *__restrict__ e,
@@ -93,10 +94,12 @@ __global__ __launch_bounds__(256) void k_divergence(Dims d, float dx, float dy,
                          + ((g[c] * v0[fc + d.fy] - h[c] * v0[fc]) * dy)
                          + ((m[c] * dzk * 0.5 * (dzk + dzp) * w0[fc + d.fz]
                              - n[c] * dzk * 0.5f * (dzk + dzm) * w0[fc])));
-  if (SPLIT) {
+  const long long row = (long long)(k * d.NY + j) * d.HP;
+  if (LAYOUT == 1) {
     const int colour = (i + j + k) & 1;
-    const long long s = (long long)(k * d.NY + j) * d.HP + (i >> 1);
-    (colour ? R1 : R0)[s] = r;
+    (colour ? R1 : R0)[row + (i >> 1)] = r;
+  } else if (LAYOUT == 2) {
+    R0[2 * row + i] = r;
   } else {
     R[c] = r;
   }
@@ -255,22 +258,30 @@ __global__ __launch_bounds__(256) void k_pack(Dims d, const float *__restrict__ 
   (((i + j + k) & 1) ? l1 : l0)[s] = lam[c];
 }
 
-// split -> natural from the buffer set the fused path left its last iterate in
-__global__ __launch_bounds__(256) void k_unpack_selected(Dims d, float *__restrict__ lam,
-                                                         const float *__restrict__ a0,
-                                                         const float *__restrict__ a1,
-                                                         const float *__restrict__ b0,
-                                                         const float *__restrict__ b1,
-                                                         const unsigned *__restrict__ cur)
+// natural -> pair layout (cell i of row (j,k) at 2*row + i), both buffer sets
+// of the march: cells that are never relaxed keep their values in both
+__global__ __launch_bounds__(256) void k_pack_pairs(Dims d, const float *__restrict__ lam, float *__restrict__ a,
+                                                    float *__restrict__ b)
 {
   const int i = blockIdx.x * 64 + threadIdx.x;
   const int j = blockIdx.y * 4 + threadIdx.y;
   const int k = blockIdx.z;
   if (i >= d.NX || j >= d.NY) return;
-  const long long c = i + (long long)j * d.sy + k * d.sz;
-  const long long s = (long long)(k * d.NY + j) * d.HP + (i >> 1);
-  const bool odd = (i + j + k) & 1;
-  lam[c] = (*cur ? (odd ? b1 : b0) : (odd ? a1 : a0))[s];
+  const float v = lam[i + (long long)j * d.sy + k * d.sz];
+  const long long s = 2 * ((long long)(k * d.NY + j) * d.HP) + i;
+  a[s] = v;
+  b[s] = v;
+}
+
+// pair layout -> natural, from the set the march left its last iterate in
+__global__ __launch_bounds__(256) void k_unpack_pairs(Dims d, float *__restrict__ lam, const float *__restrict__ a,
+                                                      const float *__restrict__ b, const unsigned *__restrict__ cur)
+{
+  const int i = blockIdx.x * 64 + threadIdx.x;
+  const int j = blockIdx.y * 4 + threadIdx.y;
+  const int k = blockIdx.z;
+  if (i >= d.NX || j >= d.NY) return;
+  lam[i + (long long)j * d.sy + k * d.sz] = (*cur ? b : a)[2 * ((long long)(k * d.NY + j) * d.HP) + i];
 }
 
 __global__ __launch_bounds__(256) void k_unpack(Dims d, float *__restrict__ lam,
@@ -413,6 +424,19 @@ __global__ __launch_bounds__(256) void k_fill_u32(unsigned *__restrict__ p, long
   for (long long q = blockIdx.x * 256LL + threadIdx.x; q < count; q += stride) p[q] = v;
 }
 
+// Start of a run: the status words and the convergence rows, in one launch.
+__global__ __launch_bounds__(256) void k_run_init(unsigned *__restrict__ status, unsigned extend,
+                                                  unsigned *__restrict__ rows, long long words)
+{
+  if (blockIdx.x == 0 && threadIdx.x < kStatusWords) {
+    const int w = threadIdx.x;
+    status[w] = w == kStopAt || w == kBadAt || w == kEnd ? 0xffffffffu : w == kStopExtend ? extend : 0u;
+  }
+  const long long stride = (long long)gridDim.x * 256;
+  // row 0 is the reference's initial max_error, 1.0f
+  for (long long q = blockIdx.x * 256LL + threadIdx.x; q < words; q += stride) rows[q] = q == 0 ? 0x3f800000u : 0u;
+}
+
 // The largest entry of one convergence row read as floats, NaN never winning
 // (the host's reading of a row).
 __device__ inline float row_max_dev(const unsigned *row)
@@ -439,13 +463,15 @@ __global__ __launch_bounds__(256) void k_rows_first_stop(const unsigned *__restr
 // recorded, if below), out[1] = bits of the max of row out[0]: the last
 // executed iteration's max|dlambda| (the sentinel 1.0 if none ran).
 __global__ void k_rows_summary(const unsigned *__restrict__ rows, const unsigned *__restrict__ first,
-                               const unsigned *__restrict__ status, int launched, unsigned *__restrict__ out)
+                               unsigned *status, int launched, unsigned *out)
 {
   unsigned count = *first;
   if (__uint_as_float(status[kStopExtend]) > 0.f) {
     const unsigned end = status[kStopAt];
     count = end < (unsigned)launched ? end : (unsigned)launched;
   }
+  // a launch of the march that the run ended inside was redone up to the end
+  if (status[kBadAt] < count) status[0] |= ST_NONFINITE;
   out[0] = count;
   out[1] = __float_as_uint(row_max_dev(rows + (long long)count * kErrSlots));
 }
@@ -464,26 +490,25 @@ static const unsigned kPlaneBlocks = 8;  // work-groups per plane of the plane r
 
 using namespace qesmc;
 
-hipError_t qesmc_launch_fused_iteration(qesmc_ctx *x, int t, int itermax, float omega_red, float omega_black,
-                                        float tol);
 hipError_t qesmc_launch_split_iteration(qesmc_ctx *x, bool masked, int t, int itermax, float omega_red,
                                         float omega_black, float tol);
 
 // Entry points used by the API translation unit.
-hipError_t qesmc_launch_divergence(qesmc_ctx *x, bool split, int alpha1)
+// layout: 0 x-fastest, 1 colour-split, 2 pairs
+hipError_t qesmc_launch_divergence(qesmc_ctx *x, int layout, int alpha1)
 {
   const Dims &d = x->d;
   if (d.NZ - 2 < 1) return hipSuccess;
   const double pre = -2.0f * pow((double)alpha1, 2.0);
-  dim3 gr = grid_xy(d.NX, d.NY, d.NZ - 2);
-  if (split)
-    hipLaunchKernelGGL(k_divergence<true>, gr, kBlock, 0, x->stream, d, x->dx, x->dy, x->d_dz,
-                       x->d_coef[0], x->d_coef[1], x->d_coef[2], x->d_coef[3], x->d_coef[4],
-                       x->d_coef[5], x->d_u0, x->d_v0, x->d_w0, pre, x->d_R, x->d_Rc[0], x->d_Rc[1]);
-  else
-    hipLaunchKernelGGL(k_divergence<false>, gr, kBlock, 0, x->stream, d, x->dx, x->dy, x->d_dz,
-                       x->d_coef[0], x->d_coef[1], x->d_coef[2], x->d_coef[3], x->d_coef[4],
-                       x->d_coef[5], x->d_u0, x->d_v0, x->d_w0, pre, x->d_R, x->d_Rc[0], x->d_Rc[1]);
+  const dim3 gr = grid_xy(d.NX, d.NY, d.NZ - 2);
+#define QESMC_DIV_LAUNCH(L)                                                                                        \
+  hipLaunchKernelGGL(k_divergence<L>, gr, kBlock, 0, x->stream, d, x->dx, x->dy, x->d_dz, x->d_coef[0],            \
+                     x->d_coef[1], x->d_coef[2], x->d_coef[3], x->d_coef[4], x->d_coef[5], x->d_u0, x->d_v0,       \
+                     x->d_w0, pre, x->d_R, x->d_Rc[0], x->d_Rc[1])
+  if (layout == 2) QESMC_DIV_LAUNCH(2);
+  else if (layout == 1) QESMC_DIV_LAUNCH(1);
+  else QESMC_DIV_LAUNCH(0);
+#undef QESMC_DIV_LAUNCH
   return hipGetLastError();
 }
 
@@ -521,15 +546,18 @@ hipError_t qesmc_launch_pack(qesmc_ctx *x, bool to_split)
   return hipGetLastError();
 }
 
-hipError_t qesmc_launch_unpack_selected(qesmc_ctx *x)
+hipError_t qesmc_launch_pack_pairs(qesmc_ctx *x, bool to_pairs)
 {
   const Dims &d = x->d;
-  hipLaunchKernelGGL(k_unpack_selected, grid_xy(d.NX, d.NY, d.NZ), kBlock, 0, x->stream, d, x->d_lam, x->d_lc[0],
-                     x->d_lc[1], x->d_lc2[0], x->d_lc2[1], x->d_cur);
+  const dim3 gr = grid_xy(d.NX, d.NY, d.NZ);
+  if (to_pairs)
+    hipLaunchKernelGGL(k_pack_pairs, gr, kBlock, 0, x->stream, d, x->d_lam, x->d_lc[0], x->d_lc2[0]);
+  else
+    hipLaunchKernelGGL(k_unpack_pairs, gr, kBlock, 0, x->stream, d, x->d_lam, x->d_lc[0], x->d_lc2[0], x->d_cur);
   return hipGetLastError();
 }
 
-// Iteration t: the red pass at omega_red, the black pass at omega_black.
+// Iteration t, a launch per colour: the red pass at omega_red, the black pass at omega_black.
 hipError_t qesmc_launch_iteration(qesmc_ctx *x, int path, bool masked, int t, int itermax,
                                   float omega_red, float omega_black, float tol)
 {
@@ -544,8 +572,6 @@ hipError_t qesmc_launch_iteration(qesmc_ctx *x, int path, bool masked, int t, in
                          x->d_coef[1], x->d_coef[2], x->d_coef[3], x->d_coef[4], x->d_coef[5],
                          x->d_R, x->d_lam, omega, 1.0f - omega, tol, x->d_err, t, itermax, x->d_status);
     }
-  } else if (path == QESMC_PATH_FUSED) {
-    return qesmc_launch_fused_iteration(x, t, itermax, omega_red, omega_black, tol);
   } else {
     return qesmc_launch_split_iteration(x, masked, t, itermax, omega_red, omega_black, tol);
   }
@@ -593,6 +619,14 @@ hipError_t qesmc_launch_fill_u32(qesmc_ctx *x, unsigned *p, long long count, uns
   long long blocks = (count + 255) / 256;
   if (blocks > 4096) blocks = 4096;
   hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)blocks), dim3(256), 0, x->stream, p, count, v);
+  return hipGetLastError();
+}
+
+hipError_t qesmc_launch_run_init(qesmc_ctx *x, long long rows, unsigned extend)
+{
+  const long long words = rows * kErrSlots, blocks = (words + 255) / 256;
+  hipLaunchKernelGGL(k_run_init, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, x->stream, x->d_status,
+                     extend, x->d_err, words);
   return hipGetLastError();
 }
 

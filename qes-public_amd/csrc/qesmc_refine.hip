@@ -81,6 +81,39 @@ __global__ __launch_bounds__(256) void k_refine_residual(Dims d, int colour, con
   }
 }
 
+// The same on the pair layout (cell i of row (j,k) at 2*row + i), both colours,
+// one pair per thread.
+__global__ __launch_bounds__(256) void k_refine_residual_pairs(Dims d, const float *__restrict__ base, const float *Rin,
+                                                               float *Rout, const unsigned *__restrict__ mask,
+                                                               const unsigned *__restrict__ canon8)
+{
+  const long long pitch = 2LL * d.HP, plane = 2 * d.splane;
+  const long long n = d.splane * d.NZ;
+  const long long stride = (long long)gridDim.x * 256;
+  for (long long x = blockIdx.x * 256LL + threadIdx.x; x < n; x += stride) {
+    const int k = (int)(x / d.splane);
+    const int rem = (int)(x - (long long)k * d.splane);
+    const int j = rem / d.HP, q = rem - j * d.HP;
+    if (k < 1 || k > d.NZ - 2 || j < 1 || j > d.NY - 2) continue;
+    const unsigned mm = mask[((long long)k * ((d.NY + 1) / 2) + j / 2) * d.HP + q] >> (16 * (j & 1));
+#pragma unroll
+    for (int o = 0; o < 2; ++o) {
+      const int i = 2 * q + o;
+      if (i < 1 || i > d.NX - 2) continue;
+      const long long f = 2 * x + o;
+      double c[6];
+#pragma unroll
+      for (int a = 0; a < 6; ++a)
+        c[a] = (mm >> (8 * o + 2 + a)) & 1u ? (double)__uint_as_float(canon8[8 * k + a]) : 0.0;
+      const double sum = c[0] * (double)base[f + 1] + c[1] * (double)base[f - 1] + c[2] * (double)base[f + pitch] +
+                         c[3] * (double)base[f - pitch] + c[4] * (double)base[f + plane] +
+                         c[5] * (double)base[f - plane];
+      const double D = ((c[0] + c[1]) + (c[2] + c[3])) + (c[4] + c[5]);
+      Rout[f] = (float)((double)Rin[f] + D * (double)base[f] - sum);
+    }
+  }
+}
+
 // dst += src over one colour array (every position: the ring and the
 // planes that are never relaxed hold zero in the correction).  With cur the
 // buffer set *cur selects (dst1 / src1 for set 1) stands for the one the
@@ -116,15 +149,32 @@ __global__ __launch_bounds__(256) void k_refine_mirror(Dims d, int colour, float
   }
 }
 
+// The same on the pair layout.
+__global__ __launch_bounds__(256) void k_refine_mirror_pairs(Dims d, float *__restrict__ base)
+{
+  const long long n = 2 * d.splane;
+  const long long stride = (long long)gridDim.x * 256;
+  for (long long f = blockIdx.x * 256LL + threadIdx.x; f < n; f += stride) {
+    const int j = (int)(f / (2 * d.HP)), i = (int)(f - 2LL * d.HP * j);
+    if (j < 1 || j > d.NY - 2 || i < 1 || i > d.NX - 2) continue;
+    base[f] = base[f + n];
+  }
+}
+
 unsigned grid_for(long long n)
 {
   const long long b = (n + 255) / 256;
   return (unsigned)(b < 8192 ? (b < 1 ? 1 : b) : 8192);
 }
 
-hipError_t residual(qesmc_ctx *x, bool masked, float *const *base, float *const *Rin)
+hipError_t residual(qesmc_ctx *x, bool masked, bool march, float *const *base, float *const *Rin)
 {
   const unsigned g = grid_for(x->nsplit);
+  if (march) {
+    hipLaunchKernelGGL(k_refine_residual_pairs, dim3(g), dim3(256), 0, x->stream, x->d, base[0], Rin[0], x->d_Rc[0],
+                       x->d_mask2, x->d_canon8);
+    return hipGetLastError();
+  }
   for (int c = 0; c < 2; ++c) {
     const float *const *cc = x->d_cc[c];
     if (masked)
@@ -140,36 +190,32 @@ hipError_t residual(qesmc_ctx *x, bool masked, float *const *base, float *const 
   return hipSuccess;
 }
 
-// the correction = 0: d_lc, and with `fused` both of the march's buffer sets
-hipError_t zero_correction(qesmc_ctx *x, bool fused)
+// the correction = 0: d_lc, and with `march` both of its buffer sets (each
+// both colours' arrays, one allocation)
+hipError_t zero_correction(qesmc_ctx *x, bool march)
 {
-  for (int set = 0; set < (fused ? 2 : 1); ++set)
-    for (int c = 0; c < 2; ++c) {
-      float *a = set ? x->d_lc2[c] : x->d_lc[c];
-      const hipError_t e = qesmc_launch_fill_u32(x, reinterpret_cast<unsigned *>(a), x->nsplit, 0u);
-      if (e != hipSuccess) return e;
-    }
-  return hipSuccess;
-}
-
-// base += correction (to_base) or correction += base, over both colour
-// arrays; the correction is the march's latest buffer set with `fused`
-hipError_t add(qesmc_ctx *x, bool to_base, bool fused)
-{
-  const unsigned g = grid_for(x->nsplit);
-  const unsigned *cur = fused ? x->d_cur : nullptr;
-  for (int c = 0; c < 2; ++c) {
-    float *d0 = x->d_lc[c], *d1 = fused ? x->d_lc2[c] : x->d_lc[c];
-    if (to_base)
-      hipLaunchKernelGGL(k_refine_add, dim3(g), dim3(256), 0, x->stream, x->nsplit, x->d_base[c], x->d_base[c],
-                         (const float *)d0, (const float *)d1, cur);
-    else
-      hipLaunchKernelGGL(k_refine_add, dim3(g), dim3(256), 0, x->stream, x->nsplit, d0, d1,
-                         (const float *)x->d_base[c], (const float *)x->d_base[c], cur);
-    const hipError_t e = hipGetLastError();
+  for (int set = 0; set < (march ? 2 : 1); ++set) {
+    float *a = set ? x->d_lc2[0] : x->d_lc[0];
+    const hipError_t e = qesmc_launch_fill_u32(x, reinterpret_cast<unsigned *>(a), 2 * x->nsplit, 0u);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
+}
+
+// base += correction (to_base) or correction += base, over both colours; the
+// correction is the march's latest buffer set with `march`
+hipError_t add(qesmc_ctx *x, bool to_base, bool march)
+{
+  const unsigned *cur = march ? x->d_cur : nullptr;
+  float *d0 = x->d_lc[0], *d1 = march ? x->d_lc2[0] : x->d_lc[0], *base = x->d_base[0];
+  const long long n = 2 * x->nsplit;
+  if (to_base)
+    hipLaunchKernelGGL(k_refine_add, dim3(grid_for(n)), dim3(256), 0, x->stream, n, base, base, (const float *)d0,
+                       (const float *)d1, cur);
+  else
+    hipLaunchKernelGGL(k_refine_add, dim3(grid_for(n)), dim3(256), 0, x->stream, n, d0, d1, (const float *)base,
+                       (const float *)base, cur);
+  return hipGetLastError();
 }
 
 }  // namespace
@@ -178,37 +224,38 @@ namespace qesmc {
 
 // After R: base = lambda (d_lc; the march's second set holds the same), R0
 // = R, R = residual of base, delta = 0.
-hipError_t refine_setup(qesmc_ctx *x, bool masked, bool fused)
+hipError_t refine_setup(qesmc_ctx *x, bool masked, bool march)
 {
-  const size_t bytes = sizeof(float) * (size_t)x->nsplit;
-  for (int c = 0; c < 2; ++c) {
-    hipError_t e = hipMemcpyAsync(x->d_R0[c], x->d_Rc[c], bytes, hipMemcpyDeviceToDevice, x->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(x->d_base[c], x->d_lc[c], bytes, hipMemcpyDeviceToDevice, x->stream);
-    if (e != hipSuccess) return e;
-  }
-  hipError_t e = residual(x, masked, x->d_base, x->d_R0);
-  return e == hipSuccess ? zero_correction(x, fused) : e;
+  const size_t bytes = 2 * sizeof(float) * (size_t)x->nsplit;
+  hipError_t e = hipMemcpyAsync(x->d_R0[0], x->d_Rc[0], bytes, hipMemcpyDeviceToDevice, x->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(x->d_base[0], x->d_lc[0], bytes, hipMemcpyDeviceToDevice, x->stream);
+  if (e == hipSuccess) e = residual(x, masked, march, x->d_base, x->d_R0);
+  return e == hipSuccess ? zero_correction(x, march) : e;
 }
 
 // Between iterations: base += delta, the base's k = 0 mirror, R = residual
 // of base, delta = 0.
-hipError_t refine_refresh(qesmc_ctx *x, bool masked, bool fused)
+hipError_t refine_refresh(qesmc_ctx *x, bool masked, bool march)
 {
-  hipError_t e = add(x, true, fused);
+  hipError_t e = add(x, true, march);
   if (e != hipSuccess) return e;
   const unsigned g = grid_for(x->d.splane);
-  for (int c = 0; c < 2; ++c) {
-    hipLaunchKernelGGL(k_refine_mirror, dim3(g), dim3(256), 0, x->stream, x->d, c, x->d_base[c],
-                       (const float *)x->d_base[c ^ 1]);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+  if (march) {
+    hipLaunchKernelGGL(k_refine_mirror_pairs, dim3(grid_for(2 * x->d.splane)), dim3(256), 0, x->stream, x->d,
+                       x->d_base[0]);
+  } else {
+    for (int c = 0; c < 2; ++c)
+      hipLaunchKernelGGL(k_refine_mirror, dim3(g), dim3(256), 0, x->stream, x->d, c, x->d_base[c],
+                         (const float *)x->d_base[c ^ 1]);
   }
-  e = residual(x, masked, x->d_base, x->d_R0);
-  return e == hipSuccess ? zero_correction(x, fused) : e;
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  e = residual(x, masked, march, x->d_base, x->d_R0);
+  return e == hipSuccess ? zero_correction(x, march) : e;
 }
 
 // lambda = base + delta, in the set that holds delta (the one the unpacking
 // reads).
-hipError_t refine_fold_final(qesmc_ctx *x, bool fused) { return add(x, false, fused); }
+hipError_t refine_fold_final(qesmc_ctx *x, bool march) { return add(x, false, march); }
 
 }  // namespace qesmc
 

@@ -1,51 +1,56 @@
-// Red-black SOR with both colour passes of an iteration in one launch, on
-// the colour-split layout with the wall-mask stencil (QESMC_PATH_FUSED).
+// Red-black SOR with whole iterations in one launch: T iterations (2 T colour
+// passes) of a column tile are pipelined along k, on the pair layout with the
+// wall-mask stencil (QESMC_PATH_FUSED, and what QESMC_PATH_AUTO runs on a
+// wall-mask geometry).
 //
-// Iteration t reads lambda from buffer set A = t & 1 and writes buffer set
-// B = A ^ 1 (each set holds both colours), so no wave ever reads a value
-// another wave of the same launch writes.  The result is the reference's
-// in-place schedule (src/winds/Solver_CPU_RB.cpp:109-162) exactly: a red
-// cell sees the old black values, a black cell the new red ones, and after
-// the iteration lambda(i,j,0) = lambda(i,j,1) — written here straight into
-// B's plane 0 when a k = 1 cell is relaxed.  Cells that are never updated
-// (the domain's ring, planes 0 and NZ-1) hold the same values in both sets.
+// Layout.  The pair layout stores row (j,k) as HP pairs, pair q holding the
+// cells i = 2q and 2q+1: x = (k*NY + j)*HP + q, one 8-byte pair of lambda
+// and of R and one 2-byte pair of wall masks per index.  A pair holds one red
+// and one black cell; which is which alternates with j + k.
 //
-// Work decomposition: one wave per column tile, marching along j.  A wave
-// owns W <= 62 consecutive half-cells q of a row (lanes 1..W; lanes 0 and
-// W+1 hold the half-cells just outside, whose red values it recomputes as
-// their owner does), the K planes [k0, k0+K) and the rows [j0, j1) of a
-// segment.  Step j (for j = j0-1 .. j1) relaxes the red cells of row j over
-// planes k0-1 .. k0+K (a halo plane each side) from the black values of A
-// in rows j-1..j+1, then the black cells of row j-1 over the wave's own
-// planes, whose six red neighbours (rows j-2..j, planes k-1..k+1, and the
-// x-neighbours in the adjacent lanes) are all in registers.  Each black row
-// of A is loaded once, as row j+1, and kept while the march passes it.
-// The halos are recomputed rather than exchanged, and the tiles that share
-// them are dispatched together so that the re-reads mostly hit in L2: the
-// four waves of a work-group are x-neighbours (a 58-lane row segment is not
-// line aligned, so neighbours share cache lines), the k-neighbours a few
-// work-groups on.  Per iteration a cell costs its own lambda read and
-// write, R and the mask: 13 bytes per update, against 17 in a split colour
-// pass (which also reads the other colour's lambda), plus the halo re-reads
-// (K+4 black planes loaded per K relaxed, W+2 lanes per W, L+2 red rows per
-// L).  The factor
-// omega / (e+f+g+h+m+n) of a cell depends only on its layer and its 6-bit
-// mask, so each wave tabulates it for its planes in LDS (with the same
-// expression, hence the same value) instead of dividing per cell; with the
-// coefficients selected by bit masks this took a quarter of the march's
-// vector instructions away.  On grids beyond the Infinity Cache the march
-// is bound by its HBM traffic, about 1.25 x 13 bytes per update with the
-// halos, against 1.17 x 17 for the split passes:
-// QESMC_PATH_AUTO picks it there and the split kernel where the arrays stay
-// in the cache, whose bandwidth the split passes use better.
-#include "qesmc_sor_tile.h"
+// A launch reads lambda from one buffer set and writes the other, so no
+// work-group reads what another writes.  The result is the reference's
+// in-place schedule (src/winds/Solver_CPU_RB.cpp:109-162) exactly: every
+// half-sweep sees the other colour as the schedule leaves it, and after each
+// iteration lambda(i,j,0) = lambda(i,j,1).
+//
+// Work decomposition.  A work-group of NW waves owns a tile of 64 half-cells
+// (one per lane) by NW*RW rows (RW rows per wave) and a segment of planes, and
+// marches up k.  Step p relaxes, for h = 0 .. 2T-1, half-sweep h (red for
+// even h) of plane p-h: its z-neighbours are half-sweep h-1's planes p-h+1 (just
+// relaxed) and p-h-1, its y-neighbours half-sweep h-1's values of plane p-h,
+// relaxed one step earlier, so the rows at the edge of a wave's block are
+// exchanged through LDS once per step (one barrier), and the x-neighbour
+// outside the pair comes from the adjacent lane (DPP).  Everything else stays
+// in registers: a window of planes per row in which each half-sweep replaces
+// its colour in place.  The window is a ring whose slots are static because
+// the step loop is unrolled over the ring, which also makes every parity
+// (j+k) static: tiles start on even rows and segments on odd planes.
+// The tiles overlap by a halo that is relaxed redundantly: 2T rows and T
+// half-cells on each inner side, 2T planes at each inner segment end.
+//
+// Per launch a cell moves 4 (lambda) + 4 (R) + 1 (mask) bytes in and 4 out plus
+// the halo's re-reads, for T iterations: at T = 2 half of what one iteration
+// per launch moves.  omega / (e+f+g+h+m+n) depends only on the layer and
+// the 6-bit mask and is tabulated per plane in LDS with the same expression
+// (one wave per half-sweep, one mask per lane), and where all masks of a wave's
+// rows are open (no wall: most of a city's planes) the six coefficients are
+// the layer's wall values themselves, in scalar registers.
+#include <cstring>
+#include <type_traits>
+#include <vector>
+
+#include "qesmc_internal.h"
+
+hipError_t qesmc_launch_fill_u32(qesmc_ctx *x, unsigned *p, long long count, unsigned v);
 
 namespace qesmc {
 
 namespace {
 
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, work-groups dispatched round-robin
-constexpr int kWaves = 4; // waves (tiles) per work-group
+constexpr int kMaxSegments = kMarchMaxSegments;
+constexpr unsigned kOpenRows = 0xfcfcfcfcu;  // the pairs of two rows without walls
 
 __device__ inline float wave_max(float v)
 {
@@ -54,315 +59,698 @@ __device__ inline float wave_max(float v)
   return v;
 }
 
-// Wall value a of a layer (its bit pattern cb) where mask bit a is set, +0
-// where it is not: the bit sign-extended to a word and ANDed with the value.
-template <int A>
-__device__ __forceinline__ float wall_coef(unsigned m, unsigned cb)
+// The value of the lane below (FROM = -1) or above (FROM = 1); 0 past the wave's ends.
+template <int FROM>
+__device__ __forceinline__ float lane_shift(float v)
 {
-  return __uint_as_float(cb & (unsigned)((int)(m << (31 - A)) >> 31));
+  constexpr int ctrl = FROM < 0 ? 0x138 : 0x130;  // wave_shr:1 / wave_shl:1
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xf, 0xf, true));
 }
 
-// relax() of qesmc_sor_tile.h with its factor omega / (e+f+g+h+m+n) read
-// from a table (wd, computed by the same expression) instead of divided per
-// cell: the same operations on the same values, so the same result.
-__device__ __forceinline__ float relax_tab(unsigned m, const unsigned *cb, float wd, float xp, float xm, float yp,
-                                           float ym, float zp, float zm, float r, float o, float one_m_omega)
+// m = max(m, |v|); a NaN never wins, as in the reference's max test.  (fmaxf
+// would first canonicalise m, which is never a signalling NaN.)
+__device__ __forceinline__ void max_abs(float &m, float v) { asm("v_max_f32 %0, %0, |%1|" : "+v"(m) : "v"(v)); }
+
+// LDS writes of this wave visible to the work-group before the barrier, LDS
+// reads after it; global loads and stores in flight are left in flight.
+__device__ __forceinline__ void lds_barrier()
 {
-  const float ec = wall_coef<0>(m, cb[0]), fc = wall_coef<1>(m, cb[1]), gc = wall_coef<2>(m, cb[2]),
-              hc = wall_coef<3>(m, cb[3]), mc = wall_coef<4>(m, cb[4]), nc = wall_coef<5>(m, cb[5]);
-  return wd * (ec * xp + fc * xm + gc * yp + hc * ym + mc * zp + nc * zm - r) + one_m_omega * o;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
+
+// Bit `bit` of a mask word, sign-extended, and the byte from `bit` up (a mask
+// times 4: the byte offset of its table entry).
+// Written out because the compiler would keep every bit of a mask as a
+// condition (a scalar register pair each) or an extended word from one
+// half-sweep to the next of the same cell, and spill.
+__device__ __forceinline__ unsigned mask_bit(unsigned m, unsigned bit)
+{
+  unsigned r;
+  asm volatile("v_bfe_i32 %0, %1, %2, 1" : "=v"(r) : "v"(m), "n"(bit));
+  return r;
+}
+
+__device__ __forceinline__ unsigned mask_index(unsigned m, unsigned bit)
+{
+  unsigned r;
+  asm volatile("v_bfe_u32 %0, %1, %2, 8" : "=v"(r) : "v"(m), "n"(bit));
+  __builtin_assume(r < 256u);
+  return r;
+}
+
+// Buffer descriptor over `bytes` bytes at a wave-uniform address: a load or
+// store then takes one lane offset and one scalar offset, and what falls past
+// the end reads 0 or is dropped.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *p, unsigned bytes)
+{
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00027000);
+}
+
+typedef unsigned uint2v __attribute__((ext_vector_type(2)));
+
+struct MarchArgs {
+  Dims d;
+  int nq, nyt;        // x tiles, y tiles
+  int ntiles;
+  float2 *set0, *set1;  // lambda, the two buffer sets
+  const float2 *R;
+  const unsigned *mask;
+  const int *top;     // highest plane with a wall, per two rows and 32 pairs
+  const unsigned *canon8;  // wall values per plane, 8 words (6 used)
+  const float *sums;       // sum of the wall values each of the 64 masks selects, per plane
+  float om[4];        // omega of each half-sweep (2T used)
+  float tol;
+  unsigned *err;
+  int t, itermax;
+  unsigned *status;
+  unsigned *cur;      // the set holding the latest iterate
+  int src;            // set this launch reads
+  int fix;            // redo the last launch's first iteration if asked to (T = 1 only)
+  short begin[kMaxSegments + 1];  // first plane of each segment (odd), then the end
+};
 
 }  // namespace
 
-template <int K>
-__global__ __launch_bounds__(256, 3) void k_sor_march(Dims d, int W, int qt, int L, int nkc, long long ntiles,
-                                                   const float *__restrict__ a0, const float *__restrict__ a1,
-                                                   float *__restrict__ b0, float *__restrict__ b1,
-                                                   const float *__restrict__ R0, const float *__restrict__ R1,
-                                                   const unsigned char *__restrict__ mask0,
-                                                   const unsigned char *__restrict__ mask1,
-                                                   const unsigned *__restrict__ canon8, float omega_r,
-                                                   float omo_r, float omega_b, float omo_b, float tol, unsigned *err,
-                                                   int t,
-                                                   int itermax, unsigned *status, unsigned *cur)
+// T iterations per launch, NW waves per work-group, RW rows (even) per row
+// group, GW lanes per row group (64: a wave is one group; 32: two).
+template <int T, int NW, int RW, int GW>
+__global__ __launch_bounds__(64 * NW, RW == 2 ? 4 : 2) void k_sor_march(MarchArgs A)
 {
-  constexpr int NB = K + 4;  // black-old plane slots: planes k0-2 .. k0+K+1
-  constexpr int NR = K + 2;  // red plane slots: planes k0-1 .. k0+K
-  __shared__ float wmax[kWaves];
-  // per wave, colour (red, black) and relaxed plane k0-1+p: omega / (sum of
-  // the wall values a cell's mask selects), for each of the 64 masks, and
-  // the six wall values
-  __shared__ float wd_tab[kWaves][2][NR][64];
-  __shared__ unsigned cv_tab[kWaves][NR][8];
+  constexpr int H = 2 * T;      // half-sweeps
+  constexpr int U = 2 * T + 4;  // ring slots (planes p-2T .. p+2 are live); even
+  constexpr int NG = NW * (64 / GW);  // row groups
+  constexpr int YR = NG * RW;   // rows of the tile
+  static_assert(RW % 2 == 0 && NW >= H && (T == 1 || T == 2), "");
+  // edge rows of each row group, per half-sweep that reads them: [buffer][h][first / last row][row group and lane]
+  __shared__ float edge[2][H][2][NW * 64];
+  __shared__ float wd_tab[2][H][64];
+  __shared__ __align__(16) unsigned cv_tab[2][H][8];
+  __shared__ float wmax[NW][T];
+  const Dims &d = A.d;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (t >= itermax) return;
-  {
-    // gate: iteration t runs iff max(err row t) > tol (row 0 = 1.0f)
-    const float g = wave_max(__uint_as_float(err[(long long)t * kErrSlots + lane]));
-    if (!gate_pass(g, t, tol, status)) return;  // identical in every wave of the grid
-  }
-  // XCD x (work-group id % 8) takes the x-th eighth of the work-group range;
-  // tiles are numbered x-tile fastest, so the 4 waves of a work-group are
-  // x-neighbours in one k-chunk and row segment and share the cache lines at
-  // their edges; the k-neighbours (sharing halo planes) follow qt tiles on
-  const long long per = (long long)gridDim.x / kXcds;  // the grid is a multiple of 8
-  const long long blk = (long long)(blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
-  if (blk == 0 && threadIdx.x == 0) *cur = (unsigned)((t + 1) & 1);
-  const long long tile = blk * kWaves + wave;
-  const int tq = (int)(tile % qt);
-  const long long tr = tile / qt;
-  const int tk = (int)(tr % nkc);
-  const long long tj = tr / nkc;
-  const bool valid = tile < ntiles;
-  {
-    // this wave's tables (planes clamped into the domain; a tile past the
-    // end fills harmless values it never reads)
-    const int k0t = 1 + tk * K;
-    for (int e = lane; e < NR * 64; e += 64) {
-      const int p = e >> 6, mm = e & 63;
-      int k = k0t - 1 + p;
-      k = k < 0 ? 0 : k > d.NZ - 1 ? d.NZ - 1 : k;
-      float v[6];
+  int t = A.t, src = A.src;
+  float om[H];
 #pragma unroll
-      for (int a = 0; a < 6; ++a) v[a] = ((mm >> a) & 1) ? __uint_as_float(canon8[k * 8 + a]) : 0.f;
-      const float sum = v[0] + v[1] + v[2] + v[3] + v[4] + v[5];
-      wd_tab[wave][0][p][mm] = omega_r / sum;
-      wd_tab[wave][1][p][mm] = omega_b / sum;
-    }
-    for (int e = lane; e < NR * 8; e += 64) {
-      const int p = e >> 3;
-      int k = k0t - 1 + p;
-      k = k < 0 ? 0 : k > d.NZ - 1 ? d.NZ - 1 : k;
-      cv_tab[wave][p][e & 7] = canon8[k * 8 + (e & 7)];
-    }
+  for (int h = 0; h < H; ++h) om[h] = A.om[h];
+  if (T == 1 && A.fix) {
+    // the last launch ran T iterations but the run ended inside it
+    if (!A.status[kFixGo]) return;
+    t = (int)A.status[kLastT];
+    src = (int)(A.cur[0] ^ 1u);
+    om[0] = __uint_as_float(A.status[kLastOmega]);
+    om[1] = __uint_as_float(A.status[kLastOmega + 1]);
+  } else {
+    if (t >= A.itermax) return;
   }
-  __syncthreads();
+  // XCD x (work-group id % 8) takes the x-th eighth of the tile range, tiles
+  // numbered x fastest, then y, then segment: neighbours that share halos
+  // march together on one L2
+  const int per = (int)gridDim.x / kXcds;  // the grid is a multiple of 8
+  const int tile = (int)(blockIdx.x % kXcds) * per + (int)(blockIdx.x / kXcds);
+  if (tile >= A.ntiles) return;
+  const int tq = tile % A.nq;
+  const int ty = (tile / A.nq) % A.nyt;
+  const int tz = tile / (A.nq * A.nyt);
 
-  float dl = 0.f;
+  // columns: this lane's half-cell, and whether this tile owns it
+  const int half = (d.NX + 1) >> 1;
+  const int gl = lane & (GW - 1);
+  const int q = tq * (GW - 2 * T) + gl;
+  const bool lown = q < half && (tq == 0 || gl >= T) && (tq == A.nq - 1 || gl < GW - T);
+  const unsigned qc = (unsigned)(q < half ? q : half - 1);
+  const bool col[2] = {q < half && 2 * q >= 1 && 2 * q <= d.NX - 2, 2 * q + 1 <= d.NX - 2};
+  // rows of this lane's group
+  const int group = (int)threadIdx.x / GW;
+  const int jt = ty * (YR - 4 * T);
+  const int j0 = jt + group * RW;
+  const int jown0 = ty == 0 ? 0 : jt + 2 * T;
+  const int jown1 = ty == A.nyt - 1 ? d.NY : jt + YR - 2 * T;
+  bool upd[RW][2], own[RW];
+  unsigned voff[RW], moff[RW / 2];  // byte offsets within a plane of lambda and R, of masks
+#pragma unroll
+  for (int a = 0; a < RW; ++a) {
+    const int j = j0 + a;
+    const unsigned jc = (unsigned)(j < d.NY ? j : d.NY - 1);
+    const bool ru = j >= 1 && j <= d.NY - 2;
+    upd[a][0] = ru && col[0];
+    upd[a][1] = ru && col[1];
+    own[a] = lown && j >= jown0 && j < jown1;
+    voff[a] = (jc * (unsigned)d.HP + qc) * 8u;
+    if (a % 2 == 0) moff[a / 2] = ((jc / 2u) * (unsigned)d.HP + qc) * 4u;
+  }
+  // planes: owned [ka, kb); half-sweep h relaxes [lo(h), hi(h)]
+  const int ka = A.begin[tz], kb = A.begin[tz + 1];
+  const int pfirst = ka - (H - 1) > 0 ? ka - (H - 1) : 0;  // even
+  const int plast = kb - 1 + (H - 1);
+  const float2 *__restrict__ in = src ? A.set1 : A.set0;
+  float2 *__restrict__ out = src ? A.set0 : A.set1;
+  const float2 *__restrict__ R = A.R;
+  const unsigned *__restrict__ mask = A.mask;
+  const unsigned *__restrict__ canon8 = A.canon8;
+  const float *__restrict__ sums = A.sums;
+  const unsigned plane8 = (unsigned)d.splane * 8u, planem = (unsigned)((d.NY + 1) / 2) * (unsigned)d.HP * 4u;
+  // this wave's half-sweep of the tables
+  float omw = om[0];
+#pragma unroll
+  for (int h = 1; h < H; ++h) omw = wave == h ? om[h] : omw;
+  auto clampk = [&](int k) -> int { return k < 0 ? 0 : k > d.NZ - 1 ? d.NZ - 1 : k; };
+
+  float W[RW][U][2];   // lambda
+  float G[RW][U][2];   // R
+  unsigned M[RW / 2][U];    // mask pairs of two rows
+  float dm[T][RW];
   bool bad = false;
-  if (valid) {  // wave-uniform, and no barrier inside
-    const int k0 = 1 + tk * K;
-    const int k1 = k0 + K < d.NZ - 1 ? k0 + K : d.NZ - 1;  // owned planes [k0, k1)
-    const int j0 = 1 + (int)tj * L;
-    const int j1 = j0 + L < d.NY - 1 ? j0 + L : d.NY - 1;  // owned rows [j0, j1)
-    // lanes past the right halo (W + 2 <= 64) repeat its address: they load
-    // nothing the wave does not already fetch, and own nothing
-    const int q = tq * W - 1 + (lane < W + 2 ? lane : W + 1);
-    const bool qv = q >= 0 && q < d.HP;
-    const unsigned qc = qv ? (unsigned)q : 0u;
-    const bool own = qv && lane >= 1 && lane <= W;
-    // the column i = 2q + s of this lane is updated (s: the cell's offset
-    // within its half-cell pair, (j + k + colour) & 1)
-    const bool col0 = qv && 2 * q >= 1 && 2 * q <= d.NX - 2;
-    const bool col1 = qv && 2 * q + 1 <= d.NX - 2;
-    // 32-bit element offsets (the launcher refuses arrays of 2^31 elements
-    // or more).  Every address is clamped into the domain, so loads need no
-    // predicate; values loaded for positions outside it are never used by
-    // an updated cell.
-    const unsigned HPu = (unsigned)d.HP, sp = (unsigned)d.splane;
-    auto row_off = [&](int j) -> unsigned {
-      const int jc = j < 0 ? 0 : j > d.NY - 1 ? d.NY - 1 : j;
-      return (unsigned)jc * HPu + qc;
-    };
-    auto plane_off = [&](int k) -> unsigned {
-      const int kc = k < 0 ? 0 : k > d.NZ - 1 ? d.NZ - 1 : k;
-      return (unsigned)kc * sp;
-    };
+#pragma unroll
+  for (int a = 0; a < RW; ++a)
+#pragma unroll
+    for (int s = 0; s < U; ++s) {
+      W[a][s][0] = W[a][s][1] = G[a][s][0] = G[a][s][1] = 0.f;
+      M[a / 2][s] = kOpenRows;
+    }
+#pragma unroll
+  for (int i = 0; i < T; ++i)
+#pragma unroll
+    for (int a = 0; a < RW; ++a) dm[i][a] = 0.f;
 
-    // black values of A, rows j-1 (bm), j (bc), j+1 (bp), planes k0-2+p
-    float bm[NB], bc[NB], bp[NB];
-    auto load_black = [&](int j, float *dst) {
-      const unsigned r = row_off(j);
+  auto load_lambda = [&](int k, int slot) {
+    const __amdgpu_buffer_rsrc_t pl =
+        buffer_of(reinterpret_cast<const char *>(in) + (unsigned long long)clampk(k) * plane8, plane8);
 #pragma unroll
-      for (int p = 0; p < NB; ++p) dst[p] = a1[r + plane_off(k0 - 2 + p)];
-    };
-    load_black(j0 - 2, bm);
-    load_black(j0 - 1, bc);
-    // new red values, rows j-2 (rm2), j-1 (rm1), j (rn), planes k0-1+p
-    float rm2[NR], rm1[NR], rn[NR];
+    for (int a = 0; a < RW; ++a) {
+      const uint2v v = __builtin_amdgcn_raw_buffer_load_b64(pl, voff[a], 0, 0);
+      W[a][slot][0] = __uint_as_float(v.x);
+      W[a][slot][1] = __uint_as_float(v.y);
+    }
+  };
+  auto load_rhs = [&](int k, int slot) {
+    const __amdgpu_buffer_rsrc_t pr =
+        buffer_of(reinterpret_cast<const char *>(R) + (unsigned long long)clampk(k) * plane8, plane8);
 #pragma unroll
-    for (int p = 0; p < NR; ++p) rm2[p] = rm1[p] = rn[p] = 0.f;
+    for (int a = 0; a < RW; ++a) {
+      const uint2v v = __builtin_amdgcn_raw_buffer_load_b64(pr, voff[a], 0, 0);
+      G[a][slot][0] = __uint_as_float(v.x);
+      G[a][slot][1] = __uint_as_float(v.y);
+    }
+  };
+  auto load_masks = [&](int k, int slot) {
+    const __amdgpu_buffer_rsrc_t pm =
+        buffer_of(reinterpret_cast<const char *>(mask) + (unsigned long long)clampk(k) * planem, planem);
+#pragma unroll
+    for (int a = 0; a < RW / 2; ++a) M[a][slot] = __builtin_amdgcn_raw_buffer_load_b32(pm, moff[a], 0, 0);
+  };
+  // the wall values of step p's planes and omega / (sum of those a mask
+  // selects): wave h for half-sweep h, the sums and values loaded a step
+  // ahead (a lane's mask is its number; lanes 0-7 hold the plane's values)
+  float tab_sum = 1.f;
+  unsigned tab_canon = 0u;
+  auto load_tables = [&](int p) {
+    if (wave < H) {
+      const int k = clampk(p - wave);
+      tab_sum = sums[64 * k + lane];
+      tab_canon = canon8[8 * k + (lane & 7)];
+    }
+  };
+  auto write_tables = [&](int buf) {
+    if (wave < H) {
+      wd_tab[buf][wave][lane] = omw / tab_sum;
+      if (lane < 8) cv_tab[buf][wave][lane] = tab_canon;
+    }
+  };
+  // the edge rows that step p's half-sweep h reads: plane p-h, the colour
+  // it reads, at the component that row's reader needs
+  auto write_edges = [&](int s, int buf) {
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const int slot = (s - h + 2 * U) % U;
+      const int ofirst = ((s - h + 2 * U) & 1) ^ (h & 1);  // own component of a row with even a
+      // my last row is the row above the next group's first row (a = 0), my
+      // first row the one below the previous group's last row (a = RW-1, odd)
+      edge[buf][h][1][threadIdx.x] = W[RW - 1][slot][ofirst];
+      edge[buf][h][0][threadIdx.x] = W[0][slot][ofirst ^ 1];
+    }
+  };
 
-#pragma unroll 1
-    for (int j = j0 - 1; j <= j1; ++j) {
-      load_black(j + 1, bp);
-      // red inputs of row j (planes k0-1 .. k0+K); j0-1 >= 0 and j1 <= NY-1
-      const unsigned rj = row_off(j);
-      float ro[NR], rr[NR];
-      unsigned rmk[NR];
+  load_lambda(pfirst - 1, U - 1);
+  load_lambda(pfirst, 0);
+  load_lambda(pfirst + 1, 1);
+  load_rhs(pfirst, 0);
+  load_masks(pfirst, 0);
+  load_tables(pfirst);
+  int wtop = 0;
+  {
+    const int nqb = (d.HP + 31) / 32;
 #pragma unroll
-      for (int p = 0; p < NR; ++p) {
-        const unsigned x = rj + plane_off(k0 - 1 + p);
-        ro[p] = a0[x];
-        rr[p] = R0[x];
-        rmk[p] = mask0[x];
+    for (int a = 0; a < RW; a += 2) wtop = max(wtop, A.top[(j0 + a < d.NY ? j0 + a : d.NY - 1) / 2 * nqb + (int)qc / 32]);
+  }
+  // the gate is read while those loads are in flight
+  if (!(T == 1 && A.fix)) {
+    if (!gate_pass_multi(A.err, t, A.tol, A.status, lane)) return;  // identical in every wave of the grid
+    if (tile == 0 && threadIdx.x == 0) {
+      *A.cur = (unsigned)(src ^ 1);
+      A.status[kLastT] = (unsigned)t;
+      A.status[kLastIters] = (unsigned)T;
+      A.status[kLastOmega] = __float_as_uint(om[0]);
+      A.status[kLastOmega + 1] = __float_as_uint(om[1]);
+    }
+  }
+  // Buildings stand on the ground: below the highest wall of its columns a
+  // wave takes every plane as masked, above it none.  (Plane 1's mirror is the
+  // masked steps' business: the first ones of a segment at the ground are.)
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) wtop = max(wtop, __shfl_xor(wtop, off, 64));
+  wtop = __builtin_amdgcn_readfirstlane(wtop);
+  write_tables(0);
+  write_edges(0, 0);
+  lds_barrier();
+
+  // the same lane of the groups above and below
+  const int tup = (int)threadIdx.x >= GW ? (int)threadIdx.x - GW : (int)threadIdx.x;
+  const int tdn = (int)threadIdx.x < (NG - 1) * GW ? (int)threadIdx.x + GW : (int)threadIdx.x;
+  // the steps p0 .. p0+U-1; OPEN: no wall in this wave's rows on the planes they relax
+  auto block = [&](int p0, auto is_open) {
+    constexpr bool OPEN = decltype(is_open)::value;
+#pragma unroll
+    for (int s = 0; s < U; ++s) {
+      const int p = p0 + s;
+      if (p > plast) break;
+      const int buf = s & 1;
+      load_lambda(p + 2, (s + 2) % U);
+      load_rhs(p + 1, (s + 1) % U);
+      if (!OPEN) load_masks(p + 1, (s + 1) % U);
+      load_tables(p + 1);
+#pragma unroll
+      for (int h = 0; h < H; ++h) {
+        const int k = p - h;
+        const int klo = ka - (H - 1 - h) > 1 ? ka - (H - 1 - h) : 1;
+        const int khi = kb - 1 + (H - 1 - h) < d.NZ - 2 ? kb - 1 + (H - 1 - h) : d.NZ - 2;
+        const bool in_range = k >= klo && k <= khi;  // uniform
+        const int sk = (s - h + 2 * U) % U, sup = (sk + 1) % U, sdn = (sk + U - 1) % U;
+        const float yabove = edge[buf][h][1][tup], ybelow = edge[buf][h][0][tdn];
+        const float omo = 1.0f - om[h];
+        const uint4 c03 = *reinterpret_cast<const uint4 *>(&cv_tab[buf][h][0]);
+        const uint2 c45 = *reinterpret_cast<const uint2 *>(&cv_tab[buf][h][4]);
+        const float wdo = OPEN ? wd_tab[buf][h][63] : 0.f;
+#pragma unroll
+        for (int a = 0; a < RW; ++a) {
+          const int e = (a + s - h + 2 * U) & 1;  // (j + k) & 1
+          const int o = e ^ (h & 1);              // the cell relaxed: i = 2q + o
+          const float old = W[a][sk][o], xc = W[a][sk][o ^ 1];
+          const float xm = o ? xc : lane_shift<-1>(xc);
+          const float xp = o ? lane_shift<1>(xc) : xc;
+          const float ym = a > 0 ? W[a > 0 ? a - 1 : 0][sk][o] : yabove;
+          const float yp = a < RW - 1 ? W[a < RW - 1 ? a + 1 : a][sk][o] : ybelow;
+          const float zp = W[a][sup][o], zm = W[a][sdn][o];
+          const float r = G[a][sk][o];
+          float ec, fc, gc, hc, mc, nc, wd;
+          if (OPEN) {
+            ec = __uint_as_float(c03.x);
+            fc = __uint_as_float(c03.y);
+            gc = __uint_as_float(c03.z);
+            hc = __uint_as_float(c03.w);
+            mc = __uint_as_float(c45.x);
+            nc = __uint_as_float(c45.y);
+            wd = wdo;
+          } else {
+            const unsigned m = M[a / 2][sk];
+            const unsigned base = 16u * (a & 1) + 8u * o;
+            auto coef = [&](unsigned bit, unsigned cb) { return __uint_as_float(cb & mask_bit(m, base + 2u + bit)); };
+            ec = coef(0, c03.x);
+            fc = coef(1, c03.y);
+            gc = coef(2, c03.z);
+            hc = coef(3, c03.w);
+            mc = coef(4, c45.x);
+            nc = coef(5, c45.y);
+            wd = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(wd_tab[buf][h]) + mask_index(m, base));
+          }
+          const float nv = wd * (ec * xp + fc * xm + gc * yp + hc * ym + mc * zp + nc * zm - r) + omo * old;
+          const float sel = (upd[a][o] & in_range) ? nv : old;
+          W[a][sk][o] = sel;
+          max_abs(dm[h >> 1][a], sel - old);
+        }
       }
-      // black inputs of row j-1 (owned planes)
-      const int jb = j - 1;
-      const bool brow = jb >= j0 && jb < j1;
-      const unsigned rb = row_off(jb);
-      float br[K];
-      unsigned bmk[K];
+      // after an iteration lambda(i,j,0) = lambda(i,j,1): what the next
+      // iteration of plane 1 reads (the first one reads plane 0 as stored)
+      if (!OPEN && T > 1 && s == 2 && p == 2) {
 #pragma unroll
-      for (int p = 0; p < K; ++p) {
-        const unsigned x = rb + plane_off(k0 + p);
-        br[p] = R1[x];
-        bmk[p] = mask1[x];
+        for (int a = 0; a < RW; ++a) {
+          W[a][0][0] = W[a][1][0];
+          W[a][0][1] = W[a][1][1];
+        }
       }
-      // ---- red cells of row j, plane by plane, each followed by the black
-      // cell of row j-1 in the same plane (its red neighbours: rows j-2..j
-      // of this plane, planes k-1 and k+1 of row j-1 from the last step)
-      const bool rowu = j >= 1 && j <= d.NY - 2;
-      const bool rown = j >= j0 && j < j1;
+      {
+        const int k = p - (H - 1), sk = (s - (H - 1) + 2 * U) % U;
+        if (k >= ka && k < kb) {
+          const __amdgpu_buffer_rsrc_t pl =
+              buffer_of(reinterpret_cast<char *>(out) + (unsigned long long)k * plane8, plane8);
 #pragma unroll
-      for (int p = 0; p < NR; ++p) {
-        const int k = k0 - 1 + p;
-        // the plane's wall values (LDS broadcast reads), read here rather
-        // than hoisted for all planes at once, which would hold 6 more
-        // VGPRs per plane through the step
-        asm volatile("" ::: "memory");
-        unsigned cv[6];
+          for (int a = 0; a < RW; ++a) {
+            const float x0 = W[a][sk][0], x1 = W[a][sk][1];
+            bad |= own[a] & ((upd[a][0] & !isfinite(x0)) | (upd[a][1] & !isfinite(x1)));
+            if (own[a]) {
+              uint2v v;
+              v.x = __float_as_uint(x0);
+              v.y = __float_as_uint(x1);
+              __builtin_amdgcn_raw_buffer_store_b64(v, pl, voff[a], 0, 0);
+            }
+          }
+          if (!OPEN && k == 1) {  // the mirror, for the relaxed columns
+            const __amdgpu_buffer_rsrc_t p0l = buffer_of(out, plane8);
 #pragma unroll
-        for (int a = 0; a < 6; ++a) cv[a] = cv_tab[wave][p][a];
-        {
-          const int s = (j + k) & 1;
-          const bool upd = (rowu && k >= 1 && k <= d.NZ - 2) && (s ? col1 : col0);
-          const float c = bc[p + 1];
-          const float cdn = __shfl_up(c, 1, 64);    // half-cell q-1
-          const float cup = __shfl_down(c, 1, 64);  // half-cell q+1
-          const float xm = s ? c : cdn;
-          const float xp = s ? cup : c;
-          const float nv = relax_tab(rmk[p], cv, wd_tab[wave][0][p][rmk[p] & 63u], xp, xm, bp[p + 1], bm[p + 1],
-                                     bc[p + 2], bc[p], rr[p], ro[p], omo_r);
-          rn[p] = upd ? nv : ro[p];
-          if (rown && k >= k0 && k < k1) {  // wave-uniform; k >= k0: never the halo plane
-            const bool cnt = own && upd;
-            const float dd = cnt ? fabsf(nv - ro[p]) : 0.f;
-            dl = (dd > dl) ? dd : dl;  // NaN never wins, as in the reference's max test
-            bad = bad || (cnt && !isfinite(nv));
-            const unsigned x = rj + plane_off(k);
-            if (own) b0[x] = rn[p];
-            // lambda(i,j,0) = lambda(i,j,1), black plane 0
-            if (p == 1 && k0 == 1 && cnt) b1[x - sp] = nv;
+            for (int a = 0; a < RW; ++a) {
+#pragma unroll
+              for (int o = 0; o < 2; ++o)
+                if (own[a] & upd[a][o])
+                  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(W[a][sk][o]), p0l, voff[a] + 4u * o, 0, 0);
+            }
           }
         }
-        if (p >= 1 && p <= K && brow && k < k1) {  // wave-uniform
-          const int s = (jb + k + 1) & 1;
-          const bool upd = s ? col1 : col0;  // row and plane are updated ones
-          const float c = rm1[p];
-          const float cdn = __shfl_up(c, 1, 64);
-          const float cup = __shfl_down(c, 1, 64);
-          const float xm = s ? c : cdn;
-          const float xp = s ? cup : c;
-          const float o = bm[p + 1];
-          const float nv = relax_tab(bmk[p - 1], cv, wd_tab[wave][1][p][bmk[p - 1] & 63u], xp, xm, rn[p], rm2[p],
-                                     rm1[p + 1], rm1[p - 1], br[p - 1], o, omo_b);
-          const bool cnt = own && upd;
-          const float dd = cnt ? fabsf(nv - o) : 0.f;
-          dl = (dd > dl) ? dd : dl;
-          bad = bad || (cnt && !isfinite(nv));
-          const unsigned x = rb + plane_off(k);
-          if (own) b1[x] = upd ? nv : o;
-          if (p == 1 && k0 == 1 && cnt) b0[x - sp] = nv;  // lambda(i,j,0) = lambda(i,j,1), red plane 0
-        }
       }
-      // ---- the march moves one row
-#pragma unroll
-      for (int p = 0; p < NB; ++p) {
-        bm[p] = bc[p];
-        bc[p] = bp[p];
-      }
-#pragma unroll
-      for (int p = 0; p < NR; ++p) {
-        rm2[p] = rm1[p];
-        rm1[p] = rn[p];
-      }
+      write_edges((s + 1) % U, buf ^ 1);
+      write_tables(buf ^ 1);
+      lds_barrier();
     }
+  };
+  int p0 = pfirst;
+#pragma unroll 1
+  for (; p0 <= plast && p0 - (H - 1) <= wtop; p0 += U) block(p0, std::false_type{});
+#pragma unroll 1
+  for (; p0 <= plast; p0 += U) block(p0, std::true_type{});
+  if (bad) atomicMin(A.status + kBadAt, (unsigned)(t + T - 1));
+#pragma unroll
+  for (int i = 0; i < T; ++i) {
+    float m = 0.f;
+#pragma unroll
+    for (int a = 0; a < RW; ++a) m = own[a] ? fmaxf(m, dm[i][a]) : m;
+    m = wave_max(m);
+    if (lane == 0) wmax[wave][i] = m;
   }
-  if (bad) atomicOr(status, ST_NONFINITE);
-  const float wm = wave_max(dl);
-  if (lane == 0) wmax[wave] = wm;
+  lds_barrier();
+  if (threadIdx.x < T) {
+    float m = 0.f;
+    for (int w = 0; w < NW; ++w) m = fmaxf(m, wmax[w][threadIdx.x]);
+    if (m > 0.f)
+      atomicMax(A.err + (long long)(t + 1 + (int)threadIdx.x) * kErrSlots + (blockIdx.x % kErrSlots),
+                __float_as_uint(m));
+  }
+}
+
+// End of a stretch of launches over iterations [.., hi): find the iteration
+// the run ended at (rows below lo were scanned before), and if that is inside
+// the last launch, order its first iteration to be redone on its own.
+__global__ __launch_bounds__(256) void k_sor_settle(const unsigned *__restrict__ rows, int lo, int hi, float tol,
+                                                    unsigned *__restrict__ status)
+{
+  __shared__ unsigned first;
+  if (threadIdx.x == 0) first = 0xffffffffu;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    const float bmax = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-    if (bmax > 0.f) atomicMax(err + (long long)(t + 1) * kErrSlots + (blockIdx.x % kErrSlots), __float_as_uint(bmax));
+  // one wave per row, one slot per lane
+  for (int t = lo + (int)(threadIdx.x >> 6); t < hi; t += 4) {
+    const float v = __uint_as_float(rows[(long long)t * kErrSlots + (threadIdx.x & 63)]);
+    const float m = wave_max(v > 0.f ? v : 0.f);
+    if ((threadIdx.x & 63) == 0 && !(m > tol)) atomicMin(&first, (unsigned)t);
   }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  unsigned end = status[kEnd];
+  if (__uint_as_float(status[kStopExtend]) > 0.f) {
+    const unsigned e = status[kStopAt];
+    end = e < (unsigned)hi ? e : end;
+  } else if (first < end) {
+    end = first;
+  }
+  status[kEnd] = end;
+  const unsigned lt = status[kLastT], li = status[kLastIters];
+  const bool fix = li > 1u && end > lt && end < lt + li;
+  status[kFixGo] = fix ? 1u : 0u;
+  if (fix) status[kLastIters] = end - lt;
+}
+
+// The wall masks of both colours in the pair layout, two rows (2r, 2r+1) to a
+// word: [k][r][q], the even row's pair in the low half, each pair's cell i = 2q
+// in its low byte, as mask times 4.  Positions that are not relaxed (the ring, the padding) are
+// open.  top[r][q / 32] (zeroed before) is the highest plane with a wall.
+__global__ __launch_bounds__(256) void k_pair_masks(Dims d, const unsigned char *__restrict__ m0,
+                                                    const unsigned char *__restrict__ m1, unsigned *__restrict__ out,
+                                                    int *__restrict__ top)
+{
+  const int nr = (d.NY + 1) / 2;
+  const int plane = nr * d.HP;
+  const long long n = (long long)plane * d.NZ;
+  const long long stride = (long long)gridDim.x * 256;
+  for (long long x = blockIdx.x * 256LL + threadIdx.x; x < n; x += stride) {
+    const int k = (int)(x / plane);
+    const int rem = (int)(x - (long long)k * plane);
+    const int r = rem / d.HP, q = rem - r * d.HP;
+    unsigned w = 0;
+#pragma unroll
+    for (int y = 0; y < 2; ++y) {
+      const int j = 2 * r + y;
+      unsigned lo = 63u, hi = 63u;
+      if (k >= 1 && k <= d.NZ - 2 && j >= 1 && j <= d.NY - 2) {
+        const long long s = (long long)(k * d.NY + j) * d.HP + q;
+        const bool odd = (j + k) & 1;
+        if (q >= 1 && 2 * q <= d.NX - 2) lo = odd ? m1[s] : m0[s];
+        if (2 * q + 1 <= d.NX - 2) hi = odd ? m0[s] : m1[s];
+      }
+      w |= ((lo << 2) | (hi << 10)) << (16 * y);
+    }
+    out[x] = w;
+    if (w != kOpenRows) atomicMax(top + r * ((d.HP + 31) / 32) + q / 32, k);
+  }
+}
+
+// The wall values layer-major, canon8[k*8 + a] = canon[a*NZ + k] (words 6 and
+// 7 unused), and per layer the sum of those each mask selects, added in the
+// order the relaxation adds them.
+__global__ __launch_bounds__(64) void k_march_tables(int NZ, const unsigned *__restrict__ canon,
+                                                     unsigned *__restrict__ canon8, float *__restrict__ sums)
+{
+  const int k = blockIdx.x, lane = threadIdx.x;
+  float v[6];
+#pragma unroll
+  for (int a = 0; a < 6; ++a) v[a] = (lane >> a) & 1 ? __uint_as_float(canon[a * NZ + k]) : 0.f;
+  sums[64 * k + lane] = v[0] + v[1] + v[2] + v[3] + v[4] + v[5];
+  if (lane < 8) canon8[8 * k + lane] = lane < 6 ? canon[lane * NZ + k] : 0u;
 }
 
 }  // namespace qesmc
 
 using namespace qesmc;
 
+// words of the highest-wall table of a domain
+long long qesmc_march_top_words(const Dims &d) { return (long long)((d.NY + 1) / 2) * ((d.HP + 31) / 32); }
+
 namespace {
 
-constexpr int kMarchWavesPerCu = 8;  // segment rule below
+// The instantiated shapes for two iterations per launch: waves, lanes per row group (two rows per group).
+constexpr int kShapes[][2] = {{4, 32}, {8, 32}, {16, 32}, {16, 64}};
+constexpr int kTail = 1;  // the shape of the single-iteration launches
+constexpr int kWavesPerCu = 16;  // 128 vector registers each
 
-// The march's tiling: lanes per tile, k planes, rows per segment.
-struct MarchTiling {
-  int K, W, qt, nkc, L;
-  long long ntiles, blocks;
-};
-
-MarchTiling march_tiling(const Dims &d, int kplanes, int n_cu)
+// Columns of tiles (x tiles, y tiles) of a shape.
+void march_columns(const Dims &d, int T, int shape, int *nq, int *nyt)
 {
-  MarchTiling m{};
-  // 16 planes would need 256 VGPRs (one wave per SIMD): 8 at most
-  m.K = kplanes >= 8 ? 8 : 4;
-  m.qt = (d.HP + 61) / 62;
-  m.W = (d.HP + m.qt - 1) / m.qt;
-  m.nkc = (d.NZ - 2 + m.K - 1) / m.K;
-  // rows per segment: the most (at most 64) that still give >= 8 wave tiles
-  // per CU (measured: 16 gave 4-row segments on 400 x 400 x 120, 72.7 us per
-  // iteration against 64 us with 8-row ones; 1000 x 1000 x 150 within 1 %)
-  auto tiles = [&](int l) { return (long long)m.qt * m.nkc * ((d.NY - 2 + l - 1) / l); };
-  m.L = 64;
-  while (m.L > 4 && tiles(m.L) < (long long)kMarchWavesPerCu * n_cu) m.L /= 2;
-  m.ntiles = tiles(m.L);
-  m.blocks = (m.ntiles + kWaves - 1) / kWaves;
-  m.blocks = (m.blocks + kXcds - 1) / kXcds * kXcds;
-  return m;
+  const int nw = kShapes[shape][0], gw = kShapes[shape][1];
+  const int half = (d.NX + 1) / 2, yr = 2 * nw * (64 / gw);
+  *nq = half <= gw ? 1 : (half - 2 * T + gw - 2 * T - 1) / (gw - 2 * T);
+  *nyt = d.NY <= yr ? 1 : (d.NY - 4 * T + yr - 4 * T - 1) / (yr - 4 * T);
+}
+
+// Relative cost of the steps a segment [ka, kb) takes: it fills its pipeline
+// over the 2T-1 planes before it (those that exist) and drains over as many
+// steps after it.  sum[p]: the cost of the steps below p.
+double segment_cost(const std::vector<double> &sum, int T, int ka, int kb)
+{
+  const int first = ka - (2 * T - 1) > 0 ? ka - (2 * T - 1) : 0;
+  return sum[(size_t)(kb + 2 * T - 1)] - sum[(size_t)first];
+}
+
+// Cut planes [1, end) into segments that cost at most `limit`, each starting
+// on an odd plane and at least `least` planes long: the number of segments, 0
+// if they do not fit the table.
+int cut_segments(const std::vector<double> &sum, int T, int end, int least, double limit, MarchPlan &m)
+{
+  int n = 0, ka = 1;
+  while (ka < end) {
+    if (n == kMaxSegments) return 0;
+    int kb = ka + least;
+    while (kb < end && segment_cost(sum, T, ka, kb + 2 < end ? kb + 2 : end) <= limit) kb += 2;
+    if (kb > end) kb = end;
+    m.begin[n++] = (short)ka;
+    ka = kb;
+  }
+  m.begin[n] = (short)end;
+  return n;
+}
+
+// The cut into at most nseg segments whose dearest is the cheapest.
+double balance_segments(const std::vector<double> &sum, int T, int end, int nseg, MarchPlan &m)
+{
+  const int least = 2 * T;
+  double lo = 0.0, hi = segment_cost(sum, T, 1, end);
+  m.nseg = cut_segments(sum, T, end, least, hi, m);
+  for (int it = 0; it < 14 && nseg > 1; ++it) {
+    const double mid = 0.5 * (lo + hi);
+    MarchPlan trial = m;
+    const int n = cut_segments(sum, T, end, least, mid, trial);
+    if (n > 0 && n <= nseg) {
+      hi = mid;
+      m = trial;
+      m.nseg = n;
+    } else {
+      lo = mid;
+    }
+  }
+  double worst = 0.0;
+  for (int q = 0; q < m.nseg; ++q) {
+    const double c = segment_cost(sum, T, m.begin[q], m.begin[q + 1]);
+    worst = c > worst ? c : worst;
+  }
+  return worst;
 }
 
 }  // namespace
 
-// The wall values layer-major for the march's scalar loads: canon8[k*8 + a]
-// = canon[a*NZ + k] (words 6 and 7 unused).
-__global__ __launch_bounds__(256) void k_canon_transpose(int NZ, const unsigned *__restrict__ canon,
-                                                         unsigned *__restrict__ canon8)
+// The march's shape and segments for the resident domain.  top: the table of
+// highest walls.  A segment's time is the sum of its steps' and the launch's
+// that of the dearest segment.  Measured with 16 waves on a CU: 1.97 us a step
+// where every plane has walls (298 vector instructions a wave: the vector ALUs
+// are busy throughout), 1.49 us where none has (172; bound by the caches), so
+// the segments near the ground are the shorter ones.  Microseconds of an open
+// step with n waves on the CU: 0.62 + 0.054 n, and a launch 4.6 besides.
+// Rows of 32 pairs touch a fifth more cache lines than rows of 64: 4 % slower
+// per step, 15 % where they come from HBM.
+// tile_k > 0 sets the planes per segment.
+void qesmc_march_choose(qesmc_ctx *x, int tile_k, const int *top)
 {
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  if (e >= NZ * 8) return;
-  const int k = e >> 3, a = e & 7;
-  canon8[e] = a < 6 ? canon[a * NZ + k] : 0u;
+  const Dims &d = x->d;
+  const int end = d.NZ - 1;
+  std::vector<double> w((size_t)d.NZ, 1.0);
+  if (top) {
+    const long long n = qesmc_march_top_words(d);
+    std::vector<int> count((size_t)d.NZ + 1, 0);
+    for (long long q = 0; q < n; ++q) ++count[(size_t)top[q]];
+    long long above = n;
+    for (int k = 0; k < d.NZ; ++k) {
+      w[(size_t)k] = 1.0 + 0.32 * (double)above / (double)n;  // the share whose top is at k or higher
+      above -= count[(size_t)k];
+    }
+  }
+  std::vector<double> sum((size_t)d.NZ + 4, 0.0);
+  for (size_t p = 0; p + 1 < sum.size(); ++p) sum[p + 1] = sum[p] + w[p < w.size() ? p : w.size() - 1];
+  auto uniform = [&](int T, int planes, MarchPlan &m) {
+    int seg = planes < 2 * T ? 2 * T : (planes + 1) / 2 * 2;
+    while ((end - 1 + seg - 1) / seg > kMaxSegments) seg += 2;
+    m.nseg = 0;
+    for (int ka = 1; ka < end; ka += seg) m.begin[m.nseg++] = (short)ka;
+    m.begin[m.nseg] = (short)end;
+  };
+  const bool beyond = (double)x->nsplit * 2.0 * (4.0 + 4.0 + 1.0) > 256.0 * (1 << 20);
+  for (int T = 2; T >= 1; --T) {
+    MarchPlan &plan = x->march[T - 1];
+    double best = 1e300;
+    const int shapes = (int)(sizeof(kShapes) / sizeof(kShapes[0]));
+    for (int c = T == 1 ? kTail : 0; c < (T == 1 ? kTail + 1 : shapes); ++c) {
+      MarchPlan m{};
+      m.shape = c;
+      march_columns(d, T, c, &m.nq, &m.nyt);
+      const long long columns = (long long)m.nq * m.nyt;
+      const int fit = kWavesPerCu / kShapes[c][0];
+      int tried = 0;
+      for (int per_cu = 1; per_cu <= 6 * fit; ++per_cu) {
+        long long nseg = (long long)per_cu * x->n_cu / columns;
+        if (nseg > kMaxSegments) nseg = kMaxSegments;
+        if (nseg < 1) nseg = 1;
+        if (nseg == tried) continue;
+        tried = (int)nseg;
+        double worst;
+        if (tile_k > 0) {
+          uniform(T, tile_k, m);
+          worst = segment_cost(sum, T, m.begin[0], m.begin[1]);
+        } else {
+          worst = balance_segments(sum, T, end, (int)nseg, m);
+        }
+        const long long per = (columns * m.nseg + x->n_cu - 1) / x->n_cu;
+        const int resident = per < fit ? (int)per : fit;
+        const double narrow = kShapes[c][1] == 64 ? 1.0 : beyond ? 1.15 : 1.04;
+        const double us = 4.6 + (double)((per + fit - 1) / fit) * worst * (0.62 + 0.054 * kShapes[c][0] * resident) * narrow;
+        if (us < best) {
+          best = us;
+          plan = m;
+        }
+        if (tile_k > 0) break;
+      }
+    }
+  }
 }
 
 hipError_t qesmc_fused_prepare(qesmc_ctx *x)
 {
-  const int n = x->d.NZ * 8;
-  hipLaunchKernelGGL(k_canon_transpose, dim3((n + 255) / 256), dim3(256), 0, x->stream, x->d.NZ, x->d_canon,
-                     x->d_canon8);
+  hipLaunchKernelGGL(k_march_tables, dim3((unsigned)x->d.NZ), dim3(64), 0, x->stream, x->d.NZ, x->d_canon,
+                     x->d_canon8, reinterpret_cast<float *>(x->d_canon8 + 8LL * x->d.NZ));
+  const long long b = (x->nsplit / 2 + 255) / 256;
+  const long long nt = qesmc_march_top_words(x->d);
+  hipError_t e = qesmc_launch_fill_u32(x, reinterpret_cast<unsigned *>(x->d_top), nt, 0u);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_pair_masks, dim3((unsigned)(b < 16384 ? b : 16384)), dim3(256), 0, x->stream, x->d,
+                     x->d_mask[0], x->d_mask[1], x->d_mask2, x->d_top);
   return hipGetLastError();
 }
 
-// Launch iteration t of the fused path: reads buffer set t & 1, writes the other.
-hipError_t qesmc_launch_fused_iteration(qesmc_ctx *x, int t, int itermax, float omega_red, float omega_black,
-                                        float tol)
+// Launch iterations t .. t + iters - 1 (iters 1 or 2), reading buffer set
+// src and writing the other; om holds omega of the red and black pass of each.
+// With fix, redo what k_sor_settle ordered instead.
+hipError_t qesmc_launch_march(qesmc_ctx *x, int t, int iters, int itermax, const float *om, float tol, int src, bool fix)
 {
   const Dims &d = x->d;
   if (d.NZ - 2 < 1 || d.NY - 2 < 1) return hipSuccess;
-  if (x->nsplit >= (1LL << 31)) return hipErrorInvalidValue;  // the kernel's 32-bit offsets
-  const MarchTiling m = march_tiling(d, x->kplanes, x->n_cu);
-  float *const *A = (t & 1) ? x->d_lc2 : x->d_lc;
-  float *const *B = (t & 1) ? x->d_lc : x->d_lc2;
-#define QESMC_MARCH_LAUNCH(KK)                                                                                 \
-  hipLaunchKernelGGL(k_sor_march<KK>, dim3((unsigned)m.blocks), dim3(64 * kWaves), 0, x->stream, d, m.W, m.qt, \
-                     m.L, m.nkc, m.ntiles, A[0], A[1], B[0], B[1], x->d_Rc[0], x->d_Rc[1], x->d_mask[0],        \
-                     x->d_mask[1], x->d_canon8, omega_red, 1.0f - omega_red, omega_black, 1.0f - omega_black, tol,  \
-                     x->d_err, t, itermax, x->d_status, x->d_cur)
-  if (m.K == 8) QESMC_MARCH_LAUNCH(8);
-  else QESMC_MARCH_LAUNCH(4);
+  const MarchPlan &m = x->march[iters - 1];
+  const int nw = kShapes[m.shape][0], gw = kShapes[m.shape][1];
+  const int ntiles = m.nq * m.nyt * m.nseg;
+  const int blocks = (ntiles + kXcds - 1) / kXcds * kXcds;
+  MarchArgs a{};
+  a.d = d;
+  a.nq = m.nq;
+  a.nyt = m.nyt;
+  a.ntiles = ntiles;
+  std::memcpy(a.begin, m.begin, sizeof(a.begin));
+  a.set0 = reinterpret_cast<float2 *>(x->d_lc[0]);
+  a.set1 = reinterpret_cast<float2 *>(x->d_lc2[0]);
+  a.R = reinterpret_cast<const float2 *>(x->d_Rc[0]);
+  a.mask = x->d_mask2;
+  a.top = x->d_top;
+  a.canon8 = x->d_canon8;
+  a.sums = reinterpret_cast<const float *>(x->d_canon8 + 8LL * d.NZ);
+  for (int h = 0; h < 2 * iters; ++h) a.om[h] = om[h];
+  a.tol = tol;
+  a.err = x->d_err;
+  a.t = t;
+  a.itermax = itermax;
+  a.status = x->d_status;
+  a.cur = x->d_cur;
+  a.src = src;
+  a.fix = fix ? 1 : 0;
+#define QESMC_MARCH_LAUNCH(T, N, R, G) \
+  hipLaunchKernelGGL((k_sor_march<T, N, R, G>), dim3((unsigned)blocks), dim3(64 * N), 0, x->stream, a)
+  if (iters == 1) QESMC_MARCH_LAUNCH(1, 8, 2, 32);
+  else if (nw == 4) QESMC_MARCH_LAUNCH(2, 4, 2, 32);
+  else if (nw == 8) QESMC_MARCH_LAUNCH(2, 8, 2, 32);
+  else if (gw == 32) QESMC_MARCH_LAUNCH(2, 16, 2, 32);
+  else QESMC_MARCH_LAUNCH(2, 16, 2, 64);
 #undef QESMC_MARCH_LAUNCH
   return hipGetLastError();
+}
+
+// The run's end over iterations [lo, hi) and, if it falls inside the last
+// launch, that launch redone up to it.
+hipError_t qesmc_march_settle(qesmc_ctx *x, int lo, int hi, float tol)
+{
+  hipLaunchKernelGGL(k_sor_settle, dim3(1), dim3(256), 0, x->stream, x->d_err, lo, hi, tol, x->d_status);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const float om[2] = {0.f, 0.f};  // taken from the launch that is redone
+  return qesmc_launch_march(x, 0, 1, 1, om, tol, 0, true);
 }

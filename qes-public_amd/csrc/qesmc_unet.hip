@@ -23,7 +23,7 @@
 
 #include "qesmc_internal.h"
 
-hipError_t qesmc_launch_divergence(qesmc_ctx *x, bool split, int alpha1);
+hipError_t qesmc_launch_divergence(qesmc_ctx *x, int layout, int alpha1);
 
 namespace qesmc {
 namespace unet {
@@ -1148,7 +1148,7 @@ int problem_features(qesmc_unet *u, qesmc_ctx *x)
   if (x->d.nx - 1 != u->ncx || x->d.ny - 1 != u->ncy || x->d.nz - 2 != u->ncz) return QESMC_ERR_ARG;
   UCHK(hipStreamSynchronize(x->stream));
   // R on the x-fastest layout, on the solver's stream
-  UCHK(qesmc_launch_divergence(x, false, 1));
+  UCHK(qesmc_launch_divergence(x, 0, 1));
   UCHK(hipStreamSynchronize(x->stream));
   hipStream_t s = u->stream;
   UCHK(hipMemsetAsync(u->dacc, 0, sizeof(double), s));
