@@ -270,6 +270,7 @@ int qesmc_create(qesmc_ctx **out, int device)
   qesmc_ctx *x = new (std::nothrow) qesmc_ctx();
   if (!x) return QESMC_ERR_OOM;
   x->device = device;
+  qesmc::host_copy_attach(device);
   int rc = QESMC_OK;
   auto fail = [&](hipError_t e) {
     rc = map_hip(e);
@@ -312,6 +313,7 @@ int qesmc_destroy(qesmc_ctx *x)
   for (auto &ev : x->ev)
     if (ev) (void)hipEventDestroy(ev);
   if (x->stream) (void)hipStreamDestroy(x->stream);
+  qesmc::host_copy_detach(x->device);
   delete x;
   return QESMC_OK;
 }
@@ -333,9 +335,12 @@ int qesmc_set_geometry(qesmc_ctx *x, const qesmc_grid *grid, const qesmc_coeffs 
   x->dy = grid->dy;
   x->dz_host.assign(grid->dz_array, grid->dz_array + (grid->nz - 1));
   const size_t cb = sizeof(float) * (size_t)x->ncell;
-  const float *src[6] = {cf->e, cf->f, cf->g, cf->h, cf->m, cf->n};
-  for (int a = 0; a < 6; ++a) HIPCHK(hipMemcpyAsync(x->d_coef[a], src[a], cb, hipMemcpyHostToDevice, x->stream));
-  HIPCHK(hipMemcpyAsync(x->d_flag, cf->icellflag, sizeof(int) * (size_t)x->ncell, hipMemcpyHostToDevice, x->stream));
+  const qesmc::HostPiece pieces[7] = {
+      qesmc::host_piece(cf->e, x->d_coef[0], cb), qesmc::host_piece(cf->f, x->d_coef[1], cb),
+      qesmc::host_piece(cf->g, x->d_coef[2], cb), qesmc::host_piece(cf->h, x->d_coef[3], cb),
+      qesmc::host_piece(cf->m, x->d_coef[4], cb), qesmc::host_piece(cf->n, x->d_coef[5], cb),
+      qesmc::host_piece(cf->icellflag, x->d_flag, sizeof(int) * (size_t)x->ncell)};
+  HIPCHK(qesmc::host_copy(x->device, x->stream, pieces, 7, true));
   HIPCHK(hipMemcpyAsync(x->d_dz, grid->dz_array, sizeof(float) * (grid->nz - 1), hipMemcpyHostToDevice, x->stream));
   return qesmc::geometry_commit(x);
 }
@@ -346,9 +351,9 @@ int qesmc_set_inflow(qesmc_ctx *x, const float *u0, const float *v0, const float
   if (!x->d_u0) return QESMC_ERR_STATE;
   HIPCHK(hipSetDevice(x->device));
   const size_t fb = sizeof(float) * (size_t)x->nface;
-  HIPCHK(hipMemcpyAsync(x->d_u0, u0, fb, hipMemcpyHostToDevice, x->stream));
-  HIPCHK(hipMemcpyAsync(x->d_v0, v0, fb, hipMemcpyHostToDevice, x->stream));
-  HIPCHK(hipMemcpyAsync(x->d_w0, w0, fb, hipMemcpyHostToDevice, x->stream));
+  const qesmc::HostPiece pieces[3] = {qesmc::host_piece(u0, x->d_u0, fb), qesmc::host_piece(v0, x->d_v0, fb),
+                                      qesmc::host_piece(w0, x->d_w0, fb)};
+  HIPCHK(qesmc::host_copy(x->device, x->stream, pieces, 3, true));
   x->have_inflow = true;
   return QESMC_OK;
 }
@@ -358,9 +363,10 @@ int qesmc_set_lambda(qesmc_ctx *x, const float *lambda)
   if (!x) return QESMC_ERR_ARG;
   if (!x->d_lam) return QESMC_ERR_STATE;
   HIPCHK(hipSetDevice(x->device));
-  if (lambda)
-    HIPCHK(hipMemcpyAsync(x->d_lam, lambda, sizeof(float) * (size_t)x->ncell, hipMemcpyHostToDevice, x->stream));
-  else
+  if (lambda) {
+    const qesmc::HostPiece piece = qesmc::host_piece(lambda, x->d_lam, sizeof(float) * (size_t)x->ncell);
+    HIPCHK(qesmc::host_copy(x->device, x->stream, &piece, 1, true));
+  } else
     HIPCHK(hipMemsetAsync(x->d_lam, 0, sizeof(float) * (size_t)x->ncell, x->stream));
   return QESMC_OK;
 }
@@ -722,10 +728,9 @@ int qesmc_get_velocity(qesmc_ctx *x, float *u, float *v, float *w)
   if (!x->d_u) return QESMC_ERR_STATE;
   HIPCHK(hipSetDevice(x->device));
   const size_t fb = sizeof(float) * (size_t)x->nface;
-  HIPCHK(hipMemcpyAsync(u, x->d_u, fb, hipMemcpyDeviceToHost, x->stream));
-  HIPCHK(hipMemcpyAsync(v, x->d_v, fb, hipMemcpyDeviceToHost, x->stream));
-  HIPCHK(hipMemcpyAsync(w, x->d_w, fb, hipMemcpyDeviceToHost, x->stream));
-  HIPCHK(hipStreamSynchronize(x->stream));
+  const qesmc::HostPiece pieces[3] = {qesmc::host_piece(u, x->d_u, fb), qesmc::host_piece(v, x->d_v, fb),
+                                      qesmc::host_piece(w, x->d_w, fb)};
+  HIPCHK(qesmc::host_copy(x->device, x->stream, pieces, 3, false));
   return QESMC_OK;
 }
 
@@ -734,8 +739,8 @@ int qesmc_get_lambda(qesmc_ctx *x, float *lambda)
   if (!x || !lambda) return QESMC_ERR_ARG;
   if (!x->d_lam) return QESMC_ERR_STATE;
   HIPCHK(hipSetDevice(x->device));
-  HIPCHK(hipMemcpyAsync(lambda, x->d_lam, sizeof(float) * (size_t)x->ncell, hipMemcpyDeviceToHost, x->stream));
-  HIPCHK(hipStreamSynchronize(x->stream));
+  const qesmc::HostPiece piece = qesmc::host_piece(lambda, x->d_lam, sizeof(float) * (size_t)x->ncell);
+  HIPCHK(qesmc::host_copy(x->device, x->stream, &piece, 1, false));
   return QESMC_OK;
 }
 

@@ -276,14 +276,15 @@ int qesmc_get_inputs(qesmc_ctx *x, float *e, float *f, float *g, float *h, float
   CCHK(hipSetDevice(x->device));
   const size_t cb = sizeof(float) * (size_t)x->ncell, fb = sizeof(float) * (size_t)x->nface;
   float *co[6] = {e, f, g, h, m, n};
+  qesmc::HostPiece pieces[10];
+  int n_pieces = 0;
   for (int a = 0; a < 6; ++a)
-    if (co[a]) CCHK(hipMemcpyAsync(co[a], x->d_coef[a], cb, hipMemcpyDeviceToHost, x->stream));
-  if (icellflag)
-    CCHK(hipMemcpyAsync(icellflag, x->d_flag, sizeof(int) * (size_t)x->ncell, hipMemcpyDeviceToHost, x->stream));
-  if (u0) CCHK(hipMemcpyAsync(u0, x->d_u0, fb, hipMemcpyDeviceToHost, x->stream));
-  if (v0) CCHK(hipMemcpyAsync(v0, x->d_v0, fb, hipMemcpyDeviceToHost, x->stream));
-  if (w0) CCHK(hipMemcpyAsync(w0, x->d_w0, fb, hipMemcpyDeviceToHost, x->stream));
-  CCHK(hipStreamSynchronize(x->stream));
+    if (co[a]) pieces[n_pieces++] = qesmc::host_piece(co[a], x->d_coef[a], cb);
+  if (icellflag) pieces[n_pieces++] = qesmc::host_piece(icellflag, x->d_flag, sizeof(int) * (size_t)x->ncell);
+  if (u0) pieces[n_pieces++] = qesmc::host_piece(u0, x->d_u0, fb);
+  if (v0) pieces[n_pieces++] = qesmc::host_piece(v0, x->d_v0, fb);
+  if (w0) pieces[n_pieces++] = qesmc::host_piece(w0, x->d_w0, fb);
+  CCHK(qesmc::host_copy(x->device, x->stream, pieces, n_pieces, false));
   return QESMC_OK;
 }
 

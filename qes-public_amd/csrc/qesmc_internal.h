@@ -236,6 +236,20 @@ float row_max(const unsigned *row);
 int geometry_reserve(qesmc_ctx *x, int nx, int ny, int nz);
 int geometry_commit(qesmc_ctx *x);
 
+// Copies between the caller's arrays and the device (see qesmc_copy.hip),
+// complete on return.  attach / detach: a context of the device exists.
+struct HostPiece {
+  void *host, *device;
+  size_t bytes;
+};
+void host_copy_attach(int device);
+void host_copy_detach(int device);
+hipError_t host_copy(int device, hipStream_t st, const HostPiece *p, int n, bool to_device);
+inline HostPiece host_piece(const void *host, const void *device, size_t bytes)
+{
+  return {const_cast<void *>(host), const_cast<void *>(device), bytes};
+}
+
 inline int map_hip_error(hipError_t e)
 {
   switch (e) {

@@ -266,7 +266,10 @@ int qesmc_velocity_gradient_walls(qesmc_ctx *x, int building_mode, int terrain_m
     TCHK(hipGetLastError());
   }
   TCHK(hipEventRecord(x->ev[1], x->stream));
-  if (G) TCHK(hipMemcpyAsync(G, x->d_grad, sizeof(float) * 9 * (size_t)x->ncell, hipMemcpyDeviceToHost, x->stream));
+  if (G) {
+    const qesmc::HostPiece piece = qesmc::host_piece(G, x->d_grad, sizeof(float) * 9 * (size_t)x->ncell);
+    TCHK(qesmc::host_copy(x->device, x->stream, &piece, 1, false));
+  }
   TCHK(hipStreamSynchronize(x->stream));
   if (ms) {
     float t = 0.f;
@@ -306,7 +309,10 @@ int qesmc_velocity_gradient(qesmc_ctx *x, int uniform_z, float dz, float *G, dou
                      (const float4 *)tmp.p, x->dx, x->dy, dz, uniform_z ? 1 : 0, x->ncell, kb, x->d_grad);
   TCHK(hipGetLastError());
   TCHK(hipEventRecord(x->ev[1], x->stream));
-  if (G) TCHK(hipMemcpyAsync(G, x->d_grad, sizeof(float) * 9 * (size_t)x->ncell, hipMemcpyDeviceToHost, x->stream));
+  if (G) {
+    const qesmc::HostPiece piece = qesmc::host_piece(G, x->d_grad, sizeof(float) * 9 * (size_t)x->ncell);
+    TCHK(qesmc::host_copy(x->device, x->stream, &piece, 1, false));
+  }
   TCHK(hipStreamSynchronize(x->stream));
   if (ms) {
     float t = 0.f;

@@ -1179,6 +1179,7 @@ int qesmc_unet_create(qesmc_unet **out, int device, const qesmc_unet_config *cfg
   qesmc_unet *u = new (std::nothrow) qesmc_unet();
   if (!u) return QESMC_ERR_OOM;
   u->device = device;
+  host_copy_attach(device);
   u->L = cfg->levels;
   u->c0 = cfg->base_channels;
   u->ncx = cfg->ncx;
@@ -1302,6 +1303,7 @@ int qesmc_unet_destroy(qesmc_unet *u)
   for (auto &e : u->ev)
     if (e) (void)hipEventDestroy(e);
   if (u->stream) (void)hipStreamDestroy(u->stream);
+  host_copy_detach(u->device);
   delete u;
   return QESMC_OK;
 }
@@ -1350,12 +1352,13 @@ int qesmc_unet_forward(qesmc_unet *u, const float *input, float *output)
   UCHK(hipSetDevice(u->device));
   const long long V0 = (long long)u->dx * u->dy * u->dz;
   const long long n = V0 * QESMC_UNET_IN_CHANNELS;
-  UCHK(hipMemcpyAsync(u->hostbuf_dev, input, sizeof(float) * n, hipMemcpyHostToDevice, u->stream));
+  const HostPiece in = host_piece(input, u->hostbuf_dev, sizeof(float) * (size_t)n);
+  UCHK(host_copy(u->device, u->stream, &in, 1, true));
   hipLaunchKernelGGL(k_f2bf, g1(n), dim3(256), 0, u->stream, u->hostbuf_dev, u->feat, n);
   UCHK(hipGetLastError());
   UCHK(forward(u, u->feat));
-  UCHK(hipMemcpyAsync(output, u->out, sizeof(float) * V0, hipMemcpyDeviceToHost, u->stream));
-  UCHK(hipStreamSynchronize(u->stream));
+  const HostPiece out = host_piece(output, u->out, sizeof(float) * (size_t)V0);
+  UCHK(host_copy(u->device, u->stream, &out, 1, false));
   return QESMC_OK;
 }
 
@@ -1364,11 +1367,12 @@ int qesmc_unet_backward(qesmc_unet *u, const float *grad_output, float *grad_par
   if (!u || !grad_output || !grad_params) return QESMC_ERR_ARG;
   UCHK(hipSetDevice(u->device));
   const long long V0 = (long long)u->dx * u->dy * u->dz;
-  UCHK(hipMemcpyAsync(u->gout, grad_output, sizeof(float) * V0, hipMemcpyHostToDevice, u->stream));
+  const HostPiece in = host_piece(grad_output, u->gout, sizeof(float) * (size_t)V0);
+  UCHK(host_copy(u->device, u->stream, &in, 1, true));
   UCHK(hipMemsetAsync(u->gp, 0, sizeof(float) * u->nparams, u->stream));
   UCHK(backward(u, u->feat));
-  UCHK(hipMemcpyAsync(grad_params, u->gp, sizeof(float) * u->nparams, hipMemcpyDeviceToHost, u->stream));
-  UCHK(hipStreamSynchronize(u->stream));
+  const HostPiece out = host_piece(grad_params, u->gp, sizeof(float) * (size_t)u->nparams);
+  UCHK(host_copy(u->device, u->stream, &out, 1, false));
   return QESMC_OK;
 }
 
