@@ -12,7 +12,8 @@
 // (v_mfma_f32_16x16x32_bf16, FP32 accumulation): rows = voxels, columns =
 // output channels, K = 27 taps x input channels.  The data gradient is the
 // same kernel with tap-flipped, transposed weights; the weight gradient is an
-// MFMA GEMM reducing over voxels (split over work-groups, FP32 atomics).
+// MFMA GEMM reducing over voxels, transposed on the matrix cores (split over
+// work-groups, FP32 atomics).
 // FP32 master weights, Adam.
 #include <chrono>
 #include <cmath>
@@ -40,6 +41,13 @@ __device__ inline bf16_t f2bf(float f)
   return (bf16_t)(u >> 16);
 }
 __device__ inline float bf2f(bf16_t h) { return __uint_as_float(((unsigned)h) << 16); }
+
+// Element e of eight BF16 values in a register quad.
+__device__ inline float bf_at(const uint4 &t, int e)
+{
+  const unsigned w = e < 2 ? t.x : e < 4 ? t.y : e < 6 ? t.z : t.w;
+  return __uint_as_float((e & 1) ? (w & 0xffff0000u) : (w << 16));
+}
 
 __device__ inline bf16x8 as_bf16x8(uint4 u) { return __builtin_bit_cast(bf16x8, u); }
 
@@ -281,122 +289,198 @@ __global__ __launch_bounds__(256) void k_conv_fwd_lds(ConvFwdArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// 3x3x3 convolution, weight gradient: dW[n][k] += sum_v g[v][n] * X[v+off(k)][c(k)]
-// One wave: 16 output channels x (16*KT) columns k, over a voxel range.
+// 3x3x3 convolution, weight gradient: dW[n][tap][c] += sum_v g[v][n] * X[v+off(tap)][c]
+//
+// An MFMA GEMM that reduces over voxels, so each lane needs several voxels of
+// one channel, while memory holds several channels of one voxel.  The 16 x 16
+// tiles are transposed on the matrix cores: a product with the identity
+// leaves D[voxel 4*(l/16)+i][channel l%16] in lane l, exactly (the other
+// terms are zeros), whose upper halves are the operand.
+//
+// A wave owns 16 input by 16 output channels (27 accumulator tiles) and a
+// strip: 32 voxels along x, one z, a range of y.  Per row of X it transposes
+// the row at the three x shifts and the three new rows of g (z-1, z, z+1 of
+// row y+1; rows y-1 and y are kept), then runs 27 products of K = 32
+// voxels.  The next row's loads are in flight meanwhile.  The four waves of a
+// work-group take strips of one channel pair and add up in LDS, so that there
+// is one atomic per work-group and weight.
+//
+// Per row 27 products and 12 transposes against 12 loads of 512 bytes: at
+// 128x128x64 with 48 -> 16 channels 2110 us before (a lane gathered its voxels
+// with eight 2-byte loads per operand, and one atomic per wave and weight),
+// 99 us now.
 // ---------------------------------------------------------------------------
 struct ConvWgradArgs {
-  const bf16_t *x;
+  const bf16_t *x;      // [V][ldx], channels [0, cin); ldx a multiple of 8
   int ldx, cin, ktot;
-  const bf16_t *g;      // gradient w.r.t. the pre-activation output [V][ldg]
+  const bf16_t *g;      // gradient w.r.t. the pre-activation output [V][ldg]; ldg a multiple of 8
   int ldg;
   float *dw;            // [cout][ktot]
   int dx, dy, dz;
-  long long vchunk;     // voxels per wave (multiple of 32)
+  int ctiles;           // 16-channel tiles of the input
+  int ylen;             // rows of X per strip
 };
 
-template <int KT>
-__global__ __launch_bounds__(64) void k_conv_wgrad(ConvWgradArgs a)
+typedef short short4v __attribute__((ext_vector_type(4)));
+
+// The transpose of a 16 x 16 tile: lane l gives voxel l%16, channels 4*(l/16)..+3
+// (raw), and gets voxels 4*(l/16)..+3 of channel l%16.
+__device__ __forceinline__ uint2 transpose16(uint2 raw, short4v ident)
 {
-  const int lane = threadIdx.x, r = lane & 15, oct = lane >> 4;
-  const long long V = (long long)a.dx * a.dy * a.dz;
-  const int n0 = blockIdx.y * 16;
-  const int kk0 = blockIdx.x * 16 * KT;
-  const long long vb = (long long)blockIdx.z * a.vchunk;
-  if (vb >= V) return;
-  const long long ve = vb + a.vchunk < V ? vb + a.vchunk : V;
-  int cc[KT], ox[KT], oy[KT], oz[KT];
-  bool kv[KT];
+  const f32x4 d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(short4v, raw), ident,
+                                                            f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+  uint2 r;
+  r.x = __builtin_amdgcn_perm(__float_as_uint(d[1]), __float_as_uint(d[0]), 0x07060302u);
+  r.y = __builtin_amdgcn_perm(__float_as_uint(d[3]), __float_as_uint(d[2]), 0x07060302u);
+  return r;
+}
+
+__global__ __launch_bounds__(256, 2) void k_conv_wgrad(ConvWgradArgs a)
+{
+  __shared__ float sum[27 * 256];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, oct = lane >> 4;
+  const int c0 = 16 * ((int)blockIdx.y % a.ctiles), n0 = 16 * ((int)blockIdx.y / a.ctiles);
+  const int nxt = (a.dx + 31) / 32, nys = (a.dy + a.ylen - 1) / a.ylen;
+  const int strips = nxt * nys * a.dz;
+  const int cch = c0 + 4 * oct;          // this lane's four input channels
+  const bool cin_ok = cch < a.cin;       // cin is 8 or a multiple of 16
+  short4v ident;
 #pragma unroll
-  for (int t = 0; t < KT; ++t) {
-    const int kk = kk0 + 16 * t + r;
-    kv[t] = kk < a.ktot;
-    const int tap = kv[t] ? kk / a.cin : 0;
-    cc[t] = kv[t] ? kk - tap * a.cin : 0;
-    ox[t] = tap % 3 - 1;
-    oy[t] = (tap / 3) % 3 - 1;
-    oz[t] = tap / 9 - 1;
+  for (int i = 0; i < 4; ++i) ident[i] = 4 * oct + i == r ? (short)0x3f80 : (short)0;
+  f32x4 acc[27];
+#pragma unroll
+  for (int t = 0; t < 27; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint2 zero2 = make_uint2(0u, 0u);
+
+  for (int strip = (int)blockIdx.x * 4 + wave; strip < strips; strip += (int)gridDim.x * 4) {
+    const int xt = strip % nxt, ys = strip / nxt % nys, z = strip / (nxt * nys);
+    const int x0 = 32 * xt, y0 = ys * a.ylen, y1 = y0 + a.ylen < a.dy ? y0 + a.ylen : a.dy;
+    // a row's 2 x 16 voxels of X at the three shifts / of g; 0 outside the volume
+    auto load_x = [&](int y, uint2 (*v)[2]) {
+      const bf16_t *row = a.x + ((long long)z * a.dy + y) * a.dx * a.ldx + cch;
+#pragma unroll
+      for (int s = 0; s < 3; ++s)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int x = x0 + 16 * h + r + s - 1;
+          v[s][h] = y < y1 && cin_ok && x >= 0 && x < a.dx ? *reinterpret_cast<const uint2 *>(row + (long long)x * a.ldx)
+                                                           : zero2;
+        }
+    };
+    auto load_g = [&](int y, uint2 (*v)[2]) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const int zz = z + q - 1;
+        const bool in = y >= 0 && y < a.dy && zz >= 0 && zz < a.dz;
+        const bf16_t *row = a.g + ((long long)zz * a.dy + y) * a.dx * a.ldg + n0 + 4 * oct;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int x = x0 + 16 * h + r;
+          v[q][h] = in && x < a.dx ? *reinterpret_cast<const uint2 *>(row + (long long)x * a.ldg) : zero2;
+        }
+      }
+    };
+    auto operand = [&](const uint2 *v) {
+      const uint2 lo = transpose16(v[0], ident), hi = transpose16(v[1], ident);
+      return as_bf16x8(make_uint4(lo.x, lo.y, hi.x, hi.y));
+    };
+    bf16x8 G[3][3];  // g rows y-1, y, y+1 (first index), z-1, z, z+1
+    uint2 rx[3][2], rg[3][2];
+    load_g(y0 - 1, rg);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) G[1][q] = operand(rg[q]);
+    load_g(y0, rg);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) G[2][q] = operand(rg[q]);
+    load_g(y0 + 1, rg);
+    load_x(y0, rx);
+    for (int y = y0; y < y1; ++y) {
+      bf16x8 X[3];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        G[0][q] = G[1][q];
+        G[1][q] = G[2][q];
+        G[2][q] = operand(rg[q]);
+        X[q] = operand(rx[q]);
+      }
+      load_g(y + 2, rg);
+      load_x(y + 1, rx);
+      // X row (y, z) meets g row (y - oy, z - oz) at tap (ox, oy, oz)
+#pragma unroll
+      for (int oz = -1; oz <= 1; ++oz)
+#pragma unroll
+        for (int oy = -1; oy <= 1; ++oy)
+#pragma unroll
+          for (int ox = -1; ox <= 1; ++ox) {
+            const int t = (oz + 1) * 9 + (oy + 1) * 3 + ox + 1;
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(G[1 - oy][1 - oz], X[ox + 1], acc[t], 0, 0, 0);
+          }
+    }
   }
-  f32x4 acc[KT];
+  // lane holds D[n0 + 4*oct + i][c0 + r] of every tap
+  for (int w = 0; w < 4; ++w) {
+    if (wave == w) {
 #pragma unroll
-  for (int t = 0; t < KT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const long long plane = (long long)a.dx * a.dy;
-  for (long long v0 = vb; v0 < ve; v0 += 32) {
-    unsigned short ga[8];
-    int px[8], py[8], pz[8];
-    bool pv[8];
+      for (int t = 0; t < 27; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float *p = sum + t * 256 + (4 * oct + i) * 16 + r;
+          *p = w == 0 ? acc[t][i] : *p + acc[t][i];
+        }
+    }
+    __syncthreads();
+  }
+  const int c = c0 + (threadIdx.x & 15);
+  if (c < a.cin)
+    for (int t = 0; t < 27; ++t)
+      atomicAdd(a.dw + (long long)(n0 + (threadIdx.x >> 4)) * a.ktot + t * a.cin + c, sum[t * 256 + threadIdx.x]);
+}
+
+// Backward of bias and ReLU, in place: g <- g where y > 0, else 0, and
+// db[c] += sum of it.  With gpool (the gradient of the 2x2x2 average pool's
+// output, [V/8][ch]) g first takes its eighth.  Eight channels (16 bytes) per
+// thread, so one pass over g and y: at 128x128x64 with 16 channels 47 us (27
+// without gpool), against 59 + 43 + 69 (30 + 63) in kernels of one element a
+// thread.
+__global__ __launch_bounds__(256) void k_relu_bias_bwd(bf16_t *g, int ldg, const bf16_t *y, int ldy, int ch,
+                                                       long long V, const bf16_t *gpool, int dx, int dy, float *db)
+{
+  const int groups = ch >> 3, per = 256 / groups;  // ch is 16, 32, 64 or 128
+  const int c8 = 8 * ((int)threadIdx.x % groups);
+  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (long long v = (long long)blockIdx.x * per + threadIdx.x / groups; v < V; v += (long long)gridDim.x * per) {
+    uint4 t = *reinterpret_cast<const uint4 *>(g + v * ldg + c8);
+    const uint4 m = *reinterpret_cast<const uint4 *>(y + v * ldy + c8);
+    uint4 pl = make_uint4(0u, 0u, 0u, 0u);
+    if (gpool) {
+      const unsigned vv = (unsigned)v;
+      const unsigned x = vv % (unsigned)dx, yy = vv / (unsigned)dx % (unsigned)dy, z = vv / ((unsigned)dx * (unsigned)dy);
+      const unsigned vp = ((z >> 1) * ((unsigned)dy >> 1) + (yy >> 1)) * ((unsigned)dx >> 1) + (x >> 1);
+      pl = *reinterpret_cast<const uint4 *>(gpool + (size_t)vp * ch + c8);
+    }
+    unsigned o[4];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const long long v = v0 + 8 * oct + e;
-      pv[e] = v < ve;
-      const long long vv = pv[e] ? v : 0;
-      ga[e] = pv[e] ? a.g[vv * a.ldg + n0 + r] : (unsigned short)0;
-      px[e] = (int)(vv % a.dx);
-      py[e] = (int)((vv / a.dx) % a.dy);
-      pz[e] = (int)(vv / plane);
+      float f = bf_at(t, e);
+      if (gpool) f = bf2f(f2bf(f + 0.125f * bf_at(pl, e)));
+      f = bf_at(m, e) > 0.f ? f : 0.f;
+      s[e] += f;
+      const unsigned h = __float_as_uint(f) >> 16;  // f is a BF16 value
+      o[e >> 1] = (e & 1) ? o[e >> 1] | (h << 16) : h;
     }
-    uint4 ua;
-    ua.x = ga[0] | ((unsigned)ga[1] << 16);
-    ua.y = ga[2] | ((unsigned)ga[3] << 16);
-    ua.z = ga[4] | ((unsigned)ga[5] << 16);
-    ua.w = ga[6] | ((unsigned)ga[7] << 16);
-    const bf16x8 av = as_bf16x8(ua);
-#pragma unroll
-    for (int t = 0; t < KT; ++t) {
-      unsigned short xb[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int nx = px[e] + ox[t], ny = py[e] + oy[t], nz = pz[e] + oz[t];
-        const bool ok = pv[e] && kv[t] && nx >= 0 && nx < a.dx && ny >= 0 && ny < a.dy && nz >= 0 && nz < a.dz;
-        const long long nv = ((long long)nz * a.dy + ny) * a.dx + nx;
-        xb[e] = ok ? a.x[nv * a.ldx + cc[t]] : (unsigned short)0;
-      }
-      uint4 ub;
-      ub.x = xb[0] | ((unsigned)xb[1] << 16);
-      ub.y = xb[2] | ((unsigned)xb[3] << 16);
-      ub.z = xb[4] | ((unsigned)xb[5] << 16);
-      ub.w = xb[6] | ((unsigned)xb[7] << 16);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, as_bf16x8(ub), acc[t], 0, 0, 0);
-    }
+    *reinterpret_cast<uint4 *>(g + v * ldg + c8) = make_uint4(o[0], o[1], o[2], o[3]);
   }
+  __shared__ float red[256 * 9];
 #pragma unroll
-  for (int t = 0; t < KT; ++t) {
-    const int kk = kk0 + 16 * t + r;
-    if (!kv[t]) continue;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) atomicAdd(a.dw + (long long)(n0 + 4 * oct + i) * a.ktot + kk, acc[t][i]);
-  }
-}
-
-// bias gradient: db[n] += sum_v g[v][n]
-__global__ __launch_bounds__(256) void k_bias_grad(const bf16_t *g, int ldg, int cout, long long V,
-                                                   long long vchunk, float *db)
-{
-  const int groups = 256 / cout;
-  const int n = threadIdx.x % cout, grp = threadIdx.x / cout;
-  const long long vb = (long long)blockIdx.x * vchunk;
-  const long long ve = vb + vchunk < V ? vb + vchunk : V;
-  float s = 0.f;
-  if (grp < groups)
-    for (long long v = vb + grp; v < ve; v += groups) s += bf2f(g[v * ldg + n]);
-  __shared__ float red[256];
-  red[threadIdx.x] = s;
+  for (int e = 0; e < 8; ++e) red[threadIdx.x * 9 + e] = s[e];
   __syncthreads();
-  if (threadIdx.x < cout) {
+  if ((int)threadIdx.x < ch) {
     float t = 0.f;
-    for (int q = 0; q < groups; ++q) t += red[q * cout + threadIdx.x];
+    for (int q = 0; q < per; ++q) t += red[(q * groups + (int)threadIdx.x / 8) * 9 + (threadIdx.x & 7)];
     atomicAdd(db + threadIdx.x, t);
   }
-}
-
-// g <- g * (y > 0), both [V][ld] slices of `ch` channels
-__global__ __launch_bounds__(256) void k_relu_bwd(bf16_t *g, int ldg, int goff, const bf16_t *y, int ldy,
-                                                  int yoff, int ch, long long V)
-{
-  const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (q >= V * ch) return;
-  const long long v = q / ch;
-  const int c = (int)(q - v * ch);
-  if (!(bf2f(y[v * ldy + yoff + c]) > 0.f)) g[v * ldg + goff + c] = 0;
 }
 
 // 2x2x2 average pool: out[V/8][ldo] <- in[V][ldi] (channels [ioff, ioff+ch))
@@ -419,22 +503,6 @@ __global__ __launch_bounds__(256) void k_pool_fwd(const bf16_t *in, int ldi, int
   out[vo * ldo + c] = f2bf(s * 0.125f);
 }
 
-// gin[child] += gout[parent] / 8
-__global__ __launch_bounds__(256) void k_pool_bwd_add(const bf16_t *gout, int ldo, bf16_t *gin, int ldi, int ioff,
-                                                      int ch, int odx, int ody, int odz)
-{
-  const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
-  const long long Vi = 8LL * odx * ody * odz;
-  if (q >= Vi * ch) return;
-  const long long vi = q / ch;
-  const int c = (int)(q - vi * ch);
-  const int idx = 2 * odx, idy = 2 * ody;
-  const int x = (int)(vi % idx), y = (int)((vi / idx) % idy), z = (int)(vi / ((long long)idx * idy));
-  const long long vo = ((long long)(z >> 1) * ody + (y >> 1)) * odx + (x >> 1);
-  bf16_t &d = gin[vi * ldi + ioff + c];
-  d = f2bf(bf2f(d) + 0.125f * bf2f(gout[vo * ldo + c]));
-}
-
 // nearest 2x upsample: out[V][ldo] (channels [ooff, ooff+ch)) <- in[V/8][ldi]
 __global__ __launch_bounds__(256) void k_up_fwd(const bf16_t *in, int ldi, bf16_t *out, int ldo, int ooff, int ch,
                                                 int dx, int dy, int dz)
@@ -449,36 +517,36 @@ __global__ __launch_bounds__(256) void k_up_fwd(const bf16_t *in, int ldi, bf16_
   out[v * ldo + ooff + c] = in[vp * ldi + c];
 }
 
-// gin[parent] = sum of gout over its 8 children
+// gin[parent] = sum of gout over its 8 children, eight channels per thread
 __global__ __launch_bounds__(256) void k_up_bwd(const bf16_t *gout, int ldo, int ooff, bf16_t *gin, int ldi, int ch,
                                                 int pdx, int pdy, int pdz)
 {
+  const unsigned g = (unsigned)ch >> 3;
   const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
   const long long Vp = (long long)pdx * pdy * pdz;
-  if (q >= Vp * ch) return;
-  const long long vp = q / ch;
-  const int c = (int)(q - vp * ch);
+  if (q >= Vp * g) return;
+  const long long vp = q / g;
+  const int c8 = 8 * (int)(q - vp * g);
   const int x = (int)(vp % pdx), y = (int)((vp / pdx) % pdy), z = (int)(vp / ((long long)pdx * pdy));
   const int dx = 2 * pdx, dy = 2 * pdy;
-  float s = 0.f;
+  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int b = 0; b < 8; ++b) {
     const long long v = ((long long)(2 * z + (b >> 2)) * dy + (2 * y + ((b >> 1) & 1))) * dx + 2 * x + (b & 1);
-    s += bf2f(gout[v * ldo + ooff + c]);
+    const uint4 t = *reinterpret_cast<const uint4 *>(gout + v * ldo + ooff + c8);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s[e] += bf_at(t, e);
   }
-  gin[vp * ldi + c] = f2bf(s);
+  unsigned o[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = (unsigned)f2bf(s[2 * e]) | ((unsigned)f2bf(s[2 * e + 1]) << 16);
+  *reinterpret_cast<uint4 *>(gin + vp * ldi + c8) = make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-// The same three data-movement steps with 8 channels (16 bytes) per thread
+// The forward data-movement steps with 8 channels (16 bytes) per thread
 // and 32-bit index math, for channel counts, strides and offsets that are
 // multiples of 8 and V * ch / 8 < 2^32 (the host checks): same arithmetic in
 // the same order per channel, so the same results.
-__device__ inline float bf_at(const uint4 &t, int e)
-{
-  const unsigned w = e < 2 ? t.x : e < 4 ? t.y : e < 6 ? t.z : t.w;
-  return __uint_as_float((e & 1) ? (w & 0xffff0000u) : (w << 16));
-}
-
 __global__ __launch_bounds__(256) void k_pool_fwd8(const bf16_t *in, int ldi, int ioff, bf16_t *out, int ldo, int ch,
                                                    int odx, int ody, int odz)
 {
@@ -543,31 +611,42 @@ __global__ __launch_bounds__(256) void k_head_fwd(const bf16_t *x, int ldx, int 
   y[v] = s;
 }
 
-// head backward: gx[v][c] = gy[v] W[c]; dW[c] += sum gy x; db += sum gy
+// head backward: gx[v][c] = gy[v] W[c]; dW[c] += sum gy x; db += sum gy.
+// Eight channels per thread, a work-group sums many voxels before its one
+// atomic per weight (878 us at 128x128x64 with a tree reduction in LDS per
+// channel and 256 voxels, 25 us now).
 __global__ __launch_bounds__(256) void k_head_bwd(const bf16_t *x, int ldx, int ch, const float *w, const float *gy,
                                                   bf16_t *gx, float *dw, long long V)
 {
-  const long long v = (long long)blockIdx.x * 256 + threadIdx.x;
-  __shared__ float red[256];
-  float acc[33];
-  for (int c = 0; c <= ch; ++c) acc[c] = 0.f;
-  if (v < V) {
+  const int groups = ch >> 3, per = 256 / groups;
+  const int c8 = 8 * ((int)threadIdx.x % groups);
+  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, sg = 0.f, wr[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) wr[e] = w[c8 + e];
+  for (long long v = (long long)blockIdx.x * per + threadIdx.x / groups; v < V; v += (long long)gridDim.x * per) {
     const float g = gy[v];
-    for (int c = 0; c < ch; ++c) {
-      gx[v * ldx + c] = f2bf(g * w[c]);
-      acc[c] = g * bf2f(x[v * ldx + c]);
+    const uint4 t = *reinterpret_cast<const uint4 *>(x + v * ldx + c8);
+    unsigned o[4];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      s[e] += g * bf_at(t, e);
+      const unsigned h = f2bf(g * wr[e]);
+      o[e >> 1] = (e & 1) ? o[e >> 1] | (h << 16) : h;
     }
-    acc[ch] = g;
+    sg += g;
+    *reinterpret_cast<uint4 *>(gx + v * ldx + c8) = make_uint4(o[0], o[1], o[2], o[3]);
   }
-  for (int c = 0; c <= ch; ++c) {
-    red[threadIdx.x] = acc[c];
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-      if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) atomicAdd(dw + c, red[0]);
-    __syncthreads();
+  __shared__ float red[256 * 9];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) red[threadIdx.x * 9 + e] = s[e];
+  red[threadIdx.x * 9 + 8] = sg;
+  __syncthreads();
+  if ((int)threadIdx.x <= ch) {
+    // thread ch sums the gradient itself, from the first channel group
+    const int grp = (int)threadIdx.x < ch ? (int)threadIdx.x / 8 : 0, e = (int)threadIdx.x < ch ? (int)threadIdx.x & 7 : 8;
+    float t = 0.f;
+    for (int q = 0; q < per; ++q) t += red[(q * groups + grp) * 9 + e];
+    atomicAdd(dw + threadIdx.x, t);
   }
 }
 
@@ -938,31 +1017,30 @@ hipError_t launch_conv_fwd(hipStream_t s, const ConvFwdArgs &a, int cout)
   return hipGetLastError();
 }
 
+// Work-groups of the weight gradient: two per CU over all channel pairs (its
+// registers allow two waves per SIMD), and strips of at least 8 rows of X,
+// shorter than the volume only as far as there are work-groups for them.
 hipError_t launch_wgrad(hipStream_t s, const ConvWgradArgs &a0, int cout)
 {
   ConvWgradArgs a = a0;
-  const long long V = (long long)a.dx * a.dy * a.dz;
-  constexpr int KT = 4;
-  const int kblocks = (a.ktot + 16 * KT - 1) / (16 * KT);
-  const int nblocks = cout / 16;
-  // about 8192 waves in flight, voxel chunks of >= 256
-  long long splits = 8192 / (kblocks * nblocks);
-  if (splits < 1) splits = 1;
-  long long chunk = (V + splits - 1) / splits;
-  chunk = (chunk + 31) / 32 * 32;
-  if (chunk < 256) chunk = 256;
-  splits = (V + chunk - 1) / chunk;
-  a.vchunk = chunk;
-  hipLaunchKernelGGL(k_conv_wgrad<KT>, dim3(kblocks, nblocks, (unsigned)splits), dim3(64), 0, s, a);
+  a.ctiles = (a.cin + 15) / 16;
+  const int pairs = a.ctiles * (cout / 16);
+  const long long columns = (long long)((a.dx + 31) / 32) * a.dz;
+  const long long waves = 2048 / pairs > 4 ? 2048 / pairs : 4;
+  a.ylen = a.dy;
+  while (a.ylen > 8 && columns * ((a.dy + a.ylen - 1) / a.ylen) < waves) a.ylen = (a.ylen + 1) / 2;
+  const long long strips = columns * ((a.dy + a.ylen - 1) / a.ylen);
+  const long long blocks = (strips < waves ? strips : waves) + 3;
+  hipLaunchKernelGGL(k_conv_wgrad, dim3((unsigned)(blocks / 4), (unsigned)pairs), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
-hipError_t launch_bias_grad(hipStream_t s, const bf16_t *g, int ldg, int cout, long long V, float *db)
+// Work-groups of the kernels that reduce over voxels, eight channels per
+// thread: enough to fill the GPU, few enough for their atomics.
+inline unsigned reduce_blocks(long long V, int ch)
 {
-  const long long chunk = 4096;
-  hipLaunchKernelGGL(k_bias_grad, dim3((unsigned)((V + chunk - 1) / chunk)), dim3(256), 0, s, g, ldg, cout, V,
-                     chunk, db);
-  return hipGetLastError();
+  const long long b = (V * (ch / 8) + 255) / 256;
+  return (unsigned)(b < 1024 ? b : 1024);
 }
 
 // One conv layer forward: x (ldx, cin) -> y (ldy at ycoff), bias + ReLU
@@ -973,22 +1051,23 @@ hipError_t conv_forward(qesmc_unet *u, const Conv &cv, const Level &lv, const bf
   return launch_conv_fwd(u->stream, a, cv.cout);
 }
 
-// Backward through one conv layer whose ReLU output y (ldy, yoff) received
-// the gradient g (ldg, goff) (masked in place); x is its input.  Adds dW, db;
-// if gx is given, writes dL/dx into it (ldgx, cin channels at offset 0).
+// Backward through one conv layer whose ReLU output y (ldy) received the
+// gradient g (ldg; masked in place, after gpool's share if given); x is its
+// input.  Adds dW, db; if gx is given, writes dL/dx into it (ldgx, cin
+// channels at offset 0).
 hipError_t conv_backward(qesmc_unet *u, const Conv &cv, const Level &lv, const bf16_t *x, int ldx,
-                         const bf16_t *y, int ldy, int yoff, bf16_t *g, int ldg, int goff, bf16_t *gx, int ldgx)
+                         const bf16_t *y, int ldy, bf16_t *g, int ldg, const bf16_t *gpool, bf16_t *gx, int ldgx)
 {
   hipStream_t s = u->stream;
   const long long V = lv.V;
-  hipLaunchKernelGGL(k_relu_bwd, g1(V * cv.cout), dim3(256), 0, s, g, ldg, goff, y, ldy, yoff, cv.cout, V);
+  hipLaunchKernelGGL(k_relu_bias_bwd, dim3(reduce_blocks(V, cv.cout)), dim3(256), 0, s, g, ldg, y, ldy, cv.cout, V,
+                     gpool, lv.dx, lv.dy, u->gp + cv.boff);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  ConvWgradArgs wa{x, ldx, cv.cin, 27 * cv.cin, g + goff, ldg, u->gp + cv.woff, lv.dx, lv.dy, lv.dz, 0};
+  ConvWgradArgs wa{x, ldx, cv.cin, 27 * cv.cin, g, ldg, u->gp + cv.woff, lv.dx, lv.dy, lv.dz, 0, 0};
   if ((e = launch_wgrad(s, wa, cv.cout)) != hipSuccess) return e;
-  if ((e = launch_bias_grad(s, g + goff, ldg, cv.cout, V, u->gp + cv.boff)) != hipSuccess) return e;
   if (gx) {
-    ConvFwdArgs a{g + goff, ldg, cv.cout, 27 * cv.cout, cv.wd, cv.kpd, nullptr, gx, ldgx, 0, lv.dx, lv.dy, lv.dz, 0};
+    ConvFwdArgs a{g, ldg, cv.cout, 27 * cv.cout, cv.wd, cv.kpd, nullptr, gx, ldgx, 0, lv.dx, lv.dy, lv.dz, 0};
     if ((e = launch_conv_fwd(s, a, cv.cin)) != hipSuccess) return e;
   }
   return hipSuccess;
@@ -1065,35 +1144,32 @@ hipError_t backward(qesmc_unet *u, const bf16_t *feat)
   hipError_t e;
   const int L = u->L;
   Level &top = u->lv[0];
-  hipLaunchKernelGGL(k_head_bwd, g1(top.V), dim3(256), 0, s, top.D, top.c, top.c, u->p + u->head_off, u->gout,
-                     top.gD, u->gp + u->head_off, top.V);
+  hipLaunchKernelGGL(k_head_bwd, dim3(reduce_blocks(top.V, top.c)), dim3(256), 0, s, top.D, top.c, top.c,
+                     u->p + u->head_off, u->gout, top.gD, u->gp + u->head_off, top.V);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   for (int l = 0; l + 1 < L; ++l) {
     Level &lv = u->lv[l];
     Level &dn = u->lv[l + 1];
-    if ((e = conv_backward(u, u->dec2[l], lv, lv.E, lv.c, lv.D, lv.c, 0, lv.gD, lv.c, 0, lv.gE, lv.c)) != hipSuccess)
+    if ((e = conv_backward(u, u->dec2[l], lv, lv.E, lv.c, lv.D, lv.c, lv.gD, lv.c, nullptr, lv.gE, lv.c)) != hipSuccess)
       return e;
-    if ((e = conv_backward(u, u->dec1[l], lv, lv.CAT, lv.ldcat, lv.E, lv.c, 0, lv.gE, lv.c, 0, lv.gCAT, lv.ldcat)) !=
+    if ((e = conv_backward(u, u->dec1[l], lv, lv.CAT, lv.ldcat, lv.E, lv.c, lv.gE, lv.c, nullptr, lv.gCAT, lv.ldcat)) !=
         hipSuccess)
       return e;
     bf16_t *gsrc = (l == L - 2) ? dn.gCAT : dn.gD;
     const int ldg = (l == L - 2) ? dn.ldcat : dn.c;
-    hipLaunchKernelGGL(k_up_bwd, g1(dn.V * dn.c), dim3(256), 0, s, lv.gCAT, lv.ldcat, lv.c, gsrc, ldg, dn.c, dn.dx,
+    hipLaunchKernelGGL(k_up_bwd, g1(dn.V * dn.c / 8), dim3(256), 0, s, lv.gCAT, lv.ldcat, lv.c, gsrc, ldg, dn.c, dn.dx,
                        dn.dy, dn.dz);
   }
   for (int l = L - 1; l >= 0; --l) {
     Level &lv = u->lv[l];
-    if (l + 1 < L) {
-      Level &dn = u->lv[l + 1];
-      hipLaunchKernelGGL(k_pool_bwd_add, g1(lv.V * lv.c), dim3(256), 0, s, dn.gP, lv.c, lv.gCAT, lv.ldcat, 0, lv.c,
-                         dn.dx, dn.dy, dn.dz);
-    }
-    if ((e = conv_backward(u, u->enc2[l], lv, lv.A, lv.c, lv.CAT, lv.ldcat, 0, lv.gCAT, lv.ldcat, 0, lv.gA, lv.c)) !=
+    // the encoder output's gradient: the skip's share, plus the pool's from below
+    const bf16_t *gpool = l + 1 < L ? u->lv[l + 1].gP : nullptr;
+    if ((e = conv_backward(u, u->enc2[l], lv, lv.A, lv.c, lv.CAT, lv.ldcat, lv.gCAT, lv.ldcat, gpool, lv.gA, lv.c)) !=
         hipSuccess)
       return e;
     const bf16_t *in = l == 0 ? feat : lv.P;
     const int ldin = l == 0 ? QESMC_UNET_IN_CHANNELS : u->lv[l - 1].c;
-    if ((e = conv_backward(u, u->enc1[l], lv, in, ldin, lv.A, lv.c, 0, lv.gA, lv.c, 0, l > 0 ? lv.gP : nullptr,
+    if ((e = conv_backward(u, u->enc1[l], lv, in, ldin, lv.A, lv.c, lv.gA, lv.c, nullptr, l > 0 ? lv.gP : nullptr,
                            ldin)) != hipSuccess)
       return e;
   }
