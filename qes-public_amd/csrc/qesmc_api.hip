@@ -36,7 +36,8 @@ hipError_t qesmc_launch_fill_u32(qesmc_ctx *x, unsigned *p, long long count, uns
 hipError_t qesmc_launch_rows_summary(qesmc_ctx *x, int launched, float tol);
 hipError_t qesmc_fused_prepare(qesmc_ctx *x);
 long long qesmc_march_top_words(const qesmc::Dims &d);
-void qesmc_march_choose(qesmc_ctx *x, int tile_k, const int *top);
+void qesmc_march_costs(qesmc_ctx *x, const int *top);
+void qesmc_march_choose(qesmc_ctx *x, int tile_k);
 
 namespace {
 
@@ -388,7 +389,7 @@ float row_max(const unsigned *row)
 
 // Validation, optional re-encoding, tiling, convergence rows, lambda packing
 // and R, on the context's current stream (ev[0] .. ev[1]).
-int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, bool batch)
+int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, BatchKind batch)
 {
   if (!x || !pp) return QESMC_ERR_ARG;
   if (!x->have_geom || !x->have_inflow) return QESMC_ERR_STATE;
@@ -428,8 +429,9 @@ int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, bool batch)
   // mask, unless the caller or the autotuner tiles the colour passes, a
   // no-allocation run finds its buffers missing, or a plane is beyond its
   // 32-bit byte offsets.
-  st.march = !batch && x->d.splane < (1LL << 28) && x->d.NZ < 32768 &&
+  st.march = batch != BatchKind::colours && x->d.splane < (1LL << 28) && x->d.NZ < 32768 &&
              (st.path == QESMC_PATH_FUSED ||
+              (batch == BatchKind::march && st.masked && x->nsplit < (1LL << 31)) ||
               (p.path == QESMC_PATH_AUTO && st.masked && x->nsplit < (1LL << 31) && p.tile_k == 0 &&
                p.tile_v == 0 && p.wg_per_cu == 0 && p.slab_planes == 0 && x->kplanes_auto == 0 &&
                x->tile_v_auto == 0 && x->wg_per_cu_auto == 0 && (!x->no_alloc_run || march_ready)));
@@ -523,14 +525,15 @@ int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, bool batch)
   if (st.march) {
     if (!x->pair_masks) {
       HIPCHK(qesmc_fused_prepare(x));
-      x->pair_masks = true;
       x->march_tile_k = -1;
-    }
-    if (x->march_tile_k != p.tile_k) {
       std::vector<int> top((size_t)qesmc_march_top_words(x->d));
       HIPCHK(hipMemcpyAsync(top.data(), x->d_top, sizeof(int) * top.size(), hipMemcpyDeviceToHost, s));
       HIPCHK(hipStreamSynchronize(s));
-      qesmc_march_choose(x, p.tile_k, top.data());
+      qesmc_march_costs(x, top.data());
+      x->pair_masks = true;
+    }
+    if (batch == BatchKind::none && x->march_tile_k != p.tile_k) {
+      qesmc_march_choose(x, p.tile_k);
       x->march_tile_k = p.tile_k;
     }
     HIPCHK(qesmc_launch_pack_pairs(x, true));

@@ -1,7 +1,9 @@
 // Batched solves: many independent problems (uneven sizes, one context each)
-// relaxed by one kernel launch per colour pass, and the tile autotuner.
+// relaxed by one kernel launch per colour pass, or, where every member has a
+// wall-mask encoding, per two iterations (the march, qesmc_sor_fused.hip),
+// and the tile autotuner.
 //
-// Every instance keeps its own colour-split arrays, stencil encoding and
+// The colour passes: every instance keeps its own colour-split arrays, stencil encoding and
 // convergence rows; a device table describes them.  Wave tiles are numbered
 // over all instances (instance-major, then plane chunk, then position); a
 // wave finds its instance by binary search of the table's tile offsets,
@@ -12,9 +14,11 @@
 // solved alone.  Iterations can be replayed as a captured HIP graph: the
 // iteration number then comes from a device counter advanced by the graph.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <vector>
 
+#include "qesmc_march.h"
 #include "qesmc_sor_tile.h"
 
 hipError_t qesmc_launch_set_u32(qesmc_ctx *x, unsigned *p, unsigned v);
@@ -180,7 +184,12 @@ __global__ __launch_bounds__(256) void k_sor_batch(const BatchItem *__restrict__
   }
 }
 
-__global__ void k_advance(int *t_base, int by) { t_base[0] += by; }
+// the next replay's iterations and launches
+__global__ void k_advance(int *t_base, int by, int launches)
+{
+  t_base[0] += by;
+  t_base[1] += launches;
+}
 
 // number of instances whose row t is still above tol (t = t_base[0] + t_off)
 __global__ __launch_bounds__(64) void k_count_active(const BatchItem *items, int n, const int *t_base, int t_off,
@@ -276,6 +285,12 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
     if (!kb) kb = bk ? bk : 4;
     if (!vq) vq = bv ? bv : 2;
   }
+  // The march (two iterations per launch) where no tiling of the colour passes
+  // is asked for and every member has a wall-mask encoding: 16 cities of
+  // 64-256 cells a side (29.6 M cells) relax in 70 us per iteration instead of 112.
+  bool march = params->path == QESMC_PATH_AUTO && params->tile_k == 0 && params->tile_v == 0 && params->wg_per_cu == 0;
+  if (!(params->flags & QESMC_RUN_REENCODE))
+    for (int i = 0; i < n; ++i) march = march && ctxs[i]->compressible;
   qesmc_params pv = *params;
   pv.tile_v = vq;
   pv.tile_k = kb;
@@ -296,7 +311,14 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
   };
   std::vector<RunState> st(n);
   int rc = QESMC_OK;
-  for (int i = 0; i < n && rc == QESMC_OK; ++i) rc = run_prepare(ctxs[i], params, st[i], true);
+  for (;;) {
+    for (int i = 0; i < n && rc == QESMC_OK; ++i)
+      rc = run_prepare(ctxs[i], params, st[i], march ? BatchKind::march : BatchKind::colours);
+    bool all = true;
+    for (int i = 0; i < n; ++i) all = all && st[i].march;
+    if (rc != QESMC_OK || !march || all) break;
+    march = false;  // a member that cannot: colour passes for all
+  }
   if (rc != QESMC_OK) {
     (void)hipStreamSynchronize(bs);
     restore();
@@ -330,6 +352,7 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
   }
   BatchItem *d_items = nullptr;
   int *d_t = nullptr, *d_active = nullptr, *h_active = nullptr;
+  MarchItem *d_march = nullptr;  // the members' tiles in launches of one and of two iterations
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -337,6 +360,7 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (graph) (void)hipGraphDestroy(graph);
     if (d_items) (void)hipFree(d_items);
+    if (d_march) (void)hipFree(d_march);
     if (d_t) (void)hipFree(d_t);
     if (d_active) (void)hipFree(d_active);
     if (h_active) (void)hipHostFree(h_active);
@@ -351,13 +375,82 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
   };
   hipError_t e;
   if ((e = hipMalloc((void **)&d_items, sizeof(BatchItem) * n)) != hipSuccess) return fail(e);
-  if ((e = hipMalloc((void **)&d_t, sizeof(int))) != hipSuccess) return fail(e);
+  if ((e = hipMalloc((void **)&d_t, 2 * sizeof(int))) != hipSuccess) return fail(e);
   if ((e = hipMalloc((void **)&d_active, sizeof(int))) != hipSuccess) return fail(e);
   if ((e = hipHostMalloc((void **)&h_active, sizeof(int), hipHostMallocDefault)) != hipSuccess) return fail(e);
   if ((e = hipEventCreate(&e0)) != hipSuccess || (e = hipEventCreate(&e1)) != hipSuccess) return fail(e);
   if ((e = hipMemcpyAsync(d_items, items.data(), sizeof(BatchItem) * n, hipMemcpyHostToDevice, bs)) != hipSuccess)
     return fail(e);
   if ((e = qesmc_launch_set_u32(lead, (unsigned *)d_t, 0u)) != hipSuccess) return fail(e);
+  if ((e = qesmc_launch_set_u32(lead, (unsigned *)d_t + 1, 0u)) != hipSuccess) return fail(e);
+  // The march may take the members in groups, each for check_every iterations
+  // in turn, so that a group's arrays (13 bytes a cell) stay in the 256 MB
+  // Infinity Cache: what leaves it costs a launch up to 0.6 of its time more
+  // (16 cities of 64-256 cells a side, 385 MB: 1.2 times the expected time).
+  // Against that stand fuller launches, so the number of groups is the one
+  // with the least expected time.
+  struct Group {
+    int begin, end;  // members
+    int shape[2], slots[2], which[2];
+    std::vector<MarchPlan> plans;  // for two iterations a launch
+  };
+  std::vector<Group> groups;
+  std::vector<MarchItem> mitems(march ? 2 * (size_t)n : 0);
+  std::vector<int> which;  // the member of each work-group, per group and iterations per launch
+  if (march) {
+    constexpr double kCache = 256.0 * (1 << 20);
+    double bytes = 0.0, least = 1e300;
+    for (int i = 0; i < n; ++i) bytes += 13.0 * (double)ctxs[i]->ncell;
+    const int most = bytes <= kCache ? 1 : (int)std::min((double)n, std::ceil(bytes / (0.5 * kCache)));
+    for (int count = 1; count <= most; count += count < 4 ? 1 : count) {
+      std::vector<Group> trial;
+      double us = 0.0, done = 0.0;
+      for (int i = 0; i < n;) {
+        Group gr{i, i, {}, {}, {}, {}};
+        double mine = 0.0;
+        // up to the next multiple of the share, to the nearest member
+        const double until = bytes * (double)(trial.size() + 1) / count;
+        while (gr.end < n) {
+          const double b = 13.0 * (double)ctxs[gr.end]->ncell;
+          if (gr.end > i && done + 0.5 * b > until) break;
+          done += b;
+          mine += b;
+          ++gr.end;
+        }
+        double t = 0.0;
+        gr.shape[1] = qesmc_march_batch_plan(ctxs + i, gr.end - i, 2, gr.plans, &t);
+        if (gr.shape[1] < 0) return fail(hipErrorInvalidValue);
+        us += t * (mine > kCache ? 1.0 + 0.6 * (1.0 - kCache / mine) : 1.0);
+        i = gr.end;
+        trial.push_back(std::move(gr));
+      }
+      if (us < least) {
+        least = us;
+        groups = std::move(trial);
+      }
+    }
+    std::vector<MarchPlan> single;
+    for (Group &gr : groups) {
+      const int m = gr.end - gr.begin;
+      gr.shape[0] = qesmc_march_batch_plan(ctxs + gr.begin, m, 1, single, nullptr);
+      if (gr.shape[0] < 0) return fail(hipErrorInvalidValue);
+      for (int T = 1; T <= 2; ++T) {
+        gr.which[T - 1] = (int)which.size();
+        for (int i = 0; i < m; ++i) {
+          MarchItem &it = mitems[(size_t)(T - 1) * n + gr.begin + i];
+          qesmc_march_item(ctxs[gr.begin + i], T == 1 ? single[(size_t)i] : gr.plans[(size_t)i], gr.slots[T - 1], it);
+          which.insert(which.end(), (size_t)it.slots, gr.begin + i);
+          gr.slots[T - 1] += it.slots;
+        }
+      }
+    }
+    const size_t tb = sizeof(MarchItem) * mitems.size();
+    if ((e = hipMalloc((void **)&d_march, tb + sizeof(int) * (which.size() + 1))) != hipSuccess) return fail(e);
+    if ((e = hipMemcpyAsync(d_march, mitems.data(), tb, hipMemcpyHostToDevice, bs)) != hipSuccess) return fail(e);
+    if ((e = hipMemcpyAsync(d_march + mitems.size(), which.data(), sizeof(int) * which.size(), hipMemcpyHostToDevice,
+                            bs)) != hipSuccess)
+      return fail(e);
+  }
 
   bool all_masked = true;
   for (int i = 0; i < n; ++i) all_masked = all_masked && st[i].masked;
@@ -405,24 +498,57 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
 #undef QESMC_BATCH_LAUNCH
       }
     };
-    if (use_graph) {
+    auto launch_march = [&](const Group &gr, int iters, const int *base, int t, int src, bool fix) -> hipError_t {
+      if (gr.slots[iters - 1] == 0) return hipSuccess;
+      MarchRun run{};
+      for (float &w : run.om) w = p.omega;
+      run.tol = p.tol;
+      run.t = t;
+      run.itermax = p.itermax;
+      run.src = src;
+      run.fix = fix ? 1 : 0;
+      run.items = d_march + (size_t)(iters - 1) * n;
+      run.which = reinterpret_cast<const int *>(d_march + 2 * (size_t)n) + gr.which[iters - 1];
+      run.base = base;
+      return qesmc_launch_march_batch(bs, iters, gr.shape[iters - 1], gr.slots[iters - 1], run);
+    };
+    // iterations [t, t + count) by twos, reading buffer set src & 1 first
+    auto march_chunk = [&](const int *base, int t, int count, int src) -> hipError_t {
+      for (const Group &gr : groups)
+        for (int j = 0; j < count; j += 2) {
+          const hipError_t le = launch_march(gr, j + 2 <= count ? 2 : 1, base, t + j, (src + j / 2) & 1, false);
+          if (le != hipSuccess) return le;
+        }
+      return hipSuccess;
+    };
+    const bool replay = use_graph && (!march || p.itermax >= C);
+    int launches = 0;
+    if (replay) {
       // one captured chunk of C iterations, advancing the device counter
       if ((e = hipStreamBeginCapture(bs, hipStreamCaptureModeThreadLocal)) != hipSuccess) return fail(e);
-      for (int j = 0; j < C; ++j) launch_iter(d_t, j);
-      hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, bs, d_t, C);
+      if (march)
+        e = march_chunk(d_t, 0, C, 0);
+      else
+        for (int j = 0; j < C; ++j) launch_iter(d_t, j);
+      hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, bs, d_t, C, (C + 1) / 2);
       if ((e = hipStreamEndCapture(bs, &graph)) != hipSuccess) return fail(e);
       if ((e = hipGraphInstantiate(&gexec, graph, nullptr, nullptr, 0)) != hipSuccess) return fail(e);
     }
     bool stop = false;
     while (launched < p.itermax && !stop) {
       const int chunk = std::min(C, p.itermax - launched);
-      if (use_graph) {
+      // the march's launches hold two iterations, so a last chunk that itermax cuts short is not replayed
+      const bool whole = replay && (!march || chunk == C);
+      if (whole) {
         if ((e = hipGraphLaunch(gexec, bs)) != hipSuccess) return fail(e);
+      } else if (march) {
+        if ((e = march_chunk(nullptr, launched, chunk, launches)) != hipSuccess) return fail(e);
       } else {
         for (int j = 0; j < chunk; ++j) launch_iter(nullptr, launched + j);
         if ((e = hipGetLastError()) != hipSuccess) return fail(e);
       }
-      launched += use_graph ? C : chunk;
+      launches += (chunk + 1) / 2;
+      launched += whole ? C : chunk;
       if (launched >= p.itermax) break;
       // instances still open at the next iteration
       hipLaunchKernelGGL(k_count_active, dim3(1), dim3(64), 0, bs, d_items, n, nullptr, launched, p.itermax, p.tol,
@@ -433,6 +559,13 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
       if (*h_active == 0) stop = true;
     }
     if (launched > p.itermax) launched = p.itermax;
+    if (march) {
+      // where a member's run ended, and the last launch redone up to it if that is inside
+      e = qesmc_march_settle_batch(bs, d_march, n, launched, p.tol);
+      for (const Group &gr : groups)
+        if (e == hipSuccess) e = launch_march(gr, 1, nullptr, 0, 0, true);
+      if (e != hipSuccess) return fail(e);
+    }
   }
   if ((e = hipEventRecord(e1, bs)) != hipSuccess) return fail(e);
   for (int i = 0; i < n; ++i) {

@@ -198,6 +198,7 @@ struct qesmc_ctx {
   int slab_planes_auto = 0;    // default when qesmc_params.slab_planes == 0
   qesmc::MarchPlan march[2];   // tiling of the march's launches of one and of two iterations
   int march_tile_k = -1;       // the tile_k they were chosen for (-1: not chosen)
+  std::vector<double> march_cost; // cost of the march's steps below each plane (with pair_masks)
   int n_cu = 256;              // compute units of the device
 };
 
@@ -211,8 +212,10 @@ struct RunState {
   bool march = false;       // whole iterations per launch on the pair layout
   bool first_runs = false;
 };
-// batch: prepared for qesmc_run_batch, which relaxes a colour per launch
-int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, bool batch = false);
+// batch: prepared for qesmc_run_batch, to relax a colour per launch or to
+// march (RunState.march tells whether it can)
+enum class BatchKind { none, colours, march };
+int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, BatchKind batch = BatchKind::none);
 int run_finish(qesmc_ctx *x, const RunState &st, int launched, qesmc_result *res);
 int run_solve(qesmc_ctx *x, const qesmc_params *pp, qesmc_result *res);
 int run_loop(qesmc_ctx *x, const RunState &st, int *launched);

@@ -36,11 +36,12 @@
 // (one wave per half-sweep, one mask per lane), and where all masks of a wave's
 // rows are open (no wall: most of a city's planes) the six coefficients are
 // the layer's wall values themselves, in scalar registers.
+#include <algorithm>
 #include <cstring>
 #include <type_traits>
 #include <vector>
 
-#include "qesmc_internal.h"
+#include "qesmc_march.h"
 
 hipError_t qesmc_launch_fill_u32(qesmc_ctx *x, unsigned *p, long long count, unsigned v);
 
@@ -110,33 +111,15 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *p, unsig
 
 typedef unsigned uint2v __attribute__((ext_vector_type(2)));
 
-struct MarchArgs {
-  Dims d;
-  int nq, nyt;        // x tiles, y tiles
-  int ntiles;
-  float2 *set0, *set1;  // lambda, the two buffer sets
-  const float2 *R;
-  const unsigned *mask;
-  const int *top;     // highest plane with a wall, per two rows and 32 pairs
-  const unsigned *canon8;  // wall values per plane, 8 words (6 used)
-  const float *sums;       // sum of the wall values each of the 64 masks selects, per plane
-  float om[4];        // omega of each half-sweep (2T used)
-  float tol;
-  unsigned *err;
-  int t, itermax;
-  unsigned *status;
-  unsigned *cur;      // the set holding the latest iterate
-  int src;            // set this launch reads
-  int fix;            // redo the last launch's first iteration if asked to (T = 1 only)
-  short begin[kMaxSegments + 1];  // first plane of each segment (odd), then the end
-};
-
 }  // namespace
 
 // T iterations per launch, NW waves per work-group, RW rows (even) per row
 // group, GW lanes per row group (64: a wave is one group; 32: two).
-template <int T, int NW, int RW, int GW>
-__global__ __launch_bounds__(64 * NW, RW == 2 ? 4 : 2) void k_sor_march(MarchArgs A)
+// BATCH: the work-group's problem is taken from A.items (A.which per
+// work-group) instead of I, and the iteration and source set from A.base, so
+// that a captured launch can be replayed.
+template <int T, int NW, int RW, int GW, bool BATCH>
+__global__ __launch_bounds__(64 * NW, RW == 2 ? 4 : 2) void k_sor_march(MarchItem I, MarchRun A)
 {
   constexpr int H = 2 * T;      // half-sweeps
   constexpr int U = 2 * T + 4;  // ring slots (planes p-2T .. p+2 are live); even
@@ -148,38 +131,49 @@ __global__ __launch_bounds__(64 * NW, RW == 2 ? 4 : 2) void k_sor_march(MarchArg
   __shared__ float wd_tab[2][H][64];
   __shared__ __align__(16) unsigned cv_tab[2][H][8];
   __shared__ float wmax[NW][T];
-  const Dims &d = A.d;
+  const int problem = BATCH ? A.which[blockIdx.x] : 0;
+  const MarchItem *const ip = BATCH ? A.items + problem : nullptr;
+#define QESMC_ITEM(f) (BATCH ? ip->f : I.f)
+#define QESMC_ITEM_PTR(f) (BATCH ? (decltype(I.f))as_global(ip->f) : I.f)
+  const Dims d = QESMC_ITEM(d);
+  unsigned *const err = QESMC_ITEM_PTR(err), *const status = QESMC_ITEM_PTR(status), *const cur = QESMC_ITEM_PTR(cur);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int t = A.t, src = A.src;
+  if (BATCH && A.base) {
+    t += A.base[0];
+    src ^= A.base[1] & 1;
+  }
   float om[H];
 #pragma unroll
   for (int h = 0; h < H; ++h) om[h] = A.om[h];
   if (T == 1 && A.fix) {
     // the last launch ran T iterations but the run ended inside it
-    if (!A.status[kFixGo]) return;
-    t = (int)A.status[kLastT];
-    src = (int)(A.cur[0] ^ 1u);
-    om[0] = __uint_as_float(A.status[kLastOmega]);
-    om[1] = __uint_as_float(A.status[kLastOmega + 1]);
+    if (!status[kFixGo]) return;
+    t = (int)status[kLastT];
+    src = (int)(cur[0] ^ 1u);
+    om[0] = __uint_as_float(status[kLastOmega]);
+    om[1] = __uint_as_float(status[kLastOmega + 1]);
   } else {
     if (t >= A.itermax) return;
   }
-  // XCD x (work-group id % 8) takes the x-th eighth of the tile range, tiles
-  // numbered x fastest, then y, then segment: neighbours that share halos
-  // march together on one L2
-  const int per = (int)gridDim.x / kXcds;  // the grid is a multiple of 8
-  const int tile = (int)(blockIdx.x % kXcds) * per + (int)(blockIdx.x / kXcds);
-  if (tile >= A.ntiles) return;
-  const int tq = tile % A.nq;
-  const int ty = (tile / A.nq) % A.nyt;
-  const int tz = tile / (A.nq * A.nyt);
+  // XCD x (work-group id % 8) takes the x-th eighth of the problem's tile
+  // range, tiles numbered x fastest, then y, then segment: neighbours that
+  // share halos march together on one L2
+  const int slot = (int)blockIdx.x - QESMC_ITEM(first);
+  const int per = QESMC_ITEM(slots) / kXcds;  // slots and first are multiples of 8
+  const int tile = (slot % kXcds) * per + slot / kXcds;
+  if (tile >= QESMC_ITEM(ntiles)) return;
+  const int nq = QESMC_ITEM(nq), nyt = QESMC_ITEM(nyt);
+  const int tq = tile % nq;
+  const int ty = (tile / nq) % nyt;
+  const int tz = tile / (nq * nyt);
 
   // columns: this lane's half-cell, and whether this tile owns it
   const int half = (d.NX + 1) >> 1;
   const int gl = lane & (GW - 1);
   const int q = tq * (GW - 2 * T) + gl;
-  const bool lown = q < half && (tq == 0 || gl >= T) && (tq == A.nq - 1 || gl < GW - T);
+  const bool lown = q < half && (tq == 0 || gl >= T) && (tq == nq - 1 || gl < GW - T);
   const unsigned qc = (unsigned)(q < half ? q : half - 1);
   const bool col[2] = {q < half && 2 * q >= 1 && 2 * q <= d.NX - 2, 2 * q + 1 <= d.NX - 2};
   // rows of this lane's group
@@ -187,7 +181,7 @@ __global__ __launch_bounds__(64 * NW, RW == 2 ? 4 : 2) void k_sor_march(MarchArg
   const int jt = ty * (YR - 4 * T);
   const int j0 = jt + group * RW;
   const int jown0 = ty == 0 ? 0 : jt + 2 * T;
-  const int jown1 = ty == A.nyt - 1 ? d.NY : jt + YR - 2 * T;
+  const int jown1 = ty == nyt - 1 ? d.NY : jt + YR - 2 * T;
   bool upd[RW][2], own[RW];
   unsigned voff[RW], moff[RW / 2];  // byte offsets within a plane of lambda and R, of masks
 #pragma unroll
@@ -202,15 +196,15 @@ __global__ __launch_bounds__(64 * NW, RW == 2 ? 4 : 2) void k_sor_march(MarchArg
     if (a % 2 == 0) moff[a / 2] = ((jc / 2u) * (unsigned)d.HP + qc) * 4u;
   }
   // planes: owned [ka, kb); half-sweep h relaxes [lo(h), hi(h)]
-  const int ka = A.begin[tz], kb = A.begin[tz + 1];
+  const int ka = QESMC_ITEM(begin[tz]), kb = QESMC_ITEM(begin[tz + 1]);
   const int pfirst = ka - (H - 1) > 0 ? ka - (H - 1) : 0;  // even
   const int plast = kb - 1 + (H - 1);
-  const float2 *__restrict__ in = src ? A.set1 : A.set0;
-  float2 *__restrict__ out = src ? A.set0 : A.set1;
-  const float2 *__restrict__ R = A.R;
-  const unsigned *__restrict__ mask = A.mask;
-  const unsigned *__restrict__ canon8 = A.canon8;
-  const float *__restrict__ sums = A.sums;
+  const float2 *__restrict__ in = src ? QESMC_ITEM_PTR(set1) : QESMC_ITEM_PTR(set0);
+  float2 *__restrict__ out = src ? QESMC_ITEM_PTR(set0) : QESMC_ITEM_PTR(set1);
+  const float2 *__restrict__ R = QESMC_ITEM_PTR(R);
+  const unsigned *__restrict__ mask = QESMC_ITEM_PTR(mask);
+  const unsigned *__restrict__ canon8 = QESMC_ITEM_PTR(canon8);
+  const float *__restrict__ sums = QESMC_ITEM_PTR(sums);
   const unsigned plane8 = (unsigned)d.splane * 8u, planem = (unsigned)((d.NY + 1) / 2) * (unsigned)d.HP * 4u;
   // this wave's half-sweep of the tables
   float omw = om[0];
@@ -302,18 +296,19 @@ __global__ __launch_bounds__(64 * NW, RW == 2 ? 4 : 2) void k_sor_march(MarchArg
   int wtop = 0;
   {
     const int nqb = (d.HP + 31) / 32;
+    const int *__restrict__ top = QESMC_ITEM_PTR(top);
 #pragma unroll
-    for (int a = 0; a < RW; a += 2) wtop = max(wtop, A.top[(j0 + a < d.NY ? j0 + a : d.NY - 1) / 2 * nqb + (int)qc / 32]);
+    for (int a = 0; a < RW; a += 2) wtop = max(wtop, top[(j0 + a < d.NY ? j0 + a : d.NY - 1) / 2 * nqb + (int)qc / 32]);
   }
   // the gate is read while those loads are in flight
   if (!(T == 1 && A.fix)) {
-    if (!gate_pass_multi(A.err, t, A.tol, A.status, lane)) return;  // identical in every wave of the grid
+    if (!gate_pass_multi(err, t, A.tol, status, lane)) return;  // identical in every wave of the grid
     if (tile == 0 && threadIdx.x == 0) {
-      *A.cur = (unsigned)(src ^ 1);
-      A.status[kLastT] = (unsigned)t;
-      A.status[kLastIters] = (unsigned)T;
-      A.status[kLastOmega] = __float_as_uint(om[0]);
-      A.status[kLastOmega + 1] = __float_as_uint(om[1]);
+      *cur = (unsigned)(src ^ 1);
+      status[kLastT] = (unsigned)t;
+      status[kLastIters] = (unsigned)T;
+      status[kLastOmega] = __float_as_uint(om[0]);
+      status[kLastOmega + 1] = __float_as_uint(om[1]);
     }
   }
   // Buildings stand on the ground: below the highest wall of its columns a
@@ -438,7 +433,7 @@ __global__ __launch_bounds__(64 * NW, RW == 2 ? 4 : 2) void k_sor_march(MarchArg
   for (; p0 <= plast && p0 - (H - 1) <= wtop; p0 += U) block(p0, std::false_type{});
 #pragma unroll 1
   for (; p0 <= plast; p0 += U) block(p0, std::true_type{});
-  if (bad) atomicMin(A.status + kBadAt, (unsigned)(t + T - 1));
+  if (bad) atomicMin(status + kBadAt, (unsigned)(t + T - 1));
 #pragma unroll
   for (int i = 0; i < T; ++i) {
     float m = 0.f;
@@ -452,22 +447,29 @@ __global__ __launch_bounds__(64 * NW, RW == 2 ? 4 : 2) void k_sor_march(MarchArg
     float m = 0.f;
     for (int w = 0; w < NW; ++w) m = fmaxf(m, wmax[w][threadIdx.x]);
     if (m > 0.f)
-      atomicMax(A.err + (long long)(t + 1 + (int)threadIdx.x) * kErrSlots + (blockIdx.x % kErrSlots),
+      atomicMax(err + (long long)(t + 1 + (int)threadIdx.x) * kErrSlots + (blockIdx.x % kErrSlots),
                 __float_as_uint(m));
   }
 }
+#undef QESMC_ITEM
+#undef QESMC_ITEM_PTR
 
 // End of a stretch of launches over iterations [.., hi): find the iteration
 // the run ended at (rows below lo were scanned before), and if that is inside
 // the last launch, order its first iteration to be redone on its own.
-__global__ __launch_bounds__(256) void k_sor_settle(const unsigned *__restrict__ rows, int lo, int hi, float tol,
-                                                    unsigned *__restrict__ status)
+// With items, of each of them (one work-group per problem).
+__global__ __launch_bounds__(1024) void k_sor_settle(const MarchItem *__restrict__ items, const unsigned *rows, int lo,
+                                                     int hi, float tol, unsigned *status)
 {
+  if (items) {
+    rows = items[blockIdx.x].err;
+    status = items[blockIdx.x].status;
+  }
   __shared__ unsigned first;
   if (threadIdx.x == 0) first = 0xffffffffu;
   __syncthreads();
   // one wave per row, one slot per lane
-  for (int t = lo + (int)(threadIdx.x >> 6); t < hi; t += 4) {
+  for (int t = lo + (int)(threadIdx.x >> 6); t < hi; t += 16) {
     const float v = __uint_as_float(rows[(long long)t * kErrSlots + (threadIdx.x & 63)]);
     const float m = wave_max(v > 0.f ? v : 0.f);
     if ((threadIdx.x & 63) == 0 && !(m > tol)) atomicMin(&first, (unsigned)t);
@@ -548,6 +550,7 @@ namespace {
 // The instantiated shapes for two iterations per launch: waves, lanes per row group (two rows per group).
 constexpr int kShapes[][2] = {{4, 32}, {8, 32}, {16, 32}, {16, 64}};
 constexpr int kTail = 1;  // the shape of the single-iteration launches
+constexpr int kBatchShape = 1;  // and of a batch's, or the one before it
 constexpr int kWavesPerCu = 16;  // 128 vector registers each
 
 // Columns of tiles (x tiles, y tiles) of a shape.
@@ -612,10 +615,33 @@ double balance_segments(const std::vector<double> &sum, int T, int end, int nseg
   return worst;
 }
 
+// Microseconds of one step with n waves on the CU, and what rows of 32 pairs cost on top.
+double step_us(int waves) { return 0.62 + 0.054 * waves; }
+double narrow_factor(int gw, bool beyond) { return gw == 64 ? 1.0 : beyond ? 1.15 : 1.04; }
+constexpr double kLaunchUs = 4.6;
+
 }  // namespace
 
-// The march's shape and segments for the resident domain.  top: the table of
-// highest walls.  A segment's time is the sum of its steps' and the launch's
+// The cost of the steps below p, for all p, from the table of highest walls:
+// 1 for an open plane, and 0.32 more for the share of the columns that have a wall there or above.
+void qesmc_march_costs(qesmc_ctx *x, const int *top)
+{
+  const Dims &d = x->d;
+  std::vector<double> w((size_t)d.NZ, 1.0);
+  const long long n = qesmc_march_top_words(d);
+  std::vector<int> count((size_t)d.NZ + 1, 0);
+  for (long long q = 0; q < n; ++q) ++count[(size_t)top[q]];
+  long long above = n;
+  for (int k = 0; k < d.NZ; ++k) {
+    w[(size_t)k] = 1.0 + 0.32 * (double)above / (double)n;
+    above -= count[(size_t)k];
+  }
+  x->march_cost.assign((size_t)d.NZ + 4, 0.0);
+  for (size_t p = 0; p + 1 < x->march_cost.size(); ++p)
+    x->march_cost[p + 1] = x->march_cost[p] + w[p < w.size() ? p : w.size() - 1];
+}
+
+// The march's shape and segments for the resident domain.  A segment's time is the sum of its steps' and the launch's
 // that of the dearest segment.  Measured with 16 waves on a CU: 1.97 us a step
 // where every plane has walls (298 vector instructions a wave: the vector ALUs
 // are busy throughout), 1.49 us where none has (172; bound by the caches), so
@@ -624,23 +650,11 @@ double balance_segments(const std::vector<double> &sum, int T, int end, int nseg
 // Rows of 32 pairs touch a fifth more cache lines than rows of 64: 4 % slower
 // per step, 15 % where they come from HBM.
 // tile_k > 0 sets the planes per segment.
-void qesmc_march_choose(qesmc_ctx *x, int tile_k, const int *top)
+void qesmc_march_choose(qesmc_ctx *x, int tile_k)
 {
   const Dims &d = x->d;
   const int end = d.NZ - 1;
-  std::vector<double> w((size_t)d.NZ, 1.0);
-  if (top) {
-    const long long n = qesmc_march_top_words(d);
-    std::vector<int> count((size_t)d.NZ + 1, 0);
-    for (long long q = 0; q < n; ++q) ++count[(size_t)top[q]];
-    long long above = n;
-    for (int k = 0; k < d.NZ; ++k) {
-      w[(size_t)k] = 1.0 + 0.32 * (double)above / (double)n;  // the share whose top is at k or higher
-      above -= count[(size_t)k];
-    }
-  }
-  std::vector<double> sum((size_t)d.NZ + 4, 0.0);
-  for (size_t p = 0; p + 1 < sum.size(); ++p) sum[p + 1] = sum[p] + w[p < w.size() ? p : w.size() - 1];
+  const std::vector<double> &sum = x->march_cost;
   auto uniform = [&](int T, int planes, MarchPlan &m) {
     int seg = planes < 2 * T ? 2 * T : (planes + 1) / 2 * 2;
     while ((end - 1 + seg - 1) / seg > kMaxSegments) seg += 2;
@@ -675,8 +689,8 @@ void qesmc_march_choose(qesmc_ctx *x, int tile_k, const int *top)
         }
         const long long per = (columns * m.nseg + x->n_cu - 1) / x->n_cu;
         const int resident = per < fit ? (int)per : fit;
-        const double narrow = kShapes[c][1] == 64 ? 1.0 : beyond ? 1.15 : 1.04;
-        const double us = 4.6 + (double)((per + fit - 1) / fit) * worst * (0.62 + 0.054 * kShapes[c][0] * resident) * narrow;
+        const double us = kLaunchUs + (double)((per + fit - 1) / fit) * worst * step_us(kShapes[c][0] * resident) *
+                                          narrow_factor(kShapes[c][1], beyond);
         if (us < best) {
           best = us;
           plan = m;
@@ -700,23 +714,18 @@ hipError_t qesmc_fused_prepare(qesmc_ctx *x)
   return hipGetLastError();
 }
 
-// Launch iterations t .. t + iters - 1 (iters 1 or 2), reading buffer set
-// src and writing the other; om holds omega of the red and black pass of each.
-// With fix, redo what k_sor_settle ordered instead.
-hipError_t qesmc_launch_march(qesmc_ctx *x, int t, int iters, int itermax, const float *om, float tol, int src, bool fix)
+// The march's view of a problem whose tiles are those of m; first: its first work-group of the launch.
+void qesmc_march_item(const qesmc_ctx *x, const MarchPlan &m, int first, MarchItem &a)
 {
   const Dims &d = x->d;
-  if (d.NZ - 2 < 1 || d.NY - 2 < 1) return hipSuccess;
-  const MarchPlan &m = x->march[iters - 1];
-  const int nw = kShapes[m.shape][0], gw = kShapes[m.shape][1];
-  const int ntiles = m.nq * m.nyt * m.nseg;
-  const int blocks = (ntiles + kXcds - 1) / kXcds * kXcds;
-  MarchArgs a{};
+  a = MarchItem{};
   a.d = d;
   a.nq = m.nq;
   a.nyt = m.nyt;
-  a.ntiles = ntiles;
-  std::memcpy(a.begin, m.begin, sizeof(a.begin));
+  a.ntiles = m.nq * m.nyt * m.nseg;
+  a.first = first;
+  a.slots = (a.ntiles + kXcds - 1) / kXcds * kXcds;
+  for (int q = 0; q <= m.nseg; ++q) a.begin[q] = m.begin[q];
   a.set0 = reinterpret_cast<float2 *>(x->d_lc[0]);
   a.set1 = reinterpret_cast<float2 *>(x->d_lc2[0]);
   a.R = reinterpret_cast<const float2 *>(x->d_Rc[0]);
@@ -724,33 +733,140 @@ hipError_t qesmc_launch_march(qesmc_ctx *x, int t, int iters, int itermax, const
   a.top = x->d_top;
   a.canon8 = x->d_canon8;
   a.sums = reinterpret_cast<const float *>(x->d_canon8 + 8LL * d.NZ);
-  for (int h = 0; h < 2 * iters; ++h) a.om[h] = om[h];
-  a.tol = tol;
   a.err = x->d_err;
-  a.t = t;
-  a.itermax = itermax;
   a.status = x->d_status;
   a.cur = x->d_cur;
-  a.src = src;
-  a.fix = fix ? 1 : 0;
+}
+
+namespace {
+
+template <bool BATCH>
+hipError_t launch_shape(hipStream_t s, int iters, int shape, int blocks, const MarchItem &item, const MarchRun &run)
+{
+  const int nw = kShapes[shape][0], gw = kShapes[shape][1];
 #define QESMC_MARCH_LAUNCH(T, N, R, G) \
-  hipLaunchKernelGGL((k_sor_march<T, N, R, G>), dim3((unsigned)blocks), dim3(64 * N), 0, x->stream, a)
+  hipLaunchKernelGGL((k_sor_march<T, N, R, G, BATCH>), dim3((unsigned)blocks), dim3(64 * N), 0, s, item, run)
   if (iters == 1) QESMC_MARCH_LAUNCH(1, 8, 2, 32);
   else if (nw == 4) QESMC_MARCH_LAUNCH(2, 4, 2, 32);
   else if (nw == 8) QESMC_MARCH_LAUNCH(2, 8, 2, 32);
+  else if constexpr (BATCH) return hipErrorInvalidValue;
   else if (gw == 32) QESMC_MARCH_LAUNCH(2, 16, 2, 32);
   else QESMC_MARCH_LAUNCH(2, 16, 2, 64);
 #undef QESMC_MARCH_LAUNCH
   return hipGetLastError();
 }
 
+}  // namespace
+
+// Launch iterations t .. t + iters - 1 (iters 1 or 2), reading buffer set
+// src and writing the other; om holds omega of the red and black pass of each.
+// With fix, redo what k_sor_settle ordered instead.
+hipError_t qesmc_launch_march(qesmc_ctx *x, int t, int iters, int itermax, const float *om, float tol, int src, bool fix)
+{
+  const Dims &d = x->d;
+  if (d.NZ - 2 < 1 || d.NY - 2 < 1) return hipSuccess;
+  MarchItem item;
+  qesmc_march_item(x, x->march[iters - 1], 0, item);
+  MarchRun a{};
+  for (int h = 0; h < 2 * iters; ++h) a.om[h] = om[h];
+  a.tol = tol;
+  a.t = t;
+  a.itermax = itermax;
+  a.src = src;
+  a.fix = fix ? 1 : 0;
+  return launch_shape<false>(x->stream, iters, x->march[iters - 1].shape, item.slots, item, a);
+}
+
 // The run's end over iterations [lo, hi) and, if it falls inside the last
 // launch, that launch redone up to it.
 hipError_t qesmc_march_settle(qesmc_ctx *x, int lo, int hi, float tol)
 {
-  hipLaunchKernelGGL(k_sor_settle, dim3(1), dim3(256), 0, x->stream, x->d_err, lo, hi, tol, x->d_status);
+  hipLaunchKernelGGL(k_sor_settle, dim3(1), dim3(1024), 0, x->stream, nullptr, x->d_err, lo, hi, tol, x->d_status);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const float om[2] = {0.f, 0.f};  // taken from the launch that is redone
   return qesmc_launch_march(x, 0, 1, 1, om, tol, 0, true);
+}
+
+// One shape and a cut of every member for launches of T iterations over a
+// batch, and the microseconds such a launch is expected to take: in R rounds of
+// resident work-groups a launch takes R times its dearest segment, so for
+// each R the least segment cost whose tiles fit in R rounds, and the best R.
+// (Measured on 4 to 16 cities of 64-256 cells a side, 8 waves: 1.04-1.19 times that,
+// the most where the arrays leave the cache.  The smooth total cost over
+// the places misleads: 556 tiles on 512 places take two rounds.)  Two work-groups of 8 waves
+// per CU fill each other's barriers: at 16 such cities 83 us per iteration against
+// 99 and 101 with 16 waves of 32 and 64 lanes a row, so 16 waves are not
+// used; 4 waves only where the chip is not full.
+int qesmc_march_batch_plan(qesmc_ctx *const *ctxs, int n, int T, std::vector<MarchPlan> &plans, double *expect_us)
+{
+  double top = 0.0;
+  for (int i = 0; i < n; ++i) top = std::max(top, segment_cost(ctxs[i]->march_cost, T, 1, ctxs[i]->d.NZ - 1));
+  const int n_cu = ctxs[0]->n_cu;
+  std::vector<MarchPlan> trial((size_t)n);
+  long long tiles = 0;
+  double worst = 0.0;
+  auto cut_all = [&](int c, double limit) {
+    tiles = 0;
+    worst = 0.0;
+    for (int i = 0; i < n; ++i) {
+      const std::vector<double> &sum = ctxs[i]->march_cost;
+      MarchPlan &m = trial[(size_t)i];
+      m.shape = c;
+      m.nseg = 0;
+      if (ctxs[i]->d.NZ < 3 || ctxs[i]->d.NY < 3) continue;  // nothing to relax
+      march_columns(ctxs[i]->d, T, c, &m.nq, &m.nyt);
+      m.nseg = cut_segments(sum, T, ctxs[i]->d.NZ - 1, 2 * T, limit, m);
+      if (m.nseg == 0) return false;
+      for (int q = 0; q < m.nseg; ++q) worst = std::max(worst, segment_cost(sum, T, m.begin[q], m.begin[q + 1]));
+      tiles += (m.nq * m.nyt * m.nseg + kXcds - 1) / kXcds * kXcds;  // what the fullest XCD sees
+    }
+    return true;
+  };
+  double best = 1e300;
+  int shape = -1;
+  for (int c = T == 1 ? kTail : 0; c <= kBatchShape; ++c) {
+    const int fit = kWavesPerCu / kShapes[c][0];
+    auto us = [&]() {
+      const long long per = (tiles + n_cu - 1) / n_cu;
+      return kLaunchUs + (double)((per + fit - 1) / fit) * worst * step_us(kShapes[c][0] * (int)(per < fit ? per : fit)) *
+                             narrow_factor(kShapes[c][1], false);
+    };
+    auto take = [&]() {
+      if (us() >= best) return;
+      best = us();
+      plans = trial;
+      shape = c;
+    };
+    if (cut_all(c, top)) take();
+    const long long uncut = tiles;
+    // R in units of one work-group per CU up to the full chip, then of full chips
+    for (int r = 1; r <= (c == kBatchShape ? fit + 5 : fit); ++r) {
+      const long long places = (long long)n_cu * (r <= fit ? r : (r - fit + 1) * fit);
+      if (places <= uncut) continue;
+      double lo = 0.0, hi = top;
+      for (int it = 0; it < 10; ++it) {
+        const double mid = 0.5 * (lo + hi);
+        if (cut_all(c, mid) && tiles <= places) {
+          hi = mid;
+          take();
+        } else {
+          lo = mid;
+        }
+      }
+    }
+  }
+  if (expect_us) *expect_us = best;
+  return shape;
+}
+
+hipError_t qesmc_launch_march_batch(hipStream_t s, int iters, int shape, int blocks, const MarchRun &run)
+{
+  return launch_shape<true>(s, iters, shape, blocks, MarchItem{}, run);
+}
+
+hipError_t qesmc_march_settle_batch(hipStream_t s, const MarchItem *items, int n, int hi, float tol)
+{
+  hipLaunchKernelGGL(k_sor_settle, dim3((unsigned)n), dim3(1024), 0, s, items, nullptr, 0, hi, tol, nullptr);
+  return hipGetLastError();
 }
