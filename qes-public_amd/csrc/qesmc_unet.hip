@@ -18,6 +18,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <new>
 #include <random>
 #include <vector>
@@ -35,10 +36,10 @@ typedef unsigned short bf16_t;  // storage of one BF16 value
 
 __device__ inline bf16_t f2bf(float f)
 {
-  unsigned u = __float_as_uint(f);
-  if ((u & 0x7f800000u) == 0x7f800000u) return (bf16_t)((u >> 16) | ((u & 0xffffu) ? 0x40u : 0u));
-  u += 0x7fffu + ((u >> 16) & 1u);  // round to nearest even
-  return (bf16_t)(u >> 16);
+  const unsigned u = __float_as_uint(f);
+  const unsigned even = u + (0x7fffu + ((u >> 16) & 1u));             // round to nearest even
+  const unsigned keep = u | ((u & 0xffffu) ? 0x400000u : 0u);  // infinity, and NaN made quiet
+  return (bf16_t)(((u & 0x7f800000u) == 0x7f800000u ? keep : even) >> 16);
 }
 __device__ inline float bf2f(bf16_t h) { return __uint_as_float(((unsigned)h) << 16); }
 
@@ -57,15 +58,19 @@ __device__ inline bf16x8 as_bf16x8(uint4 u) { return __builtin_bit_cast(bf16x8, 
 struct ConvFwdArgs {
   const bf16_t *x;      // input [V][ldx], channels [0, cin)
   int ldx, cin, ktot;   // ktot = 27 * cin
-  const bf16_t *w;      // packed weights [cout][kp]
-  int kp;
+  int cout;
+  const bf16_t *w;      // packed weights (k_pack_w)
+  int kp;               // of a row of them (ConvKind::rows)
   const float *bias;    // [cout] or null
-  bf16_t *y;            // output [V][ldy] at channel offset ycoff
-  int ldy, ycoff;
+  bf16_t *y;            // output [V][ldy]
+  int ldy;
   int dx, dy, dz;
   int relu;
 };
 
+// Taps and channels in one sequence k = tap*cin + c, 32 at a time, both
+// operands gathered from L2: for channel counts that are neither one chunk
+// nor a multiple of 32, on volumes of few bricks (ConvKind::rows).
 // A wave computes MT tiles of 16 voxels x NT tiles of 16 output channels.
 // MFMA operand layout (16x16x32): lane l holds A[l%16][8*(l/16)+0..7],
 // B[8*(l/16)+0..7][l%16]; the result D[4*(l/16)+i][l%16].
@@ -101,44 +106,6 @@ __global__ __launch_bounds__(256) void k_conv_fwd(ConvFwdArgs a)
     ++tap;
   }
   const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
-  if (a.cin % 32 == 0) {
-    // Each 32-wide K step lies inside one tap: taps outer, channel chunks
-    // inner, same K order as below.  The A loads read a clamped in-bounds
-    // address and the zero padding is selected after the load, so the loads
-    // of several K steps can be in flight together (the small tiles of the
-    // deep levels run long K loops with one output tile per wave).
-    constexpr int kTapUnroll = MT * NT <= 2 ? 3 : 1;
-#pragma unroll kTapUnroll
-    for (int tap = 0; tap < 27; ++tap) {
-      const int ox = tap % 3 - 1, oy = (tap / 3) % 3 - 1, oz = tap / 9 - 1;
-      long long nvt[MT];
-      bool okt[MT];
-#pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        const int nx = vx[t] + ox, ny = vy[t] + oy, nz = vz[t] + oz;
-        okt[t] = vin[t] && nx >= 0 && nx < a.dx && ny >= 0 && ny < a.dy && nz >= 0 && nz < a.dz;
-        nvt[t] = okt[t] ? ((long long)nz * a.dy + ny) * a.dx + nx : 0;
-      }
-      for (int c0 = 0; c0 < a.cin; c0 += 32) {
-        const int cc = c0 + 8 * oct;
-        const int koct = tap * a.cin + cc;
-        bf16x8 av[MT];
-#pragma unroll
-        for (int t = 0; t < MT; ++t) {
-          const uint4 raw = *reinterpret_cast<const uint4 *>(a.x + nvt[t] * a.ldx + cc);
-          av[t] = as_bf16x8(okt[t] ? raw : zero4);
-        }
-#pragma unroll
-        for (int n = 0; n < NT; ++n) {
-          const bf16x8 bv =
-              as_bf16x8(*reinterpret_cast<const uint4 *>(a.w + (long long)(16 * (nb + n) + r) * a.kp + koct));
-#pragma unroll
-          for (int t = 0; t < MT; ++t)
-            acc[t][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[t], bv, acc[t][n], 0, 0, 0);
-        }
-      }
-    }
-  } else
   for (int kc = 0; kc < a.kp; kc += 32) {
     const int koct = kc + 8 * oct;
     const bool kvalid = koct < a.ktot;
@@ -175,117 +142,309 @@ __global__ __launch_bounds__(256) void k_conv_fwd(ConvFwdArgs a)
         if (m >= V) continue;
         float v = acc[t][n][i] + b;
         if (a.relu) v = v > 0.f ? v : 0.f;
-        as_global(a.y)[m * a.ldy + a.ycoff + col] = f2bf(v);
+        as_global(a.y)[m * a.ldy + col] = f2bf(v);
       }
     }
 }
 
 // ---------------------------------------------------------------------------
-// 3x3x3 convolution, forward, LDS-staged (used when cin is 8 or a multiple
-// of 16).  A work-group owns a brick of 8 x 8 x MT output voxels (4*MT
-// M-tiles of 16 voxels, MT per wave, x fastest) and all cout.  For each
-// chunk of CH input channels it stages the brick plus a one-voxel halo,
-// (10 x 10 x (MT+2)) x CH BF16, in LDS (zero outside the volume), then
-// every MFMA takes its A fragment from LDS at a per-tap constant offset:
-// with CH = 16 one 16x16x32 MFMA covers two taps x 16 channels, with CH = 8
-// four taps x 8 channels (27 taps padded to 28 with zeros).  K order
-// (tap-major, k = tap*cin + c) is the packed weights', so each lane's B
-// octet is 8 consecutive weights.
+// 3x3x3 convolution, forward, from bricks in LDS
+//
+// A work-group of four waves owns a brick of 16 x SY x SZ voxels: SY * SZ tiles
+// of 16 voxels along x.  It stages the brick and a halo of one voxel (zero
+// outside the volume), and every matrix operand is one 16-byte LDS read per
+// lane at a fixed offset from the lane's voxel.  The weights are the A operand
+// (rows are output channels) and the voxels the B operand, so a lane ends
+// with four consecutive channels of one voxel, an 8-byte store, and the
+// weights, stored in lane order, come in 1 KB loads.
+//
+// The order of a voxel's products is part of the result (activations are
+// rounded to BF16).  Two orders, by the volume (conv_kind):
+//   k_conv_chunks  chunks of CH = 16 channels (8 for the input) outermost, within
+//                  them 16-channel taps two by two (8-channel taps four by four)
+//   k_conv_whole   taps outermost, within them 32 channels at a time; all
+//                  channels are staged
+//
+// Within a voxel's 16-byte octets the octet index is XORed with bits of x, so
+// that the 16 lanes of an LDS phase (16 consecutive x, one octet) hit all
+// banks once.
+//
+// Bound: LDS, one 1 KB read per product (8 cycles of the CU's LDS where the
+// product takes 4 of its matrix cores), and the staging before it.  All
+// convolutions of a forward pass of 4 levels at 128x128x64 take 366 us, and took 972
+// with bricks of 8x8x4 whose reads hit half the banks, weights read by
+// output row (64 cache lines a load) and results stored two bytes at a
+// time, and, below 1024 of them, both operands gathered from L2 for each
+// product.  16 -> 16 channels at 128x128x64: 100 -> 34 us; 48 -> 16: 190 -> 80;
+// its gradient, 16 -> 48: 197 -> 84; 192 -> 64 at 32x32x16: 145 -> 30.
+// Operands in flight need the order of the code kept (sched_barrier): left to
+// itself the compiler reads each just before its product, 46 us instead of 34.
 // ---------------------------------------------------------------------------
-template <int NT, int MT, int CH>
-__global__ __launch_bounds__(256) void k_conv_fwd_lds(ConvFwdArgs a)
+typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+
+enum class ConvKind { chunks8, chunks16, whole, rows };
+
+constexpr int kBrickX = 16, kHaloX = kBrickX + 2;
+constexpr int kXcdsU = 8;  // work-groups are dealt to the XCDs in turn
+
+// The order of products for cin input channels on a volume, and so the kernel
+// and the weights' layout.  (One chunk, or one tap group, is the same in either order.)
+__host__ __device__ inline ConvKind conv_kind(int cin, int dx, int dy, int dz)
 {
-  constexpr int HX = 10, HY = 10, HZ = MT + 2, HV = HX * HY * HZ;  // halo brick
-  constexpr int OPT = CH / 8;                                      // lane octets per tap
-  constexpr int TPM = 4 / OPT;                                     // taps per MFMA
-  constexpr int NG = (27 + TPM - 1) / TPM;                         // MFMAs per channel chunk
-  __shared__ __attribute__((aligned(16))) bf16_t lds[HV * CH];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (cin == 8) return ConvKind::chunks8;
+  if (cin == 16) return ConvKind::chunks16;
+  const long long bricks = (long long)((dx + 7) / 8) * ((dy + 7) / 8) * ((dz + 3) / 4);
+  if (bricks >= 1024) return ConvKind::chunks16;
+  return cin % 32 == 0 ? ConvKind::whole : ConvKind::rows;
+}
+
+// BF16 values of the packed weights
+__host__ __device__ inline long long packed_weights(ConvKind k, int cin, int cout)
+{
+  switch (k) {
+  case ConvKind::chunks8: return (long long)(cout / 16) * 7 * 512;
+  case ConvKind::chunks16: return (long long)(cout / 16) * (cin / 16) * 14 * 512;
+  case ConvKind::whole: return (long long)(cout / 16) * 27 * (cin / 32) * 512;
+  default: return (long long)cout * ((27 * cin + 31) / 32 * 32);
+  }
+}
+
+// brick b of the XCD-ordered grid: x fastest, then y, then z; false past the end
+template <int SY, int SZ>
+__device__ __forceinline__ bool brick_origin(const ConvFwdArgs &a, int *x0, int *y0, int *z0)
+{
+  const unsigned nbx = (unsigned)(a.dx + kBrickX - 1) / kBrickX, nby = (unsigned)(a.dy + SY - 1) / SY,
+                 nbz = (unsigned)(a.dz + SZ - 1) / SZ;
+  const unsigned per = gridDim.x / kXcdsU, b = blockIdx.x % kXcdsU * per + blockIdx.x / kXcdsU;
+  const unsigned row = b / nbx, layer = row / nby;
+  if (layer >= nbz) return false;
+  *x0 = (int)(b - row * nbx) * kBrickX;
+  *y0 = (int)(row - layer * nby) * SY;
+  *z0 = (int)layer * SZ;
+  return true;
+}
+
+__device__ __forceinline__ uint2 pack_out(const f32x4 &acc, const float *b, int relu)
+{
+  float v[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v[i] = acc[i] + b[i];
+    if (relu) v[i] = v[i] > 0.f ? v[i] : 0.f;
+  }
+  return make_uint2((unsigned)f2bf(v[0]) | ((unsigned)f2bf(v[1]) << 16),
+                    (unsigned)f2bf(v[2]) | ((unsigned)f2bf(v[3]) << 16));
+}
+
+// SY = 8, SZ = 4: a wave takes one z and its 8 rows, with the chunk's 14 (7)
+// weight fragments in registers and seven voxel operands in flight.  grid.y
+// splits the output channels.  WIDE: the brick's planes pass 31 bits of offset.
+template <int CH, bool WIDE>
+__global__ __launch_bounds__(256, 3) void k_conv_chunks(ConvFwdArgs a)
+{
+  constexpr int SY = 8, SZ = 4, HY = SY + 2, HZ = SZ + 2, HV = kHaloX * HY * HZ;
+  constexpr int OPT = CH / 8;               // octets per voxel
+  constexpr int TPM = 4 / OPT;              // taps per product
+  constexpr int NG = (27 + TPM - 1) / TPM;  // products per chunk
+  constexpr int NE = (HV * OPT + 255) / 256, AHEAD = 7;
+  typedef typename std::conditional<WIDE, unsigned long long, unsigned>::type off_t;
+  constexpr off_t kNowhere = (off_t)~0ull;
+  __shared__ __attribute__((aligned(16))) uint4v lds[NE * 256];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, oct = lane >> 4;
-  const int nbx = (a.dx + 7) / 8, nby = (a.dy + 7) / 8;
-  const int bx = blockIdx.x % nbx, by = (blockIdx.x / nbx) % nby, bz = blockIdx.x / (nbx * nby);
-  const int x0 = bx * 8, y0 = by * 8, z0 = bz * MT;
-  // this lane's A rows: voxel of row r in each of the wave's MT M-tiles
-  int abase[MT];
+  int x0, y0, z0;
+  if (!brick_origin<SY, SZ>(a, &x0, &y0, &z0)) return;
+  const uint4v zero4 = {0u, 0u, 0u, 0u};
+  auto slot = [](int voxel, int x, int h) { return OPT == 1 ? voxel : 2 * voxel + (h ^ ((x >> 3) & 1)); };
+  // the octets this thread stages: offset from the halo's first voxel (nowhere: 0)
+  const char *base = reinterpret_cast<const char *>(a.x) +
+                     ((((long long)z0 - 1) * a.dy + y0 - 1) * a.dx + x0 - 1) * a.ldx * 2;
+  off_t off[NE];
+  int put[NE];
+#pragma unroll
+  for (int q = 0; q < NE; ++q) {
+    const int e = q * 256 + (int)threadIdx.x, hv = e / OPT, h = e % OPT;
+    const int x = hv % kHaloX, row = hv / kHaloX, y = row % HY, z = row / HY;
+    const int gx = x0 + x - 1, gy = y0 + y - 1, gz = z0 + z - 1;
+    const bool in = e < HV * OPT && gx >= 0 && gx < a.dx && gy >= 0 && gy < a.dy && gz >= 0 && gz < a.dz;
+    off[q] = in ? (((off_t)z * (off_t)a.dy + (off_t)y) * (off_t)a.dx + (off_t)x) * (off_t)(2 * a.ldx) + (off_t)(16 * h)
+                : kNowhere;
+    put[q] = slot(hv, x, h);
+  }
+  // this lane's octet of each product, for the wave's first row
+  unsigned at[NG];
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    const int tap = g * TPM + oct / OPT < 27 ? g * TPM + oct / OPT : 0;  // (the 28th has zero weights)
+    const int x = r + tap % 3;
+    at[g] = (unsigned)slot(((wave + tap / 9) * HY + tap / 3 % 3) * kHaloX + x, x, oct % OPT);
+  }
+  const bool live27 = oct / OPT + (NG - 1) * TPM < 27;
+  const int nchunk = a.cin / CH, nper = a.cin == CH ? a.cout / 16 / (int)gridDim.y : 1;
+#pragma unroll 1
+  for (int nn = 0; nn < nper; ++nn) {
+    const int n = (int)blockIdx.y * nper + nn;
+    f32x4 acc[SY];
+#pragma unroll
+    for (int t = 0; t < SY; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int c = 0; c < nchunk; ++c) {
+      if (nn == 0) {
+        uint4v v[NE];
+        const char *from = base + 2 * CH * c;
+        if constexpr (WIDE) {
+#pragma unroll
+          for (int q = 0; q < NE; ++q)
+            v[q] = off[q] == kNowhere ? zero4 : *reinterpret_cast<const uint4v *>(from + off[q]);
+        } else {
+          const __amdgpu_buffer_rsrc_t rs =
+              __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(from), 0, 0x7fffffff, 0x00027000);
+#pragma unroll
+          for (int q = 0; q < NE; ++q) v[q] = __builtin_amdgcn_raw_buffer_load_b128(rs, off[q], 0, 0);
+        }
+        if (c > 0) __syncthreads();  // the previous chunk's readers are done
+#pragma unroll
+        for (int q = 0; q < NE; ++q) lds[put[q]] = v[q];
+      }
+      const bf16_t *wl = a.w + ((long long)n * nchunk + c) * (NG * 512) + lane * 8;
+      bf16x8 W[NG];
+#pragma unroll
+      for (int g = 0; g < NG; ++g) W[g] = *reinterpret_cast<const bf16x8 *>(wl + g * 512);
+      if (nn == 0) __syncthreads();
+      uint4v f[AHEAD];
+#pragma unroll
+      for (int q = 0; q < AHEAD; ++q) f[q] = lds[at[q % NG] + (unsigned)(q / NG * kHaloX * OPT)];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < SY; ++t)
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+          const int q = t * NG + g, next = q + AHEAD;
+          uint4v o = f[q % AHEAD];
+          if (g == NG - 1) o = live27 ? o : zero4;
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W[g], __builtin_bit_cast(bf16x8, o), acc[t], 0, 0, 0);
+          if (next < SY * NG) f[q % AHEAD] = lds[at[next % NG] + (unsigned)(next / NG * kHaloX * OPT)];
+          __builtin_amdgcn_sched_barrier(0);  // or every read would move down to its use
+        }
+    }
+    // lane holds channels 16 n + 4 oct + 0..3 of voxel x0 + r
+    const int col = 16 * n + 4 * oct, gx = x0 + r, gz = z0 + wave;
+    float b[4] = {0.f, 0.f, 0.f, 0.f};
+    if (a.bias) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) b[i] = a.bias[col + i];
+    }
+    if (gx < a.dx && gz < a.dz) {
+#pragma unroll
+      for (int t = 0; t < SY; ++t)
+        if (y0 + t < a.dy)
+          *reinterpret_cast<uint2 *>(a.y + (((long long)gz * a.dy + y0 + t) * a.dx + gx) * a.ldy + col) =
+              pack_out(acc[t], b, a.relu);
+    }
+  }
+}
+
+// The waves split into WN over the output channels and 4 / WN over the tiles,
+// MT tiles each; grid.y takes further channels.  Weights are read nine products
+// ahead; LDS holds the whole brick, cin channels a voxel.
+template <int SY, int SZ, int WN>
+__global__ __launch_bounds__(256, 2) void k_conv_whole(ConvFwdArgs a)
+{
+  constexpr int HY = SY + 2, HZ = SZ + 2, HV = kHaloX * HY * HZ, WM = 4 / WN, MT = SY * SZ / WM;
+  static_assert(SY * SZ % WM == 0, "");
+  constexpr int PF = 9;  // divides the 27 cin / 32 products
+  extern __shared__ __attribute__((aligned(16))) uint4 whole_lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, oct = lane >> 4;
+  int x0, y0, z0;
+  if (!brick_origin<SY, SZ>(a, &x0, &y0, &z0)) return;
+  const int m = a.cin / 32, so = a.cin / 8;  // products per tap, octets per voxel
+  // octets move within groups of `grp`, the power of two in so up to 16
+  const int grp = (so & -so) < 16 ? (so & -so) : 16, sh = grp == 4 ? 2 : grp == 8 ? 1 : 0;
+  auto swizzle = [&](int s, int x) { return (s & ~(grp - 1)) | ((s ^ (x >> sh)) & (grp - 1)); };
+  const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
+  const int n = (int)blockIdx.y * WN + wave % WN, mw = wave / WN;
+  const bf16_t *wl = a.w + (long long)n * (27 * m) * 512 + lane * 8;
+  bf16x8 W[PF];
+#pragma unroll
+  for (int u = 0; u < PF; ++u) W[u] = *reinterpret_cast<const bf16x8 *>(wl + u * 512);
+  for (int e0 = 0; e0 < HV * so; e0 += 256 * 4) {
+    uint4 v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int e = e0 + q * 256 + (int)threadIdx.x, hv = (int)((unsigned)e / (unsigned)so), s = e - hv * so;
+      const int x = hv % kHaloX, row = hv / kHaloX, y = row % HY, z = row / HY;
+      const int gx = x0 + x - 1, gy = y0 + y - 1, gz = z0 + z - 1;
+      v[q] = zero4;
+      if (hv < HV && gx >= 0 && gx < a.dx && gy >= 0 && gy < a.dy && gz >= 0 && gz < a.dz)
+        v[q] = *reinterpret_cast<const uint4 *>(a.x + (((long long)gz * a.dy + gy) * a.dx + gx) * a.ldx + 8 * s);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int e = e0 + q * 256 + (int)threadIdx.x, hv = (int)((unsigned)e / (unsigned)so), s = e - hv * so;
+      if (hv < HV) whole_lds[hv * so + swizzle(s, hv % kHaloX)] = v[q];
+    }
+  }
+  __syncthreads();
+  f32x4 acc[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int tile[MT];  // the tiles' first halo row (uniform)
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
-    const int v = 16 * (wave * MT + t) + r;
-    const int lx = v & 7, ly = (v >> 3) & 7, lz = v >> 6;
-    abase[t] = (lz * HY + ly) * HX + lx;  // halo origin is (-1,-1,-1)
+    const int q = mw * MT + t;
+    tile[t] = (q / SY * HY + q % SY) * kHaloX * so;
   }
-  f32x4 acc[MT][NT];
+  const int steps = 27 * m;
+  // the next product's 32 channels, x shift, and rows (z, y) passed
+  int c = 0, ox = 0, rows = 0, oy = 0;
+  uint4 f[2][MT];
+  auto read = [&](uint4 *v) {
+    const int x = r + ox;
+    const int at = (rows * kHaloX + x) * so + swizzle(4 * c + oct, x);
 #pragma unroll
-  for (int t = 0; t < MT; ++t)
-#pragma unroll
-    for (int n = 0; n < NT; ++n) acc[t][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
-  // lane octet -> (tap within the MFMA, channel octet within the chunk)
-  const int otap = oct / OPT, och = 8 * (oct % OPT);
-  for (int c0 = 0; c0 < a.cin; c0 += CH) {
-    // with one output tile the chunk's weight fragments fit in registers:
-    // load them before the staging so their latency overlaps it
-    bf16x8 bpre[NT == 1 ? NG : 1];
-    if constexpr (NT == 1) {
-#pragma unroll
-      for (int g = 0; g < NG; ++g) {
-        const int tap = g * TPM + otap;
-        bpre[g] = as_bf16x8(tap < 27 ? *reinterpret_cast<const uint4 *>(a.w + (long long)r * a.kp +
-                                                                         (long long)tap * a.cin + c0 + och)
-                                     : zero4);
+    for (int t = 0; t < MT; ++t) v[t] = whole_lds[at + tile[t]];
+    if (++c == m) {
+      c = 0;
+      if (++ox == 3) {
+        ox = 0;
+        ++rows;
+        if (++oy == 3) {
+          oy = 0;
+          rows += HY - 3;
+        }
       }
     }
-    __syncthreads();  // the previous chunk's readers are done
-    for (int e = threadIdx.x; e < HV * OPT; e += 256) {
-      const int hv = e / OPT, h = e % OPT;
-      const int hx = hv % HX, hy = (hv / HX) % HY, hz = hv / (HX * HY);
-      const int gx = x0 + hx - 1, gy = y0 + hy - 1, gz = z0 + hz - 1;
-      uint4 val = zero4;
-      if (gx >= 0 && gx < a.dx && gy >= 0 && gy < a.dy && gz >= 0 && gz < a.dz)
-        val = *reinterpret_cast<const uint4 *>(a.x + (((long long)gz * a.dy + gy) * a.dx + gx) * a.ldx + c0 + 8 * h);
-      *reinterpret_cast<uint4 *>(lds + hv * CH + 8 * h) = val;
-    }
-    __syncthreads();
+  };
+  read(f[0]);
+  // by twos, so that the operands in flight keep their registers
+  for (int base = 0; base < steps; base += PF) {
 #pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      const int tap = g * TPM + otap;
-      const bool live = tap < 27;
-      const int tz = tap / 9, ty = (tap / 3) % 3, tx = tap % 3;
-      const int toff = (tz * HY + ty) * HX + tx;
-      bf16x8 av[MT];
+    for (int u = 0; u < PF; ++u) {
+      if (base + u + 1 < steps) read(f[(u + 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);  // or the reads would move down to their use
 #pragma unroll
       for (int t = 0; t < MT; ++t)
-        av[t] = as_bf16x8(live ? *reinterpret_cast<const uint4 *>(lds + (abase[t] + toff) * CH + och) : zero4);
-      const long long kw = (long long)tap * a.cin + c0 + och;  // weight column of this lane's octet
-#pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        bf16x8 bv;
-        if constexpr (NT == 1)
-          bv = bpre[g];
-        else
-          bv = as_bf16x8(live ? *reinterpret_cast<const uint4 *>(a.w + (long long)(16 * n + r) * a.kp + kw) : zero4);
-#pragma unroll
-        for (int t = 0; t < MT; ++t) acc[t][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[t], bv, acc[t][n], 0, 0, 0);
-      }
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W[u], as_bf16x8(f[u & 1][t]), acc[t], 0, 0, 0);
+      const int next = base + u + PF < steps ? base + u + PF : steps - 1;
+      W[u] = *reinterpret_cast<const bf16x8 *>(wl + (long long)next * 512);
     }
+    // PF is odd: the operand read last is where the next round looks for it
+#pragma unroll
+    for (int t = 0; t < MT; ++t) f[0][t] = f[PF & 1][t];
   }
-  // epilogue: lane holds D[4*oct + i][r] of each tile
+  const int col = 16 * n + 4 * oct, gx = x0 + r;
+  float b[4] = {0.f, 0.f, 0.f, 0.f};
+  if (a.bias) {
 #pragma unroll
-  for (int t = 0; t < MT; ++t)
+    for (int i = 0; i < 4; ++i) b[i] = a.bias[col + i];
+  }
 #pragma unroll
-    for (int n = 0; n < NT; ++n) {
-      const int col = 16 * n + r;
-      const float b = a.bias ? a.bias[col] : 0.f;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int v = 16 * (wave * MT + t) + 4 * oct + i;
-        const int gx = x0 + (v & 7), gy = y0 + ((v >> 3) & 7), gz = z0 + (v >> 6);
-        if (gx >= a.dx || gy >= a.dy || gz >= a.dz) continue;
-        float val = acc[t][n][i] + b;
-        if (a.relu) val = val > 0.f ? val : 0.f;
-        const long long m = ((long long)gz * a.dy + gy) * a.dx + gx;
-        as_global(a.y)[m * a.ldy + a.ycoff + col] = f2bf(val);
-      }
-    }
+  for (int t = 0; t < MT; ++t) {
+    const int q = mw * MT + t, gy = y0 + q % SY, gz = z0 + q / SY;
+    if (gx < a.dx && gy < a.dy && gz < a.dz)
+      *reinterpret_cast<uint2 *>(a.y + (((long long)gz * a.dy + gy) * a.dx + gx) * a.ldy + col) = pack_out(acc[t], b, a.relu);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -743,34 +902,62 @@ __global__ __launch_bounds__(256) void k_adam(float *p, const float *g, float *m
   p[q] -= lr * (mq / c1) / (sqrtf(vq / c2) + eps);
 }
 
-// packed BF16 weights from the FP32 master W[cout][27*cin]:
-//   forward  wt[n][kp],  wt[n][tap*cin + c] = W[n][tap*cin + c]
-//   dgrad    wd[c][kpd], wd[c][tap'*cout + n] = W[n][(26 - tap')*cin + c]
-__global__ __launch_bounds__(256) void k_pack_w(const float *W, int cin, int cout, int kp, int kpd, bf16_t *wt,
+// BF16 weights from the FP32 master W[cout][27*cin], as the convolution's lanes
+// read them: [16 outputs][chunk][product][lane][8] (chunks), [16 outputs]
+// [product][lane][8] (whole) or [cout][kp], kp = 27 cin rounded up to 32 (rows).
+// The data gradient is the same convolution with the taps reversed and the
+// channels exchanged, W'[c][26 - tap][n]; its weights follow in wd (null: none).
+__global__ __launch_bounds__(256) void k_pack_w(const float *W, int cin, int cout, int kind, int kind_d, bf16_t *wt,
                                                 bf16_t *wd)
 {
   const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
-  const long long nt = (long long)cout * kp, nd = (long long)cin * kpd;
-  if (q < nt) {
-    const int n = (int)(q / kp), k = (int)(q - (long long)n * kp);
-    wt[q] = k < 27 * cin ? f2bf(W[(long long)n * 27 * cin + k]) : (bf16_t)0;
-  } else if (q < nt + nd) {
-    const long long r = q - nt;
-    const int c = (int)(r / kpd), k = (int)(r - (long long)c * kpd);
-    bf16_t val = 0;
-    if (k < 27 * cout) {
-      const int tp = k / cout, n = k - tp * cout;
-      val = f2bf(W[(long long)n * 27 * cin + (26 - tp) * cin + c]);
+  const long long nt = packed_weights((ConvKind)kind, cin, cout);
+  const long long nd = wd ? packed_weights((ConvKind)kind_d, cout, cin) : 0;
+  if (q >= nt + nd) return;
+  const bool grad = q >= nt;
+  const ConvKind k = (ConvKind)(grad ? kind_d : kind);
+  const long long p = grad ? q - nt : q;
+  const int ci = grad ? cout : cin;  // channels summed over
+  int n, tap, c;
+  if (k == ConvKind::rows) {
+    const int kp = (27 * ci + 31) / 32 * 32;
+    n = (int)(p / kp);
+    const int kk = (int)(p - (long long)n * kp);
+    tap = kk / ci;
+    c = kk - tap * ci;
+  } else {
+    const int j = (int)(p & 7), lane = (int)(p >> 3) & 63, oct = lane >> 4;
+    const int f = (int)(p >> 9);
+    if (k == ConvKind::whole) {
+      const int m = ci / 32, step = f % (27 * m);
+      n = f / (27 * m);
+      tap = step / m;
+      c = 32 * (step - tap * m) + 8 * oct + j;
+    } else {
+      const int opt = k == ConvKind::chunks8 ? 1 : 2, tpm = 4 / opt, ng = (27 + tpm - 1) / tpm;
+      const int g = f % ng, nchunk = ci / (8 * opt), chunk = f / ng % nchunk;
+      n = f / ng / nchunk;
+      tap = g * tpm + oct / opt;
+      c = 8 * opt * chunk + 8 * (oct % opt) + j;
     }
-    wd[r] = val;
+    n = 16 * n + (lane & 15);
   }
+  bf16_t val = 0;
+  if (tap < 27)
+    val = f2bf(grad ? W[(long long)c * 27 * cin + (26 - tap) * cin + n] : W[(long long)n * 27 * cin + tap * cin + c]);
+  (grad ? wd : wt)[p] = val;
 }
 
-// fp32 host volume -> BF16 device volume
+// fp32 host volume -> BF16 device volume, eight values per thread (n is a
+// multiple of eight): 20 -> 8 us for 8.4 M values
 __global__ __launch_bounds__(256) void k_f2bf(const float *src, bf16_t *dst, long long n)
 {
-  const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (q < n) dst[q] = f2bf(src[q]);
+  const long long q = 8 * ((long long)blockIdx.x * 256 + threadIdx.x);
+  if (q >= n) return;
+  const float4 a = *reinterpret_cast<const float4 *>(src + q), b = *reinterpret_cast<const float4 *>(src + q + 4);
+  *reinterpret_cast<uint4 *>(dst + q) =
+      make_uint4((unsigned)f2bf(a.x) | ((unsigned)f2bf(a.y) << 16), (unsigned)f2bf(a.z) | ((unsigned)f2bf(a.w) << 16),
+                 (unsigned)f2bf(b.x) | ((unsigned)f2bf(b.y) << 16), (unsigned)f2bf(b.z) | ((unsigned)f2bf(b.w) << 16));
 }
 
 // Per-problem scales: s = rms(R) over updated cells, u = max inflow speed of
@@ -882,6 +1069,7 @@ namespace {
 struct Conv {
   int cin, cout, kp, kpd;
   long long woff, boff;  // offsets in the parameter vector
+  ConvKind kind, kind_d;  // forward, data gradient
   bf16_t *wt = nullptr, *wd = nullptr;
 };
 
@@ -955,66 +1143,66 @@ inline bool vec8(int ch, int ld_a, int ld_b, int off, long long V)
   return ch % 8 == 0 && ld_a % 8 == 0 && ld_b % 8 == 0 && off % 8 == 0 && V * (long long)(ld_a > ld_b ? ld_a : ld_b) < (1LL << 31);
 }
 
-hipError_t launch_conv_fwd(hipStream_t s, const ConvFwdArgs &a, int cout)
+template <int SY, int SZ, int WN>
+hipError_t launch_whole(hipStream_t s, const ConvFwdArgs &a)
 {
+  const size_t bytes = 2 * (size_t)kHaloX * (SY + 2) * (SZ + 2) * a.cin;
+  const long long bricks =
+      (long long)((a.dx + kBrickX - 1) / kBrickX) * ((a.dy + SY - 1) / SY) * ((a.dz + SZ - 1) / SZ);
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv_whole<SY, SZ, WN>),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((k_conv_whole<SY, SZ, WN>), dim3((unsigned)((bricks + kXcdsU - 1) / kXcdsU * kXcdsU), (unsigned)(a.cout / 16 / WN)),
+                     dim3(256), bytes, s, a);
+  return hipGetLastError();
+}
+
+template <int WN>
+hipError_t launch_whole_size(hipStream_t s, const ConvFwdArgs &a)
+{
+  // the largest brick that fits the 160 KB of LDS and leaves a work-group per CU
+  auto fits = [&](int sy, int sz) {
+    const long long bricks =
+        (long long)((a.dx + kBrickX - 1) / kBrickX) * ((a.dy + sy - 1) / sy) * ((a.dz + sz - 1) / sz);
+    return 2LL * kHaloX * (sy + 2) * (sz + 2) * a.cin <= 160 * 1024 && bricks * (a.cout / 16 / WN) >= 256;
+  };
+  if constexpr (WN < 4)  // 16 tiles a wave would spill
+    if (fits(4, 4)) return launch_whole<4, 4, WN>(s, a);
+  if (fits(4, 2)) return launch_whole<4, 2, WN>(s, a);
+  if (fits(2, 2)) return launch_whole<2, 2, WN>(s, a);
+  return launch_whole<WN == 1 ? 2 : 1, 2, WN>(s, a);
+}
+
+hipError_t launch_conv_fwd(hipStream_t s, const ConvFwdArgs &a)
+{
+  if (a.cout % 16 || a.ldx % 8 || a.ldy % 4) return hipErrorInvalidValue;
+  const int NT = a.cout / 16;
   const long long V = (long long)a.dx * a.dy * a.dz;
-  const int NT = cout / 16;
-  // LDS-staged kernel: cin 8 or a multiple of 16, 16-byte aligned channel
-  // rows, and enough 8x8x4 bricks to fill the GPU (the large, shallow levels;
-  // the deep levels have too few voxels for bricks and use the kernel above)
-  const long long bxy = (long long)((a.dx + 7) / 8) * ((a.dy + 7) / 8);
-  if ((a.cin == 8 || a.cin % 16 == 0) && a.ldx % 8 == 0 && cout % 16 == 0 && bxy * ((a.dz + 3) / 4) >= 1024) {
-    auto lds = [&](auto kern, int MT) {
-      const long long nb = bxy * ((a.dz + MT - 1) / MT);
-      hipLaunchKernelGGL(kern, dim3((unsigned)nb), dim3(256), 0, s, a);
-      return hipGetLastError();
-    };
-    if (a.cin == 8) {
-      switch (NT) {
-      case 1: return lds(k_conv_fwd_lds<1, 4, 8>, 4);
-      case 2: return lds(k_conv_fwd_lds<2, 4, 8>, 4);
-      default: break;
-      }
-    } else {
-      switch (NT) {
-      case 1: return lds(k_conv_fwd_lds<1, 4, 16>, 4);
-      case 2: return lds(k_conv_fwd_lds<2, 4, 16>, 4);
-      case 3: return lds(k_conv_fwd_lds<3, 4, 16>, 4);
-      case 4: return lds(k_conv_fwd_lds<4, 4, 16>, 4);
-      case 6: return lds(k_conv_fwd_lds<6, 2, 16>, 2);
-      case 8: return lds(k_conv_fwd_lds<8, 2, 16>, 2);
-      case 12: return lds(k_conv_fwd_lds<12, 2, 16>, 2);
-      default: break;
-      }
-    }
+  auto chunks = [&](auto kern) {
+    const long long bricks = (long long)((a.dx + kBrickX - 1) / kBrickX) * ((a.dy + 7) / 8) * ((a.dz + 3) / 4);
+    // one chunk: staged once for all outputs where there are bricks enough
+    const bool split = a.cin > 16 || bricks < 1024;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((bricks + kXcdsU - 1) / kXcdsU * kXcdsU), (unsigned)(split ? NT : 1)),
+                       dim3(256), 0, s, a);
+    return hipGetLastError();
+  };
+  // a lane's offset within a brick's six planes has 31 bits in a buffer load
+  const bool wide = 12LL * a.dy * a.dx * a.ldx >= 0x7fffffffLL;
+  switch (conv_kind(a.cin, a.dx, a.dy, a.dz)) {
+  case ConvKind::chunks8: return wide ? chunks(k_conv_chunks<8, true>) : chunks(k_conv_chunks<8, false>);
+  case ConvKind::chunks16: return wide ? chunks(k_conv_chunks<16, true>) : chunks(k_conv_chunks<16, false>);
+  case ConvKind::whole:
+    return NT % 4 == 0 ? launch_whole_size<4>(s, a) : NT % 2 == 0 ? launch_whole_size<2>(s, a) : launch_whole_size<1>(s, a);
+  default: break;
   }
   auto go = [&](auto kern, int MT, int rows = 1) {
     const long long waves = (V + 16LL * MT - 1) / (16LL * MT);
     hipLaunchKernelGGL(kern, dim3((unsigned)((waves + 3) / 4), (unsigned)rows), dim3(256), 0, s, a);
-  };
-  // Small volumes (the deep levels, fewer than 2048 waves with the tiles
-  // below): one output tile per wave and fewer voxel tiles, so that up to
-  // 4096 waves cover the GPU.
-  const long long want = 4096;
-  const int mt_default = NT == 1 ? 8 : NT == 2 ? 4 : NT <= 4 ? 2 : 1;
-  if ((V + 16LL * mt_default - 1) / (16LL * mt_default) < 2048) {
-    const long long w4 = (V + 63) / 64 * NT, w2 = (V + 31) / 32 * NT;
-    if (w4 >= want) go(k_conv_fwd<1, 4>, 4, NT);
-    else if (w2 >= want) go(k_conv_fwd<1, 2>, 2, NT);
-    else go(k_conv_fwd<1, 1>, 1, NT);
     return hipGetLastError();
-  }
-  switch (NT) {
-  case 1: go(k_conv_fwd<1, 8>, 8); break;
-  case 2: go(k_conv_fwd<2, 4>, 4); break;
-  case 3: go(k_conv_fwd<3, 2>, 2); break;
-  case 4: go(k_conv_fwd<4, 2>, 2); break;
-  case 6: go(k_conv_fwd<6, 1>, 1); break;
-  case 8: go(k_conv_fwd<8, 1>, 1); break;
-  case 12: go(k_conv_fwd<12, 1>, 1); break;
-  default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
+  };
+  // up to 4096 waves cover the GPU
+  const long long want = 4096, w4 = (V + 63) / 64 * NT, w2 = (V + 31) / 32 * NT;
+  return w4 >= want ? go(k_conv_fwd<1, 4>, 4, NT) : w2 >= want ? go(k_conv_fwd<1, 2>, 2, NT) : go(k_conv_fwd<1, 1>, 1, NT);
 }
 
 // Work-groups of the weight gradient: two per CU over all channel pairs (its
@@ -1043,12 +1231,11 @@ inline unsigned reduce_blocks(long long V, int ch)
   return (unsigned)(b < 1024 ? b : 1024);
 }
 
-// One conv layer forward: x (ldx, cin) -> y (ldy at ycoff), bias + ReLU
-hipError_t conv_forward(qesmc_unet *u, const Conv &cv, const Level &lv, const bf16_t *x, int ldx, bf16_t *y,
-                        int ldy, int ycoff)
+// One conv layer forward: x (ldx, cin) -> y (ldy), bias + ReLU
+hipError_t conv_forward(qesmc_unet *u, const Conv &cv, const Level &lv, const bf16_t *x, int ldx, bf16_t *y, int ldy)
 {
-  ConvFwdArgs a{x, ldx, cv.cin, 27 * cv.cin, cv.wt, cv.kp, u->p + cv.boff, y, ldy, ycoff, lv.dx, lv.dy, lv.dz, 1};
-  return launch_conv_fwd(u->stream, a, cv.cout);
+  ConvFwdArgs a{x, ldx, cv.cin, 27 * cv.cin, cv.cout, cv.wt, cv.kp, u->p + cv.boff, y, ldy, lv.dx, lv.dy, lv.dz, 1};
+  return launch_conv_fwd(u->stream, a);
 }
 
 // Backward through one conv layer whose ReLU output y (ldy) received the
@@ -1067,8 +1254,8 @@ hipError_t conv_backward(qesmc_unet *u, const Conv &cv, const Level &lv, const b
   ConvWgradArgs wa{x, ldx, cv.cin, 27 * cv.cin, g, ldg, u->gp + cv.woff, lv.dx, lv.dy, lv.dz, 0, 0};
   if ((e = launch_wgrad(s, wa, cv.cout)) != hipSuccess) return e;
   if (gx) {
-    ConvFwdArgs a{g, ldg, cv.cout, 27 * cv.cout, cv.wd, cv.kpd, nullptr, gx, ldgx, 0, lv.dx, lv.dy, lv.dz, 0};
-    if ((e = launch_conv_fwd(s, a, cv.cin)) != hipSuccess) return e;
+    ConvFwdArgs a{g, ldg, cv.cout, 27 * cv.cout, cv.cin, cv.wd, cv.kpd, nullptr, gx, ldgx, lv.dx, lv.dy, lv.dz, 0};
+    if ((e = launch_conv_fwd(s, a)) != hipSuccess) return e;
   }
   return hipSuccess;
 }
@@ -1076,9 +1263,9 @@ hipError_t conv_backward(qesmc_unet *u, const Conv &cv, const Level &lv, const b
 hipError_t pack_weights(qesmc_unet *u)
 {
   auto pk = [&](Conv &c) {
-    const long long n = (long long)c.cout * c.kp + (long long)c.cin * c.kpd;
-    hipLaunchKernelGGL(k_pack_w, g1(n), dim3(256), 0, u->stream, u->p + c.woff, c.cin, c.cout, c.kp, c.kpd, c.wt,
-                       c.wd);
+    const long long n = packed_weights(c.kind, c.cin, c.cout) + (c.wd ? packed_weights(c.kind_d, c.cout, c.cin) : 0);
+    hipLaunchKernelGGL(k_pack_w, g1(n), dim3(256), 0, u->stream, u->p + c.woff, c.cin, c.cout, (int)c.kind,
+                       (int)c.kind_d, c.wt, c.wd);
   };
   for (int l = 0; l < u->L; ++l) {
     pk(u->enc1[l]);
@@ -1100,8 +1287,8 @@ hipError_t forward(qesmc_unet *u, const bf16_t *feat)
     Level &lv = u->lv[l];
     const bf16_t *in = l == 0 ? feat : lv.P;
     const int ldin = l == 0 ? QESMC_UNET_IN_CHANNELS : u->lv[l - 1].c;
-    if ((e = conv_forward(u, u->enc1[l], lv, in, ldin, lv.A, lv.c, 0)) != hipSuccess) return e;
-    if ((e = conv_forward(u, u->enc2[l], lv, lv.A, lv.c, lv.CAT, lv.ldcat, 0)) != hipSuccess) return e;
+    if ((e = conv_forward(u, u->enc1[l], lv, in, ldin, lv.A, lv.c)) != hipSuccess) return e;
+    if ((e = conv_forward(u, u->enc2[l], lv, lv.A, lv.c, lv.CAT, lv.ldcat)) != hipSuccess) return e;
     if (l + 1 < L) {
       Level &nx = u->lv[l + 1];
       if (vec8(lv.c, lv.ldcat, lv.c, 0, nx.V))
@@ -1123,8 +1310,8 @@ hipError_t forward(qesmc_unet *u, const bf16_t *feat)
     else
       hipLaunchKernelGGL(k_up_fwd, g1(lv.V * dn.c), dim3(256), 0, s, src, ldsrc, lv.CAT, lv.ldcat, lv.c, dn.c, lv.dx,
                          lv.dy, lv.dz);
-    if ((e = conv_forward(u, u->dec1[l], lv, lv.CAT, lv.ldcat, lv.E, lv.c, 0)) != hipSuccess) return e;
-    if ((e = conv_forward(u, u->dec2[l], lv, lv.E, lv.c, lv.D, lv.c, 0)) != hipSuccess) return e;
+    if ((e = conv_forward(u, u->dec1[l], lv, lv.CAT, lv.ldcat, lv.E, lv.c)) != hipSuccess) return e;
+    if ((e = conv_forward(u, u->dec2[l], lv, lv.E, lv.c, lv.D, lv.c)) != hipSuccess) return e;
   }
   Level &top = u->lv[0];
   if (vec8(top.c, top.c, top.c, 0, top.V))
@@ -1311,8 +1498,14 @@ int qesmc_unet_create(qesmc_unet **out, int device, const qesmc_unet_config *cfg
   bool bad = fail(dmalloc(&u->p, off)) || fail(dmalloc(&u->gp, off)) || fail(dmalloc(&u->m1, off)) ||
              fail(dmalloc(&u->m2, off));
   for (auto *v : {&u->enc1, &u->enc2, &u->dec1, &u->dec2})
-    for (auto &c : *v)
-      bad = bad || fail(dmalloc(&c.wt, (long long)c.cout * c.kp)) || fail(dmalloc(&c.wd, (long long)c.cin * c.kpd));
+    for (size_t l = 0; l < v->size(); ++l) {
+      Conv &c = (*v)[l];
+      c.kind = conv_kind(c.cin, u->dx >> l, u->dy >> l, u->dz >> l);
+      c.kind_d = conv_kind(c.cout, u->dx >> l, u->dy >> l, u->dz >> l);
+      bad = bad || fail(dmalloc(&c.wt, packed_weights(c.kind, c.cin, c.cout)));
+      if (c.cin % 16 == 0)  // the network's input needs no gradient
+        bad = bad || fail(dmalloc(&c.wd, packed_weights(c.kind_d, c.cout, c.cin)));
+    }
   double flops = 0.0;
   for (int l = 0; l < u->L && !bad; ++l) {
     Level &lv = u->lv[l];
@@ -1430,7 +1623,7 @@ int qesmc_unet_forward(qesmc_unet *u, const float *input, float *output)
   const long long n = V0 * QESMC_UNET_IN_CHANNELS;
   const HostPiece in = host_piece(input, u->hostbuf_dev, sizeof(float) * (size_t)n);
   UCHK(host_copy(u->device, u->stream, &in, 1, true));
-  hipLaunchKernelGGL(k_f2bf, g1(n), dim3(256), 0, u->stream, u->hostbuf_dev, u->feat, n);
+  hipLaunchKernelGGL(k_f2bf, g1(n / 8), dim3(256), 0, u->stream, u->hostbuf_dev, u->feat, n);
   UCHK(hipGetLastError());
   UCHK(forward(u, u->feat));
   const HostPiece out = host_piece(output, u->out, sizeof(float) * (size_t)V0);
