@@ -778,19 +778,33 @@ def reference_schedule(ctx, params, steps, warmup):
     return time.perf_counter() - t0, results
 
 
-def roofline_of(results, lups_per_iteration, workload_key):
+def marches(path, tiles, compressed):
+    """Whether a run takes two iterations per launch: any wall-mask geometry
+    unless a path or a tiling of the colour passes is asked for."""
+    if path == Q.PATH_FUSED:
+        return True
+    return path == Q.PATH_AUTO and bool(compressed) and not any(tiles.values())
+
+
+def roofline_of(results, lups_per_iteration, workload_key, iterations_per_launch=None):
     """Roofline object of the dominant SOR kernel from the run's own HIP-event
-    timings: achieved = algorithmic bytes per launch / mean launch time."""
+    timings: achieved = algorithmic bytes per launch / mean launch time.  With
+    iterations_per_launch = 2 (the march) a launch's 13 bytes per cell serve
+    two updates of it, 6.5 bytes each; the march is bound by its caches and
+    vector ALUs then, and the HBM fraction says how far it is from needing HBM."""
     last = results[-1]
     its = last["iterations"]
-    fused = last["path"] == Q.PATH_FUSED
-    launches = its if fused else 2 * its
+    fused = last["path"] == Q.PATH_FUSED or iterations_per_launch is not None
+    per = iterations_per_launch or 1
+    launches = (its + per - 1) // per if fused else 2 * its
     ms_sor = float(np.mean([r["ms_sor"] for r in results]))
     launch_ms = ms_sor / launches
-    bpl = bytes_per_lup(last)
-    per_launch_updates = lups_per_iteration / (1 if fused else 2)
+    bpl = 13.0 / per if fused else bytes_per_lup(last)
+    per_launch_updates = lups_per_iteration * its / launches if fused else lups_per_iteration / 2
     achieved = bpl * per_launch_updates / (launch_ms * 1e-3) / 1e9
-    if last["path"] == Q.PATH_PLAIN:
+    if iterations_per_launch is not None:
+        kernel = "k_sor_march, %d iterations per launch" % per
+    elif last["path"] == Q.PATH_PLAIN:
         kernel = "k_rb_plain"
     elif fused:
         kernel = "k_sor_march<%d>" % (8 if last["tile_k"] >= 8 else 4)
@@ -798,7 +812,7 @@ def roofline_of(results, lups_per_iteration, workload_key):
         kernel = "k_sor_split<%s, %d>" % ("true" if last["compressed"] else "false", last["tile_v"])
     traffic, source = load_traffic(kernel, workload_key)
     ref36 = 36.0 * per_launch_updates / (launch_ms * 1e-3) / 1e9
-    return {"bound": "hbm", "kernel": kernel, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
+    return {"bound": "hbm" if iterations_per_launch is None else "caches and vector ALUs", "kernel": kernel, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
             "traffic_source": source, "bytes_per_lup": bpl, "avg_launch_us": round(launch_ms * 1e3, 2),
             "updates_per_launch": int(per_launch_updates),
@@ -835,7 +849,8 @@ def city400_leg(path, tiles, steps=5, warmup=1):
         div_ref = ctx.divergence_linf(False)
         grad_ms = min(ctx.velocity_gradient(uniform_z=False, copy=False)[1] for _ in range(3))
     its = results[-1]["iterations"]
-    roof, ms_sor = roofline_of(results, city.interior_lups(), "city400x400x120")
+    roof, ms_sor = roofline_of(results, city.interior_lups(), "city400x400x120",
+                               2 if marches(path, tiles, results[-1]["compressed"]) else None)
     return {"workload": desc, "steps": steps, "t_ref_ms": round(wall / steps * 1e3, 3), "sor_ms": round(ms_sor, 3),
             "glups": round(city.interior_lups() * its * steps / wall / 1e9, 3), "div_linf_ref_operator": div_ref,
             "velocity_gradient": {"ms": round(grad_ms, 4), "bytes_per_cell": 52,
@@ -916,7 +931,8 @@ def main():
     lups_it = shape.interior_lups()
     its = results[-1]["iterations"]
     last = results[-1]
-    roof, ms_sor = roofline_of(results, lups_it, "city1000x1000x150")
+    roof, ms_sor = roofline_of(results, lups_it, "city1000x1000x150",
+                               2 if marches(path, tiles, last["compressed"]) else None)
     glups = lups_it * its * a.steps / wall / 1e9
     out = {
         "metric": METRIC,

@@ -11,7 +11,7 @@
 // |dlambda|), relaxes the tile exactly as the single-problem kernel does and
 // publishes its max into the instance's striped slots.  Converged instances
 // cost one gate read per tile, so a batch behaves as if each problem were
-// solved alone.  Iterations can be replayed as a captured HIP graph: the
+// solved alone.  Colour passes can be replayed as a captured HIP graph: the
 // iteration number then comes from a device counter advanced by the graph.
 #include <algorithm>
 #include <cmath>
@@ -184,12 +184,7 @@ __global__ __launch_bounds__(256) void k_sor_batch(const BatchItem *__restrict__
   }
 }
 
-// the next replay's iterations and launches
-__global__ void k_advance(int *t_base, int by, int launches)
-{
-  t_base[0] += by;
-  t_base[1] += launches;
-}
+__global__ void k_advance(int *t_base, int by) { t_base[0] += by; }
 
 // number of instances whose row t is still above tol (t = t_base[0] + t_off)
 __global__ __launch_bounds__(64) void k_count_active(const BatchItem *items, int n, const int *t_base, int t_off,
@@ -375,14 +370,13 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
   };
   hipError_t e;
   if ((e = hipMalloc((void **)&d_items, sizeof(BatchItem) * n)) != hipSuccess) return fail(e);
-  if ((e = hipMalloc((void **)&d_t, 2 * sizeof(int))) != hipSuccess) return fail(e);
+  if ((e = hipMalloc((void **)&d_t, sizeof(int))) != hipSuccess) return fail(e);
   if ((e = hipMalloc((void **)&d_active, sizeof(int))) != hipSuccess) return fail(e);
   if ((e = hipHostMalloc((void **)&h_active, sizeof(int), hipHostMallocDefault)) != hipSuccess) return fail(e);
   if ((e = hipEventCreate(&e0)) != hipSuccess || (e = hipEventCreate(&e1)) != hipSuccess) return fail(e);
   if ((e = hipMemcpyAsync(d_items, items.data(), sizeof(BatchItem) * n, hipMemcpyHostToDevice, bs)) != hipSuccess)
     return fail(e);
   if ((e = qesmc_launch_set_u32(lead, (unsigned *)d_t, 0u)) != hipSuccess) return fail(e);
-  if ((e = qesmc_launch_set_u32(lead, (unsigned *)d_t + 1, 0u)) != hipSuccess) return fail(e);
   // The march may take the members in groups, each for check_every iterations
   // in turn, so that a group's arrays (13 bytes a cell) stay in the 256 MB
   // Infinity Cache: what leaves it costs a launch up to 0.6 of its time more
@@ -498,7 +492,7 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
 #undef QESMC_BATCH_LAUNCH
       }
     };
-    auto launch_march = [&](const Group &gr, int iters, const int *base, int t, int src, bool fix) -> hipError_t {
+    auto launch_march = [&](const Group &gr, int iters, int t, int src, bool fix) -> hipError_t {
       if (gr.slots[iters - 1] == 0) return hipSuccess;
       MarchRun run{};
       for (float &w : run.om) w = p.omega;
@@ -509,46 +503,42 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
       run.fix = fix ? 1 : 0;
       run.items = d_march + (size_t)(iters - 1) * n;
       run.which = reinterpret_cast<const int *>(d_march + 2 * (size_t)n) + gr.which[iters - 1];
-      run.base = base;
       return qesmc_launch_march_batch(bs, iters, gr.shape[iters - 1], gr.slots[iters - 1], run);
     };
     // iterations [t, t + count) by twos, reading buffer set src & 1 first
-    auto march_chunk = [&](const int *base, int t, int count, int src) -> hipError_t {
+    auto march_chunk = [&](int t, int count, int src) -> hipError_t {
       for (const Group &gr : groups)
         for (int j = 0; j < count; j += 2) {
-          const hipError_t le = launch_march(gr, j + 2 <= count ? 2 : 1, base, t + j, (src + j / 2) & 1, false);
+          const hipError_t le = launch_march(gr, j + 2 <= count ? 2 : 1, t + j, (src + j / 2) & 1, false);
           if (le != hipSuccess) return le;
         }
       return hipSuccess;
     };
-    const bool replay = use_graph && (!march || p.itermax >= C);
+    // The march is launched directly: a launch takes 20 us or more and two
+    // iterations, so the host is far ahead of the device without a replay.
+    const bool replay = use_graph && !march;
     int launches = 0;
     if (replay) {
       // one captured chunk of C iterations, advancing the device counter
       if ((e = hipStreamBeginCapture(bs, hipStreamCaptureModeThreadLocal)) != hipSuccess) return fail(e);
-      if (march)
-        e = march_chunk(d_t, 0, C, 0);
-      else
-        for (int j = 0; j < C; ++j) launch_iter(d_t, j);
-      hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, bs, d_t, C, (C + 1) / 2);
+      for (int j = 0; j < C; ++j) launch_iter(d_t, j);
+      hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, bs, d_t, C);
       if ((e = hipStreamEndCapture(bs, &graph)) != hipSuccess) return fail(e);
       if ((e = hipGraphInstantiate(&gexec, graph, nullptr, nullptr, 0)) != hipSuccess) return fail(e);
     }
     bool stop = false;
     while (launched < p.itermax && !stop) {
       const int chunk = std::min(C, p.itermax - launched);
-      // the march's launches hold two iterations, so a last chunk that itermax cuts short is not replayed
-      const bool whole = replay && (!march || chunk == C);
-      if (whole) {
+      if (replay) {
         if ((e = hipGraphLaunch(gexec, bs)) != hipSuccess) return fail(e);
       } else if (march) {
-        if ((e = march_chunk(nullptr, launched, chunk, launches)) != hipSuccess) return fail(e);
+        if ((e = march_chunk(launched, chunk, launches)) != hipSuccess) return fail(e);
+        launches += (chunk + 1) / 2;
       } else {
         for (int j = 0; j < chunk; ++j) launch_iter(nullptr, launched + j);
         if ((e = hipGetLastError()) != hipSuccess) return fail(e);
       }
-      launches += (chunk + 1) / 2;
-      launched += whole ? C : chunk;
+      launched += replay ? C : chunk;
       if (launched >= p.itermax) break;
       // instances still open at the next iteration
       hipLaunchKernelGGL(k_count_active, dim3(1), dim3(64), 0, bs, d_items, n, nullptr, launched, p.itermax, p.tol,
@@ -563,7 +553,7 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
       // where a member's run ended, and the last launch redone up to it if that is inside
       e = qesmc_march_settle_batch(bs, d_march, n, launched, p.tol);
       for (const Group &gr : groups)
-        if (e == hipSuccess) e = launch_march(gr, 1, nullptr, 0, 0, true);
+        if (e == hipSuccess) e = launch_march(gr, 1, 0, 0, true);
       if (e != hipSuccess) return fail(e);
     }
   }

@@ -33,11 +33,9 @@ struct MarchRun {
   int t, itermax;
   int src;  // set this launch reads
   int fix;  // redo the last launch's first iteration if asked to (T = 1 only)
-  // a batch: its problems, the problem of each work-group, and, where the
-  // launch is replayed, the iterations (added to t) and launches (parity added to src) before it
+  // a batch: its problems, and the problem of each work-group
   const MarchItem *items;
   const int *which;
-  const int *base;
 };
 
 }  // namespace qesmc

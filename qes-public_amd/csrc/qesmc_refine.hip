@@ -117,7 +117,7 @@ __global__ __launch_bounds__(256) void k_refine_residual_pairs(Dims d, const flo
 // dst += src over one colour array (every position: the ring and the
 // planes that are never relaxed hold zero in the correction).  With cur the
 // buffer set *cur selects (dst1 / src1 for set 1) stands for the one the
-// two-colour march wrote last; without it set 0.
+// march wrote last; without it set 0.
 __global__ __launch_bounds__(256) void k_refine_add(long long n, float *dst0, float *dst1, const float *src0,
                                                     const float *src1, const unsigned *__restrict__ cur)
 {

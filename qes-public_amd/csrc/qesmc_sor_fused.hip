@@ -116,8 +116,7 @@ typedef unsigned uint2v __attribute__((ext_vector_type(2)));
 // T iterations per launch, NW waves per work-group, RW rows (even) per row
 // group, GW lanes per row group (64: a wave is one group; 32: two).
 // BATCH: the work-group's problem is taken from A.items (A.which per
-// work-group) instead of I, and the iteration and source set from A.base, so
-// that a captured launch can be replayed.
+// work-group) instead of I.
 template <int T, int NW, int RW, int GW, bool BATCH>
 __global__ __launch_bounds__(64 * NW, RW == 2 ? 4 : 2) void k_sor_march(MarchItem I, MarchRun A)
 {
@@ -140,10 +139,6 @@ __global__ __launch_bounds__(64 * NW, RW == 2 ? 4 : 2) void k_sor_march(MarchIte
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int t = A.t, src = A.src;
-  if (BATCH && A.base) {
-    t += A.base[0];
-    src ^= A.base[1] & 1;
-  }
   float om[H];
 #pragma unroll
   for (int h = 0; h < H; ++h) om[h] = A.om[h];
