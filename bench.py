@@ -790,8 +790,8 @@ def roofline_of(results, lups_per_iteration, workload_key, iterations_per_launch
     """Roofline object of the dominant SOR kernel from the run's own HIP-event
     timings: achieved = algorithmic bytes per launch / mean launch time.  With
     iterations_per_launch = 2 (the march) a launch's 13 bytes per cell serve
-    two updates of it, 6.5 bytes each; the march is bound by its caches and
-    vector ALUs then, and the HBM fraction says how far it is from needing HBM."""
+    two updates of it, 6.5 bytes each; where the arrays fit the Infinity
+    Cache the march is bound by the caches and its vector ALUs."""
     last = results[-1]
     its = last["iterations"]
     fused = last["path"] == Q.PATH_FUSED or iterations_per_launch is not None
@@ -812,7 +812,8 @@ def roofline_of(results, lups_per_iteration, workload_key, iterations_per_launch
         kernel = "k_sor_split<%s, %d>" % ("true" if last["compressed"] else "false", last["tile_v"])
     traffic, source = load_traffic(kernel, workload_key)
     ref36 = 36.0 * per_launch_updates / (launch_ms * 1e-3) / 1e9
-    return {"bound": "hbm" if iterations_per_launch is None else "caches and vector ALUs", "kernel": kernel, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
+    in_cache = iterations_per_launch is not None and last["path"] != Q.PATH_FUSED
+    return {"bound": "caches and vector ALUs" if in_cache else "hbm", "kernel": kernel, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
             "traffic_source": source, "bytes_per_lup": bpl, "avg_launch_us": round(launch_ms * 1e3, 2),
             "updates_per_launch": int(per_launch_updates),
