@@ -415,26 +415,21 @@ int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, BatchKind ba
   }
   st.masked = x->compressible;
   const bool march_ready = x->d_lc2[0] && x->d_cur && x->d_canon8 && x->d_mask2 && x->d_top;
-  // QESMC_PATH_AUTO is reported as FUSED where the colour arrays (lambda and
-  // R of both colours, the masks) exceed MI355X's 256 MB Infinity Cache, as
-  // SPLIT otherwise
-  if (p.path == QESMC_PATH_AUTO && st.masked &&
-      x->nsplit < (1LL << 31) && (double)x->nsplit * 2.0 * (4.0 + 4.0 + 1.0) > 256.0 * (1 << 20) &&
-      (!x->no_alloc_run || march_ready))
-    st.path = QESMC_PATH_FUSED;
-  if (st.path == QESMC_PATH_FUSED && !st.masked) return QESMC_ERR_UNSUPPORTED;
-  // the fused path addresses its arrays with 32-bit element offsets
-  if (st.path == QESMC_PATH_FUSED && x->nsplit >= (1LL << 31)) return QESMC_ERR_UNSUPPORTED;
   // The march (two iterations per launch) runs wherever it can: on every wall
-  // mask, unless the caller or the autotuner tiles the colour passes, a
-  // no-allocation run finds its buffers missing, or a plane is beyond its
-  // 32-bit byte offsets.
-  st.march = batch != BatchKind::colours && x->d.splane < (1LL << 28) && x->d.NZ < 32768 &&
-             (st.path == QESMC_PATH_FUSED ||
-              (batch == BatchKind::march && st.masked && x->nsplit < (1LL << 31)) ||
-              (p.path == QESMC_PATH_AUTO && st.masked && x->nsplit < (1LL << 31) && p.tile_k == 0 &&
-               p.tile_v == 0 && p.wg_per_cu == 0 && p.slab_planes == 0 && x->kplanes_auto == 0 &&
-               x->tile_v_auto == 0 && x->wg_per_cu_auto == 0 && (!x->no_alloc_run || march_ready)));
+  // mask below 2^31 half-cells whose planes its 32-bit byte offsets reach.
+  // QESMC_PATH_AUTO takes it unless the caller or the autotuner tiles the
+  // colour passes, or a no-allocation run finds its buffers missing.  Where
+  // the colour arrays (lambda and R of both colours, the masks) exceed
+  // MI355X's 256 MB Infinity Cache, AUTO is the fused path, as which it is
+  // reported, and the tile fields of the colour passes do not apply to it.
+  const bool fits = st.masked && x->nsplit < (1LL << 31);
+  if (st.path == QESMC_PATH_FUSED && !fits) return QESMC_ERR_UNSUPPORTED;
+  const bool beyond = (double)x->nsplit * 2.0 * (4.0 + 4.0 + 1.0) > 256.0 * (1 << 20);
+  const bool untiled = p.tile_k == 0 && p.tile_v == 0 && p.wg_per_cu == 0 && p.slab_planes == 0 &&
+                       x->kplanes_auto == 0 && x->tile_v_auto == 0 && x->wg_per_cu_auto == 0;
+  st.march = batch != BatchKind::colours && fits && x->d.splane < (1LL << 28) && x->d.NZ < 32768 &&
+             (p.path == QESMC_PATH_FUSED || batch == BatchKind::march ||
+              (p.path == QESMC_PATH_AUTO && (beyond || untiled) && (!x->no_alloc_run || march_ready)));
   if (st.march && !march_ready) {
     hipError_t e = hipSuccess;
     if (!x->d_lc2[0]) e = dalloc2(x->d_lc2, x->nsplit);
@@ -443,11 +438,12 @@ int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, BatchKind ba
     if (e == hipSuccess && !x->d_mask2) e = dalloc(&x->d_mask2, (long long)((x->d.NY + 1) / 2) * x->d.HP * x->d.NZ);
     if (e == hipSuccess && !x->d_top) e = dalloc(&x->d_top, qesmc_march_top_words(x->d));
     if (e != hipSuccess) {
-      if (st.path == QESMC_PATH_FUSED) return map_hip(e);
+      if (p.path == QESMC_PATH_FUSED) return map_hip(e);
       (void)hipGetLastError();
       st.march = false;  // no room for a second lambda: the colour passes need none
     }
   }
+  if (st.march && p.path == QESMC_PATH_AUTO && beyond) st.path = QESMC_PATH_FUSED;
   x->kplanes = p.tile_k > 0 ? p.tile_k : x->kplanes_auto;
   x->tile_v = p.tile_v > 0 ? p.tile_v : x->tile_v_auto;
   if (x->kplanes == 0 || x->tile_v == 0) {
@@ -491,9 +487,8 @@ int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, BatchKind ba
     // measured best; the split path's choice above does not apply to it)
     x->kplanes = p.tile_k > 0 ? p.tile_k : 8;
   }
-  if (st.path == QESMC_PATH_FUSED) {
-    // one wave per column tile of tile_k planes (4 or 8; tile_v and
-    // wg_per_cu unused)
+  if (st.path == QESMC_PATH_FUSED && st.march) {
+    // its own tiling is march[]; tile_v and wg_per_cu are unused
     x->kplanes = p.tile_k > 0 ? p.tile_k : 8;
     x->tile_v = 1;
     x->wg_per_cu = 0;

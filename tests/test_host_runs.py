@@ -1,0 +1,113 @@
+"""What the library's host code decides, on the CPU: which kernels a call
+launches, what it allocates, and what becomes of it when an allocation fails.
+
+Each case runs in a process of its own against tests/cpp/hip_stand_in.cpp, a
+stand-in for the HIP runtime whose kernels do nothing; what the kernels compute
+is the GPU tests' business."""
+import ctypes as C
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+FLAT = (1, 4.0, 10.0, 0.5, 230.0)
+
+
+class StandIn:
+    """The stand-in's controls: allocations and launches since reset()."""
+
+    def __init__(self, path):
+        # under the runtime's own soname, so that the library finds it loaded
+        self.lib = C.CDLL(path, mode=C.RTLD_GLOBAL)
+        self.lib.stand_in_value.restype = C.c_longlong
+        self.lib.stand_in_cost.argtypes = [C.c_char_p, C.c_double]
+        self.lib.stand_in_fail_at.argtypes = self.lib.stand_in_fail_above.argtypes = [C.c_longlong]
+        self.lib.stand_in_news.argtypes = [C.c_int, C.c_longlong]
+        self.reset, self.fail_at, self.fail_above = (getattr(self.lib, "stand_in_" + n)
+                                                     for n in ("reset", "fail_at", "fail_above"))
+
+    def launches(self, kernel):
+        return self.lib.stand_in_launches(kernel.encode())
+
+    def cost(self, kernel, us):
+        self.lib.stand_in_cost(kernel.encode(), us)
+
+    def news(self, fail_at=0):
+        """Count this thread's C++ allocations; the fail_at-th fails."""
+        self.lib.stand_in_news(1, fail_at)
+
+    def value(self, what):
+        return self.lib.stand_in_value(
+            ("device_allocs", "host_allocs", "live", "news", "syncs", "graph_launches").index(what))
+
+
+def flat_city(Q, ncx, ncy, ncz):
+    c = Q.Context(0)
+    c.set_city(ncx, ncy, 2.0, Q.dz_uniform(ncz, 1.0), [], FLAT)
+    return c
+
+
+# 32.8 M cells: arrays beyond the 256 MB Infinity Cache, so AUTO is reported as FUSED
+BEYOND = (640, 400, 127)
+LAMBDA = 4 * 640 * 400 * 128  # bytes of the second lambda, at least
+
+
+def case_auto_beyond_the_cache_without_memory(Q, S):
+    """AUTO takes the colour passes, and says so, where the march's buffers
+    cannot be had; an explicit FUSED is refused."""
+    with flat_city(Q, *BEYOND) as c:
+        c.run(itermax=2, path=Q.PATH_SPLIT)  # the convergence rows
+        S.reset()
+        S.fail_above(LAMBDA - 1)
+        r = c.run(itermax=4)
+        assert r["path"] == Q.PATH_SPLIT and r["tile_v"] in (1, 2, 4) and r["wg_per_cu"] > 0, r
+        assert S.launches("k_sor_split") == 8 and S.launches("k_sor_march") == 0
+        try:
+            c.run(itermax=4, path=Q.PATH_FUSED)
+            assert False, "FUSED without its buffers"
+        except Q.QesmcError as e:
+            assert e.code == Q.ERR_OOM
+        S.reset()
+        r = c.run(itermax=4)
+        assert r["path"] == Q.PATH_FUSED and S.launches("k_sor_march") > 0 and S.launches("k_sor_split") == 0
+
+
+def case_batch_with_a_member_without_memory(Q, S):
+    """A member beyond the cache whose march buffers cannot be had sends the
+    whole batch to the colour passes."""
+    with flat_city(Q, 40, 30, 20) as a, flat_city(Q, *BEYOND) as b:
+        for c in (a, b):
+            c.run(itermax=2, path=Q.PATH_SPLIT)
+        S.reset()
+        S.fail_above(LAMBDA - 1)
+        Q.run_batch([a, b], itermax=4, check_every=4, use_graph=False)
+        assert S.launches("k_sor_batch") == 8 and S.launches("k_sor_march") == 0
+
+
+CASES = sorted(n for n in globals() if n.startswith("case_"))
+
+
+@pytest.fixture(scope="session")
+def stand_in(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("stand_in") / "libamdhip64.so.7")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-fPIC", "-shared", "-Wl,-soname,libamdhip64.so.7",
+                    os.path.join(ROOT, "tests", "cpp", "hip_stand_in.cpp"), "-o", out], check=True)
+    return out
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_host_run(stand_in, case):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), case, stand_in], capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0, (r.returncode, r.stdout[-2000:] + r.stderr[-4000:])
+
+
+if __name__ == "__main__":
+    S = StandIn(sys.argv[2])
+    sys.path.insert(0, os.path.join(ROOT, "qes-public_amd"))
+    import qesmc as Q
+
+    globals()[sys.argv[1]](Q, S)
