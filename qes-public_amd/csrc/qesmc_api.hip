@@ -414,7 +414,6 @@ int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, BatchKind ba
     if (rc != QESMC_OK) return rc;
   }
   st.masked = x->compressible;
-  const bool march_ready = x->d_lc2[0] && x->d_cur && x->d_canon8 && x->d_mask2 && x->d_top;
   // The march (two iterations per launch) runs wherever it can: on every wall
   // mask below 2^31 half-cells whose planes its 32-bit byte offsets reach.
   // QESMC_PATH_AUTO takes it unless the caller or the autotuner tiles the
@@ -429,8 +428,8 @@ int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, BatchKind ba
                        x->kplanes_auto == 0 && x->tile_v_auto == 0 && x->wg_per_cu_auto == 0;
   st.march = batch != BatchKind::colours && fits && x->d.splane < (1LL << 28) && x->d.NZ < 32768 &&
              (p.path == QESMC_PATH_FUSED || batch == BatchKind::march ||
-              (p.path == QESMC_PATH_AUTO && (beyond || untiled) && (!x->no_alloc_run || march_ready)));
-  if (st.march && !march_ready) {
+              (p.path == QESMC_PATH_AUTO && (beyond || untiled) && (!x->no_alloc_run || march_ready(x))));
+  if (st.march && !march_ready(x)) {
     hipError_t e = hipSuccess;
     if (!x->d_lc2[0]) e = dalloc2(x->d_lc2, x->nsplit);
     if (e == hipSuccess && !x->d_cur) e = dalloc(&x->d_cur, 1);

@@ -204,6 +204,12 @@ struct qesmc_ctx {
 
 namespace qesmc {
 
+// The march has all its buffers: a run that takes it allocates nothing.
+inline bool march_ready(const qesmc_ctx *x)
+{
+  return x->d_lc2[0] && x->d_cur && x->d_canon8 && x->d_mask2 && x->d_top;
+}
+
 // Phases of one solve shared by qesmc_run and qesmc_run_batch.
 struct RunState {
   qesmc_params p{};

@@ -87,6 +87,23 @@ def case_batch_with_a_member_without_memory(Q, S):
         assert S.launches("k_sor_batch") == 8 and S.launches("k_sor_march") == 0
 
 
+def case_static_run_after_a_half_made_set(Q, S):
+    """Whichever of the march's five buffers could not be had, a FUSED
+    qesmc_run_static is refused and allocates nothing."""
+    for nth in range(1, 6):
+        with flat_city(Q, 40, 30, 20) as c:
+            c.run(itermax=2, path=Q.PATH_SPLIT)
+            S.fail_at(nth)
+            c.run(itermax=2)
+            S.reset()
+            try:
+                c.run_static(itermax=2, path=Q.PATH_FUSED)
+                assert False, nth
+            except Q.QesmcError as e:
+                assert e.code == Q.ERR_STATE, (nth, e.code)
+            assert S.value("device_allocs") == S.value("host_allocs") == 0, nth
+
+
 CASES = sorted(n for n in globals() if n.startswith("case_"))
 
 
