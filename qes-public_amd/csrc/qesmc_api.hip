@@ -88,8 +88,32 @@ void dfree2(float **p)
   p[1] = nullptr;
 }
 
+void free_march(qesmc_ctx *x)
+{
+  dfree2(x->d_lc2);
+  dfree(x->d_cur);
+  dfree(x->d_canon8);
+  dfree(x->d_mask2);
+  dfree(x->d_top);
+  x->pair_masks = false;
+}
+
+// The march's buffers, all of them or none.
+hipError_t alloc_march(qesmc_ctx *x)
+{
+  const qesmc::Dims &d = x->d;
+  hipError_t e = dalloc2(x->d_lc2, x->nsplit);
+  if (e == hipSuccess) e = dalloc(&x->d_cur, 1);
+  if (e == hipSuccess) e = dalloc(&x->d_canon8, (8LL + 64LL) * d.NZ);
+  if (e == hipSuccess) e = dalloc(&x->d_mask2, (long long)((d.NY + 1) / 2) * d.HP * d.NZ);
+  if (e == hipSuccess) e = dalloc(&x->d_top, qesmc_march_top_words(d));
+  if (e != hipSuccess) free_march(x);
+  return e;
+}
+
 void free_geometry(qesmc_ctx *x)
 {
+  free_march(x);
   for (auto &p : x->d_coef) dfree(p);
   dfree(x->d_flag);
   dfree(x->d_dz);
@@ -105,18 +129,13 @@ void free_geometry(qesmc_ctx *x)
   x->have_velocity = false;
   dfree2(x->d_lc);
   dfree2(x->d_Rc);
-  dfree2(x->d_lc2);
   dfree2(x->d_R0);
   dfree2(x->d_base);
   for (int c = 0; c < 2; ++c) {
     dfree(x->d_mask[c]);
     for (auto &p : x->d_cc[c]) dfree(p);
   }
-  dfree(x->d_mask2);
-  dfree(x->d_top);
-  x->pair_masks = false;
   dfree(x->d_canon);
-  dfree(x->d_canon8);
   x->have_geom = x->have_inflow = false;
   x->geom_checked = false;
   x->d = qesmc::Dims{};
@@ -307,7 +326,6 @@ int qesmc_destroy(qesmc_ctx *x)
   dfree(x->d_err);
   dfree(x->d_status);
   dfree(x->d_norm);
-  dfree(x->d_cur);
   dfree(x->d_probe);
   dfree(x->d_probe_val);
   if (x->h_poll) (void)hipHostFree(x->h_poll);
@@ -430,12 +448,7 @@ int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, BatchKind ba
              (p.path == QESMC_PATH_FUSED || batch == BatchKind::march ||
               (p.path == QESMC_PATH_AUTO && (beyond || untiled) && (!x->no_alloc_run || march_ready(x))));
   if (st.march && !march_ready(x)) {
-    hipError_t e = hipSuccess;
-    if (!x->d_lc2[0]) e = dalloc2(x->d_lc2, x->nsplit);
-    if (e == hipSuccess && !x->d_cur) e = dalloc(&x->d_cur, 1);
-    if (e == hipSuccess && !x->d_canon8) e = dalloc(&x->d_canon8, (8LL + 64LL) * x->d.NZ);
-    if (e == hipSuccess && !x->d_mask2) e = dalloc(&x->d_mask2, (long long)((x->d.NY + 1) / 2) * x->d.HP * x->d.NZ);
-    if (e == hipSuccess && !x->d_top) e = dalloc(&x->d_top, qesmc_march_top_words(x->d));
+    const hipError_t e = alloc_march(x);
     if (e != hipSuccess) {
       if (p.path == QESMC_PATH_FUSED) return map_hip(e);
       (void)hipGetLastError();

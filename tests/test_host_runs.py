@@ -104,6 +104,28 @@ def case_static_run_after_a_half_made_set(Q, S):
             assert S.value("device_allocs") == S.value("host_allocs") == 0, nth
 
 
+def case_half_made_set_is_given_back(Q, S):
+    """A run that cannot have all of the march's buffers keeps none of them,
+    whether it goes on with the colour passes or is refused."""
+    for nth in range(1, 6):
+        with flat_city(Q, 40, 30, 20) as c:
+            c.run(itermax=2, path=Q.PATH_SPLIT)
+            before = S.value("live")
+            S.fail_at(nth)
+            assert c.run(itermax=2)["path"] == Q.PATH_SPLIT
+            assert S.value("live") == before, nth
+            S.fail_at(nth)
+            try:
+                c.run(itermax=2, path=Q.PATH_FUSED)
+                assert False, nth
+            except Q.QesmcError as e:
+                assert e.code == Q.ERR_OOM
+            assert S.value("live") == before, nth
+            S.reset()
+            c.run(itermax=2)
+            assert S.launches("k_sor_march") > 0 and S.value("live") > before
+
+
 CASES = sorted(n for n in globals() if n.startswith("case_"))
 
 
