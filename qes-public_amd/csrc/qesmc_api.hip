@@ -36,7 +36,7 @@ hipError_t qesmc_launch_fill_u32(qesmc_ctx *x, unsigned *p, long long count, uns
 hipError_t qesmc_launch_rows_summary(qesmc_ctx *x, int launched, float tol);
 hipError_t qesmc_fused_prepare(qesmc_ctx *x);
 long long qesmc_march_top_words(const qesmc::Dims &d);
-void qesmc_march_costs(qesmc_ctx *x, const int *top);
+void qesmc_march_costs(qesmc_ctx *x);
 void qesmc_march_choose(qesmc_ctx *x, int tile_k);
 
 namespace {
@@ -95,6 +95,8 @@ void free_march(qesmc_ctx *x)
   dfree(x->d_canon8);
   dfree(x->d_mask2);
   dfree(x->d_top);
+  if (x->h_top) (void)hipHostFree(x->h_top);
+  x->h_top = nullptr;
   x->pair_masks = false;
 }
 
@@ -106,7 +108,16 @@ hipError_t alloc_march(qesmc_ctx *x)
   if (e == hipSuccess) e = dalloc(&x->d_cur, 1);
   if (e == hipSuccess) e = dalloc(&x->d_canon8, (8LL + 64LL) * d.NZ);
   if (e == hipSuccess) e = dalloc(&x->d_mask2, (long long)((d.NY + 1) / 2) * d.HP * d.NZ);
-  if (e == hipSuccess) e = dalloc(&x->d_top, qesmc_march_top_words(d));
+  const long long top = qesmc_march_top_words(d);
+  if (e == hipSuccess) e = dalloc(&x->d_top, top);
+  if (e == hipSuccess) e = hipHostMalloc((void **)&x->h_top, sizeof(int) * (size_t)top, hipHostMallocDefault);
+  if (e == hipSuccess) {
+    try {
+      x->march_cost.resize((size_t)d.NZ + 4);
+    } catch (const std::bad_alloc &) {
+      e = hipErrorOutOfMemory;
+    }
+  }
   if (e != hipSuccess) free_march(x);
   return e;
 }
@@ -533,10 +544,10 @@ int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, BatchKind ba
     if (!x->pair_masks) {
       HIPCHK(qesmc_fused_prepare(x));
       x->march_tile_k = -1;
-      std::vector<int> top((size_t)qesmc_march_top_words(x->d));
-      HIPCHK(hipMemcpyAsync(top.data(), x->d_top, sizeof(int) * top.size(), hipMemcpyDeviceToHost, s));
+      HIPCHK(hipMemcpyAsync(x->h_top, x->d_top, sizeof(int) * (size_t)qesmc_march_top_words(x->d),
+                            hipMemcpyDeviceToHost, s));
       HIPCHK(hipStreamSynchronize(s));
-      qesmc_march_costs(x, top.data());
+      qesmc_march_costs(x);
       x->pair_masks = true;
     }
     if (batch == BatchKind::none && x->march_tile_k != p.tile_k) {

@@ -172,6 +172,7 @@ struct qesmc_ctx {
   unsigned char *d_mask[2] = {};
   unsigned *d_mask2 = nullptr; // march: both colours' masks in the pair layout, two rows a word (allocated on first use)
   int *d_top = nullptr;        // march: highest plane with a wall, per two rows and 32 pairs
+  int *h_top = nullptr;        // march: the same on the host (pinned)
   bool pair_masks = false;           // d_mask2, d_top and d_canon8 hold the resident geometry's
   float *d_cc[2][6] = {};     // full coefficients, split (only if not compressible)
   unsigned *d_canon = nullptr; // 6*NZ wall values per layer (float bits)
@@ -198,7 +199,7 @@ struct qesmc_ctx {
   int slab_planes_auto = 0;    // default when qesmc_params.slab_planes == 0
   qesmc::MarchPlan march[2];   // tiling of the march's launches of one and of two iterations
   int march_tile_k = -1;       // the tile_k they were chosen for (-1: not chosen)
-  std::vector<double> march_cost; // cost of the march's steps below each plane (with pair_masks)
+  std::vector<double> march_cost; // cost of the march's steps below each plane (with pair_masks; sized with the buffers)
   int n_cu = 256;              // compute units of the device
 };
 
@@ -207,7 +208,7 @@ namespace qesmc {
 // The march has all its buffers: a run that takes it allocates nothing.
 inline bool march_ready(const qesmc_ctx *x)
 {
-  return x->d_lc2[0] && x->d_cur && x->d_canon8 && x->d_mask2 && x->d_top;
+  return x->d_lc2[0] && x->d_cur && x->d_canon8 && x->d_mask2 && x->d_top && x->h_top;
 }
 
 // Phases of one solve shared by qesmc_run and qesmc_run_batch.

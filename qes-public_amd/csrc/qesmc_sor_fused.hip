@@ -619,21 +619,22 @@ constexpr double kLaunchUs = 4.6;
 
 // The cost of the steps below p, for all p, from the table of highest walls:
 // 1 for an open plane, and 0.32 more for the share of the columns that have a wall there or above.
-void qesmc_march_costs(qesmc_ctx *x, const int *top)
+// In place, so that a run that may not allocate can do it.
+void qesmc_march_costs(qesmc_ctx *x)
 {
-  const Dims &d = x->d;
-  std::vector<double> w((size_t)d.NZ, 1.0);
-  const long long n = qesmc_march_top_words(d);
-  std::vector<int> count((size_t)d.NZ + 1, 0);
-  for (long long q = 0; q < n; ++q) ++count[(size_t)top[q]];
-  long long above = n;
-  for (int k = 0; k < d.NZ; ++k) {
-    w[(size_t)k] = 1.0 + 0.32 * (double)above / (double)n;
-    above -= count[(size_t)k];
+  const size_t NZ = (size_t)x->d.NZ;
+  const long long n = qesmc_march_top_words(x->d);
+  std::vector<double> &c = x->march_cost;
+  std::fill(c.begin(), c.end(), 0.0);
+  // first, one place up, the columns whose highest wall is plane k
+  for (long long q = 0; q < n; ++q) c[(size_t)x->h_top[q] + 1] += 1.0;
+  double above = (double)n, w = 1.0;
+  for (size_t k = 0; k + 1 < c.size(); ++k) {
+    const double here = c[k + 1];
+    if (k < NZ) w = 1.0 + 0.32 * above / (double)n;
+    above -= here;
+    c[k + 1] = c[k] + w;
   }
-  x->march_cost.assign((size_t)d.NZ + 4, 0.0);
-  for (size_t p = 0; p + 1 < x->march_cost.size(); ++p)
-    x->march_cost[p + 1] = x->march_cost[p] + w[p < w.size() ? p : w.size() - 1];
 }
 
 // The march's shape and segments for the resident domain.  A segment's time is the sum of its steps' and the launch's

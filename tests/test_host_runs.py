@@ -126,6 +126,20 @@ def case_half_made_set_is_given_back(Q, S):
             assert S.launches("k_sor_march") > 0 and S.value("live") > before
 
 
+def case_static_run_on_a_new_geometry(Q, S):
+    """qesmc_run_static allocates nothing, on the device or the host, on its
+    first march after a new geometry of the same size."""
+    with flat_city(Q, 300, 40, 20) as c:
+        c.run(itermax=2)
+        for path in (Q.PATH_AUTO, Q.PATH_FUSED):
+            c.set_city(300, 40, 2.0, Q.dz_uniform(20, 1.0), [], FLAT)
+            S.reset()
+            S.news()
+            c.run_static(itermax=4, path=path)
+            assert S.value("news") == S.value("device_allocs") == S.value("host_allocs") == 0, S.value("news")
+            assert S.launches("k_pair_masks") == 1 and S.launches("k_sor_march") > 0
+
+
 CASES = sorted(n for n in globals() if n.startswith("case_"))
 
 
