@@ -13,9 +13,9 @@
 // runtime's copy) and freed with the device's last context.
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -188,8 +188,8 @@ hipError_t host_copy(int device, hipStream_t st, const HostPiece *p, int n, bool
     const int want = (int)(count / 2 < (size_t)kWorkers ? count / 2 : (size_t)kWorkers);
     try {
       for (; started < want; ++started) threads[started] = std::thread(work);
-    } catch (const std::system_error &) {
-      // fewer threads do the work; without any the runtime does
+    } catch (const std::exception &) {
+      // no thread or no memory for one: fewer do the work; without any the runtime does
     }
     if (started == 0) {
       give_back(s);

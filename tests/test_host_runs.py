@@ -140,6 +140,34 @@ def case_static_run_on_a_new_geometry(Q, S):
             assert S.launches("k_pair_masks") == 1 and S.launches("k_sor_march") > 0
 
 
+def refusing_each_allocation(Q, S, call):
+    """call() once for every C++ allocation it makes, that one refused: it
+    returns (a status, not an exception across the C interface)."""
+    refused = 0
+    for nth in range(1, 10000):
+        S.news(fail_at=nth)
+        try:
+            call()
+        except Q.QesmcError as e:
+            assert e.code == Q.ERR_OOM, e.code
+            refused += 1
+        hit = S.value("news") >= nth
+        S.news()
+        if not hit:
+            return refused
+    assert False, "never done"
+
+
+def case_no_host_memory_for_a_copy(Q, S):
+    """A large copy without the memory for its chunks or its threads."""
+    with flat_city(Q, 200, 200, 60) as c:
+        c.run(itermax=2)
+        refusing_each_allocation(Q, S, c.get_velocity)
+        refusing_each_allocation(Q, S, lambda: c.run(itermax=2))
+        u, v, w = c.get_velocity()
+        assert not u.any() and not v.any() and not w.any()
+
+
 CASES = sorted(n for n in globals() if n.startswith("case_"))
 
 
