@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <new>
 #include <vector>
 
 #include "qesmc_march.h"
@@ -293,7 +294,16 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
   qesmc_ctx *lead = ctxs[0];
   BCHK(hipSetDevice(lead->device));
   hipStream_t bs = lead->stream;
-  std::vector<hipStream_t> own_streams(n);
+  std::vector<hipStream_t> own_streams;
+  std::vector<RunState> st;
+  std::vector<BatchItem> items;
+  try {
+    own_streams.resize((size_t)n);
+    st.resize((size_t)n);
+    items.resize((size_t)n);
+  } catch (const std::bad_alloc &) {
+    return QESMC_ERR_OOM;
+  }
   // every instance's own work completes before any context is moved to the
   // batch stream, so a failure here leaves every context untouched
   for (int i = 0; i < n; ++i) BCHK(hipStreamSynchronize(ctxs[i]->stream));
@@ -304,7 +314,6 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
   auto restore = [&]() {
     for (int i = 0; i < n; ++i) ctxs[i]->stream = own_streams[i];
   };
-  std::vector<RunState> st(n);
   int rc = QESMC_OK;
   for (;;) {
     for (int i = 0; i < n && rc == QESMC_OK; ++i)
@@ -321,7 +330,6 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
   }
   const qesmc_params &p = st[0].p;
   // device table
-  std::vector<BatchItem> items(n);
   long long total = 0;
   for (int i = 0; i < n; ++i) {
     qesmc_ctx *x = ctxs[i];
@@ -389,54 +397,59 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
     std::vector<MarchPlan> plans;  // for two iterations a launch
   };
   std::vector<Group> groups;
-  std::vector<MarchItem> mitems(march ? 2 * (size_t)n : 0);
+  std::vector<MarchItem> mitems;
   std::vector<int> which;  // the member of each work-group, per group and iterations per launch
   if (march) {
-    constexpr double kCache = 256.0 * (1 << 20);
-    double bytes = 0.0, least = 1e300;
-    for (int i = 0; i < n; ++i) bytes += 13.0 * (double)ctxs[i]->ncell;
-    const int most = bytes <= kCache ? 1 : (int)std::min((double)n, std::ceil(bytes / (0.5 * kCache)));
-    for (int count = 1; count <= most; count += count < 4 ? 1 : count) {
-      std::vector<Group> trial;
-      double us = 0.0, done = 0.0;
-      for (int i = 0; i < n;) {
-        Group gr{i, i, {}, {}, {}, {}};
-        double mine = 0.0;
-        // up to the next multiple of the share, to the nearest member
-        const double until = bytes * (double)(trial.size() + 1) / count;
-        while (gr.end < n) {
-          const double b = 13.0 * (double)ctxs[gr.end]->ncell;
-          if (gr.end > i && done + 0.5 * b > until) break;
-          done += b;
-          mine += b;
-          ++gr.end;
+    try {
+      mitems.resize(2 * (size_t)n);
+      constexpr double kCache = 256.0 * (1 << 20);
+      double bytes = 0.0, least = 1e300;
+      for (int i = 0; i < n; ++i) bytes += 13.0 * (double)ctxs[i]->ncell;
+      const int most = bytes <= kCache ? 1 : (int)std::min((double)n, std::ceil(bytes / (0.5 * kCache)));
+      for (int count = 1; count <= most; count += count < 4 ? 1 : count) {
+        std::vector<Group> trial;
+        double us = 0.0, done = 0.0;
+        for (int i = 0; i < n;) {
+          Group gr{i, i, {}, {}, {}, {}};
+          double mine = 0.0;
+          // up to the next multiple of the share, to the nearest member
+          const double until = bytes * (double)(trial.size() + 1) / count;
+          while (gr.end < n) {
+            const double b = 13.0 * (double)ctxs[gr.end]->ncell;
+            if (gr.end > i && done + 0.5 * b > until) break;
+            done += b;
+            mine += b;
+            ++gr.end;
+          }
+          double t = 0.0;
+          gr.shape[1] = qesmc_march_batch_plan(ctxs + i, gr.end - i, 2, gr.plans, &t);
+          if (gr.shape[1] < 0) return fail(hipErrorInvalidValue);
+          us += t * (mine > kCache ? 1.0 + 0.6 * (1.0 - kCache / mine) : 1.0);
+          i = gr.end;
+          trial.push_back(std::move(gr));
         }
-        double t = 0.0;
-        gr.shape[1] = qesmc_march_batch_plan(ctxs + i, gr.end - i, 2, gr.plans, &t);
-        if (gr.shape[1] < 0) return fail(hipErrorInvalidValue);
-        us += t * (mine > kCache ? 1.0 + 0.6 * (1.0 - kCache / mine) : 1.0);
-        i = gr.end;
-        trial.push_back(std::move(gr));
-      }
-      if (us < least) {
-        least = us;
-        groups = std::move(trial);
-      }
-    }
-    std::vector<MarchPlan> single;
-    for (Group &gr : groups) {
-      const int m = gr.end - gr.begin;
-      gr.shape[0] = qesmc_march_batch_plan(ctxs + gr.begin, m, 1, single, nullptr);
-      if (gr.shape[0] < 0) return fail(hipErrorInvalidValue);
-      for (int T = 1; T <= 2; ++T) {
-        gr.which[T - 1] = (int)which.size();
-        for (int i = 0; i < m; ++i) {
-          MarchItem &it = mitems[(size_t)(T - 1) * n + gr.begin + i];
-          qesmc_march_item(ctxs[gr.begin + i], T == 1 ? single[(size_t)i] : gr.plans[(size_t)i], gr.slots[T - 1], it);
-          which.insert(which.end(), (size_t)it.slots, gr.begin + i);
-          gr.slots[T - 1] += it.slots;
+        if (us < least) {
+          least = us;
+          groups = std::move(trial);
         }
       }
+      std::vector<MarchPlan> single;
+      for (Group &gr : groups) {
+        const int m = gr.end - gr.begin;
+        gr.shape[0] = qesmc_march_batch_plan(ctxs + gr.begin, m, 1, single, nullptr);
+        if (gr.shape[0] < 0) return fail(hipErrorInvalidValue);
+        for (int T = 1; T <= 2; ++T) {
+          gr.which[T - 1] = (int)which.size();
+          for (int i = 0; i < m; ++i) {
+            MarchItem &it = mitems[(size_t)(T - 1) * n + gr.begin + i];
+            qesmc_march_item(ctxs[gr.begin + i], T == 1 ? single[(size_t)i] : gr.plans[(size_t)i], gr.slots[T - 1], it);
+            which.insert(which.end(), (size_t)it.slots, gr.begin + i);
+            gr.slots[T - 1] += it.slots;
+          }
+        }
+      }
+    } catch (const std::bad_alloc &) {
+      return fail(hipErrorOutOfMemory);
     }
     const size_t tb = sizeof(MarchItem) * mitems.size();
     if ((e = hipMalloc((void **)&d_march, tb + sizeof(int) * (which.size() + 1))) != hipSuccess) return fail(e);

@@ -158,6 +158,18 @@ def refusing_each_allocation(Q, S, call):
     assert False, "never done"
 
 
+def case_no_host_memory_for_a_batch(Q, S):
+    ctxs = [flat_city(Q, 30 + 5 * q, 40, 20) for q in range(3)]
+    for kw in (dict(), dict(path=Q.PATH_SPLIT)):
+        n = refusing_each_allocation(Q, S, lambda: Q.run_batch(ctxs, itermax=4, check_every=4, use_graph=True, **kw))
+        assert n >= 3
+        S.reset()
+        Q.run_batch(ctxs, itermax=4, check_every=4, use_graph=False, **kw)  # as if nothing had happened
+        assert S.launches("k_sor_march" if not kw else "k_sor_batch") > 0
+    for c in ctxs:
+        c.close()
+
+
 def case_no_host_memory_for_a_copy(Q, S):
     """A large copy without the memory for its chunks or its threads."""
     with flat_city(Q, 200, 200, 60) as c:
