@@ -70,12 +70,15 @@ typedef struct qesmc_fields {
 /* Kernel path selection (qesmc_params.path). */
 #define QESMC_PATH_AUTO 0     /* fastest available.  On a wall mask: whole
                                  iterations per launch, as FUSED, unless the
-                                 tile fields or qesmc_autotune tile the colour
-                                 passes, or its second lambda buffer cannot be
-                                 had (no memory, or not yet allocated in a
-                                 qesmc_run_static call); else SPLIT.  Reported
-                                 as FUSED where the colour arrays exceed the
-                                 256 MB Infinity Cache, as SPLIT otherwise     */
+                                 tile fields tile the colour passes (where the
+                                 colour arrays exceed the 256 MB Infinity Cache
+                                 they do not apply, as on FUSED),
+                                 qesmc_autotune found these faster, or the
+                                 march's buffers cannot be had (no memory, or
+                                 not yet allocated in a qesmc_run_static call);
+                                 else SPLIT.  Whole iterations per launch are
+                                 reported as FUSED beyond the Infinity Cache,
+                                 as SPLIT within it                            */
 #define QESMC_PATH_PLAIN 1    /* in-place red/black launches on the x-fastest
                                  layout, full fp32 coefficients: the classic
                                  GPU red-black SOR (baseline)                   */
@@ -238,9 +241,12 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
                     int use_graph, double *ms_loop);
 
 /* Time `iterations` SOR iterations of the resident problem for a set of
- * candidate tilings (tile_k, tile_v, wg_per_cu) and keep the fastest as the
- * context's default for tile fields left at 0.  lambda is restored.  best
- * (optional) receives base with the chosen tile fields. */
+ * candidate tilings (tile_k, tile_v, wg_per_cu) of the colour passes and keep
+ * the fastest as the context's default for tile fields left at 0.  With
+ * base->path AUTO or FUSED whole iterations per launch are timed too, and
+ * QESMC_PATH_AUTO leaves them on this grid only if the colour passes were
+ * faster.  lambda is restored.  best (optional) receives base with the chosen
+ * tile fields; a run of this context that is given them decides as with 0. */
 int qesmc_autotune(qesmc_ctx *ctx, const qesmc_params *base, int iterations, qesmc_params *best);
 
 /* ---- input builder (flat stair-step cities) ------------------------------ */

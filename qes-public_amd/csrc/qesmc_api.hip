@@ -228,6 +228,7 @@ int geometry_reserve(qesmc_ctx *x, int nx, int ny, int nz)
   if (x->d.nx != nx || x->d.ny != ny || x->d.nz != nz || !x->d_lam) {
     HIPCHK(hipStreamSynchronize(x->stream));
     free_geometry(x);
+  x->colours_faster = false;  // measured on another grid
     int rc = alloc_geometry(x, nx, ny, nz);
     if (rc != QESMC_OK) {
       free_geometry(x);
@@ -445,19 +446,23 @@ int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, BatchKind ba
   st.masked = x->compressible;
   // The march (two iterations per launch) runs wherever it can: on every wall
   // mask below 2^31 half-cells whose planes its 32-bit byte offsets reach.
-  // QESMC_PATH_AUTO takes it unless the caller or the autotuner tiles the
-  // colour passes, or a no-allocation run finds its buffers missing.  Where
+  // QESMC_PATH_AUTO takes it unless the caller tiles the colour passes, the
+  // autotuner found them faster, or a no-allocation run finds its buffers missing.  Where
   // the colour arrays (lambda and R of both colours, the masks) exceed
   // MI355X's 256 MB Infinity Cache, AUTO is the fused path, as which it is
   // reported, and the tile fields of the colour passes do not apply to it.
   const bool fits = st.masked && x->nsplit < (1LL << 31);
   if (st.path == QESMC_PATH_FUSED && !fits) return QESMC_ERR_UNSUPPORTED;
   const bool beyond = (double)x->nsplit * 2.0 * (4.0 + 4.0 + 1.0) > 256.0 * (1 << 20);
-  const bool untiled = p.tile_k == 0 && p.tile_v == 0 && p.wg_per_cu == 0 && p.slab_planes == 0 &&
-                       x->kplanes_auto == 0 && x->tile_v_auto == 0 && x->wg_per_cu_auto == 0;
+  // the tile fields the autotuner returned mean what 0 does
+  const bool tuned = p.tile_k > 0 && p.tile_k == x->kplanes_auto && p.tile_v == x->tile_v_auto &&
+                     p.wg_per_cu == x->wg_per_cu_auto;
+  const bool untiled = (tuned || (p.tile_k == 0 && p.tile_v == 0 && p.wg_per_cu == 0)) && p.slab_planes == 0;
+  const int march_tile_k = tuned ? 0 : p.tile_k;
   st.march = batch != BatchKind::colours && fits && x->d.splane < (1LL << 28) && x->d.NZ < 32768 &&
              (p.path == QESMC_PATH_FUSED || batch == BatchKind::march ||
-              (p.path == QESMC_PATH_AUTO && (beyond || untiled) && (!x->no_alloc_run || march_ready(x))));
+              (p.path == QESMC_PATH_AUTO && (beyond || untiled) && !x->colours_faster &&
+               (!x->no_alloc_run || march_ready(x))));
   if (st.march && !march_ready(x)) {
     const hipError_t e = alloc_march(x);
     if (e != hipSuccess) {
@@ -550,9 +555,9 @@ int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, BatchKind ba
       qesmc_march_costs(x);
       x->pair_masks = true;
     }
-    if (batch == BatchKind::none && x->march_tile_k != p.tile_k) {
-      qesmc_march_choose(x, p.tile_k);
-      x->march_tile_k = p.tile_k;
+    if (batch == BatchKind::none && x->march_tile_k != march_tile_k) {
+      qesmc_march_choose(x, march_tile_k);
+      x->march_tile_k = march_tile_k;
     }
     HIPCHK(qesmc_launch_pack_pairs(x, true));
     HIPCHK(qesmc_launch_set_u32(x, x->d_cur, 0u));

@@ -586,8 +586,9 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
   return rc;
 }
 
-// Time `iterations` SOR iterations for each candidate tiling on the resident
-// problem and keep the fastest as the context's default (tile fields 0).
+// Time `iterations` SOR iterations for each candidate tiling of the colour
+// passes on the resident problem and keep the fastest as the context's default
+// (tile fields 0), and time the march: AUTO leaves it only if they are faster.
 // lambda is saved and restored, so the problem's state is unchanged.
 int qesmc_autotune(qesmc_ctx *x, const qesmc_params *base, int iterations, qesmc_params *best)
 {
@@ -607,29 +608,47 @@ int qesmc_autotune(qesmc_ctx *x, const qesmc_params *base, int iterations, qesmc
   static const int cand[][3] = {{4, 2, 4}, {8, 2, 4}, {10, 2, 6}, {6, 2, 4}, {7, 2, 5},
                                 {3, 2, 4}, {10, 2, 8}, {6, 2, 8}, {2, 2, 4}, {4, 1, 5},
                                 {6, 1, 6}, {10, 1, 6}, {2, 1, 5}, {1, 2, 4}, {1, 1, 6}};
-  double best_ms = 1e300;
+  double best_ms = 1e300, march_ms = 1e300;
   int bi = 0, rc = QESMC_OK;
+  auto time_of = [&](qesmc_params p, double *ms) {
+    p.tol = -1.0f;  // never converges: every candidate runs the same iterations
+    p.flags &= ~QESMC_RUN_REENCODE;
+    qesmc_result r;
+    int got = QESMC_OK;
+    for (int rep = 0; rep < 2 && got == QESMC_OK; ++rep) {  // first repetition warms caches
+      const hipError_t e =
+          hipMemcpyAsync(x->d_lam, saved, sizeof(float) * (size_t)x->ncell, hipMemcpyDeviceToDevice, x->stream);
+      got = e != hipSuccess ? map_hip_error(e) : qesmc_run(x, &p, &r);
+      *ms = r.ms_sor;
+    }
+    return got;
+  };
   for (int c = 0; c < (int)(sizeof(cand) / sizeof(cand[0])); ++c) {
     qesmc_params p = *base;
     p.path = QESMC_PATH_SPLIT;
     p.itermax = iterations;
-    p.tol = -1.0f;  // never converges: every candidate runs the same iterations
     p.tile_k = cand[c][0];
     p.tile_v = cand[c][1];
     p.wg_per_cu = cand[c][2];
-    p.flags &= ~QESMC_RUN_REENCODE;
-    qesmc_result r;
     double ms = 0.0;
-    for (int rep = 0; rep < 2 && rc == QESMC_OK; ++rep) {  // first repetition warms caches
-      const hipError_t e =
-          hipMemcpyAsync(x->d_lam, saved, sizeof(float) * (size_t)x->ncell, hipMemcpyDeviceToDevice, x->stream);
-      rc = e != hipSuccess ? map_hip_error(e) : qesmc_run(x, &p, &r);
-      ms = r.ms_sor;
-    }
-    if (rc != QESMC_OK) break;
+    if ((rc = time_of(p, &ms)) != QESMC_OK) break;
     if (ms < best_ms) {
       best_ms = ms;
       bi = c;
+    }
+  }
+  if (rc == QESMC_OK && x->compressible && (base->path == QESMC_PATH_AUTO || base->path == QESMC_PATH_FUSED)) {
+    // over enough iterations that the two launches that end a run of the march weigh little
+    qesmc_params p = *base;
+    p.path = QESMC_PATH_FUSED;
+    p.itermax = iterations > 40 ? iterations : 40;
+    p.tile_k = p.tile_v = p.wg_per_cu = 0;
+    rc = time_of(p, &march_ms);
+    march_ms /= p.itermax;  // an iteration
+    if (rc == QESMC_ERR_OOM || rc == QESMC_ERR_UNSUPPORTED) {
+      (void)hipGetLastError();
+      rc = QESMC_OK;
+      march_ms = 1e300;
     }
   }
   (void)hipMemcpyAsync(x->d_lam, saved, sizeof(float) * (size_t)x->ncell, hipMemcpyDeviceToDevice, x->stream);
@@ -639,6 +658,7 @@ int qesmc_autotune(qesmc_ctx *x, const qesmc_params *base, int iterations, qesmc
   x->kplanes_auto = cand[bi][0];
   x->tile_v_auto = cand[bi][1];
   x->wg_per_cu_auto = cand[bi][2];
+  x->colours_faster = march_ms < 1e300 && best_ms / iterations < march_ms;
   if (best) {
     *best = *base;
     best->tile_k = cand[bi][0];

@@ -195,6 +195,7 @@ struct qesmc_ctx {
   int tile_v_auto = 0;         // 0: chosen per run from the domain size
   int wg_per_cu = 8;           // resident work-groups per CU of the split kernel
   int wg_per_cu_auto = 0;      // 0: chosen per run from tile_v
+  bool colours_faster = false; // the autotuner measured the tuned colour passes faster than the march
   int slab_planes = 0;         // split path: k-slab of the interleaved red/black schedule (this run; 0: whole passes)
   int slab_planes_auto = 0;    // default when qesmc_params.slab_planes == 0
   qesmc::MarchPlan march[2];   // tiling of the march's launches of one and of two iterations

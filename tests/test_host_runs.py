@@ -180,6 +180,54 @@ def case_no_host_memory_for_a_copy(Q, S):
         assert not u.any() and not v.any() and not w.any()
 
 
+def tiles(r):
+    return (r["tile_k"], r["tile_v"], r["wg_per_cu"])
+
+
+def case_autotune_keeps_the_march_where_it_is_faster(Q, S):
+    """The tuned tiling of the colour passes is kept and reported, and AUTO
+    goes on marching: with tile fields 0 and with the tuned ones."""
+    for dims, path in (((40, 30, 20), Q.PATH_SPLIT), (BEYOND, Q.PATH_FUSED)):
+        with flat_city(Q, *dims) as c:
+            S.cost("k_sor_split", 20.0)
+            for iterations in (1, 20):
+                best = Q.autotune(c, iterations=iterations)
+                assert best.tile_k > 0 and best.tile_v > 0 and best.wg_per_cu > 0
+                for p in (Q.default_params(itermax=10), best):
+                    p.itermax = 10
+                    S.reset()
+                    r = c.run(p)
+                    assert S.launches("k_sor_march") > 0 and S.launches("k_sor_split") == 0, iterations
+                    assert r["path"] == path and (path == Q.PATH_FUSED or tiles(r) == tiles(vars_of(best)))
+            if path == Q.PATH_SPLIT:  # another tiling, or a path, is still the caller's word
+                for kw in (dict(tile_v=3 - min(best.tile_v, 2)), dict(tile_k=best.tile_k), dict(path=Q.PATH_SPLIT)):
+                    S.reset()
+                    c.run(itermax=10, **kw)
+                    assert S.launches("k_sor_march") == 0 and S.launches("k_sor_split") == 20, kw
+
+
+def vars_of(p):
+    return {n: getattr(p, n) for n, _ in p._fields_}
+
+
+def case_autotune_leaves_the_march_where_it_is_slower(Q, S):
+    for dims in ((40, 30, 20), BEYOND):
+        with flat_city(Q, *dims) as c:
+            S.cost("k_sor_march", 1000.0)
+            best = Q.autotune(c, iterations=20)
+            for p in (Q.default_params(), best):
+                p.itermax = 10
+                S.reset()
+                r = c.run(p)
+                assert S.launches("k_sor_march") == 0 and S.launches("k_sor_split") == 20
+                assert r["path"] == Q.PATH_SPLIT and tiles(r) == tiles(vars_of(best))
+            # another grid has not been tuned
+            c.set_city(50, 30, 2.0, Q.dz_uniform(20, 1.0), [], FLAT)
+            S.reset()
+            c.run(itermax=10)
+            assert S.launches("k_sor_march") > 0
+
+
 CASES = sorted(n for n in globals() if n.startswith("case_"))
 
 
