@@ -156,8 +156,11 @@ typedef struct qesmc_result {
   double ms_total;           /* device time of R + SOR + correction (HIP events)  */
   double ms_sor;             /* device time of the SOR loop alone                 */
   double glups;              /* (nx-3)(ny-3)(nz-3) * iterations / ms_sor          */
-  int tile_k, tile_v, wg_per_cu; /* tiling that ran                               */
-  int reserved;
+  int tile_k, tile_v, wg_per_cu; /* tiling of the colour passes, chosen whether they
+                                ran or whole iterations per launch (path FUSED:
+                                tile_k as given or 8, tile_v 1, wg_per_cu 0)    */
+  int reserved;              /* SOR iterations per launch of the kernel that ran:
+                                2, or 0 for a launch per colour                 */
 } qesmc_result;
 
 typedef struct qesmc_ctx qesmc_ctx;
@@ -225,18 +228,24 @@ int qesmc_divergence_linf(qesmc_ctx *ctx, int physical, double *out);
 /* ---- batches and tuning --------------------------------------------------- */
 
 /* Solve n resident problems (one context each, same device, any sizes)
- * together: every SOR colour pass of all of them is one kernel launch, each
- * problem keeping its own stop test (the reference solves one domain per
- * Solver::solve; this has no counterpart there).  With use_graph != 0 the
- * iterations are replayed as a captured HIP graph of check_every iterations.
- * Per problem the results equal qesmc_run's; results[i] (optional) receives
- * them (their timings span the whole batch).  ms_loop (optional): device
- * time of the batched iterations.  Split path only.  One tiling serves the
- * whole batch: tile_v 1 or 2 and tile_k as given, else the most work per
- * wave tile (at most 4 planes x 2 half-cells) that leaves >= 6 wave tiles
- * per CU over all members; wg_per_cu as given, else 5 from 48 wave tiles
- * per CU up and qesmc_run's untuned choice below that.  Tilings autotuned
- * per context are not used. */
+ * together, each keeping its own stop test (the reference solves one domain
+ * per Solver::solve; this has no counterpart there).  Per problem the results
+ * equal qesmc_run's; results[i] (optional) receives them (their timings span
+ * the whole batch).  ms_loop (optional): device time of the batched iterations.
+ * Paths AUTO and SPLIT.
+ *
+ * AUTO without tile fields, every problem on a wall mask and with memory for
+ * the march's buffers: two iterations of all problems, or of a group of them
+ * whose arrays stay in the Infinity Cache, are one kernel launch
+ * (results[i].reserved 2).  Launched directly, whatever use_graph says.
+ *
+ * Otherwise every SOR colour pass of all problems is one kernel launch, and
+ * with use_graph != 0 the iterations are replayed as a captured HIP graph of
+ * check_every iterations.  One tiling serves the whole batch: tile_v 1 or 2
+ * and tile_k as given, else the most work per wave tile (at most 4 planes x 2
+ * half-cells) that leaves >= 6 wave tiles per CU over all members; wg_per_cu
+ * as given, else 5 from 55 wave tiles per CU up and qesmc_run's untuned
+ * choice below that.  Tilings autotuned per context are not used. */
 int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_result *results,
                     int use_graph, double *ms_loop);
 

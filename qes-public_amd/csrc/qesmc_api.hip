@@ -609,7 +609,7 @@ int run_finish(qesmc_ctx *x, const RunState &st, int launched, qesmc_result *res
     res->tile_k = x->kplanes;
     res->tile_v = x->tile_v;
     res->wg_per_cu = x->wg_per_cu;
-    res->reserved = 0;
+    res->reserved = st.march ? 2 : 0;
   }
   return rc;
 }

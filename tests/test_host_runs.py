@@ -228,6 +228,25 @@ def case_autotune_leaves_the_march_where_it_is_slower(Q, S):
             assert S.launches("k_sor_march") > 0
 
 
+def case_results_tell_what_ran(Q, S):
+    """qesmc_result.reserved: SOR iterations per launch, 0 for a launch per colour."""
+    with flat_city(Q, 40, 30, 20) as a, flat_city(Q, 50, 30, 20) as b:
+        for kw, per in ((dict(), 2), (dict(path=Q.PATH_FUSED), 2), (dict(tile_v=2), 0), (dict(path=Q.PATH_SPLIT), 0),
+                        (dict(path=Q.PATH_PLAIN), 0)):
+            S.reset()
+            r = a.run(itermax=6, **kw)
+            assert r["reserved"] == per and (S.launches("k_sor_march") > 0) == (per == 2), kw
+        for kw, per in ((dict(), 2), (dict(tile_k=2), 0), (dict(path=Q.PATH_SPLIT), 0)):
+            for g in (False, True):
+                res, _ = Q.run_batch([a, b], itermax=6, check_every=6, use_graph=g, **kw)
+                assert [r["reserved"] for r in res] == [per] * 2, kw
+    S.reset()
+    with flat_city(Q, 60, 30, 20) as c:
+        c.run(itermax=2, path=Q.PATH_SPLIT)
+        S.fail_at(1)
+        assert c.run(itermax=6)["reserved"] == 0
+
+
 CASES = sorted(n for n in globals() if n.startswith("case_"))
 
 
