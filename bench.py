@@ -778,18 +778,10 @@ def reference_schedule(ctx, params, steps, warmup):
     return time.perf_counter() - t0, results
 
 
-def marches(path, tiles, compressed):
-    """Whether a run takes two iterations per launch: any wall-mask geometry
-    unless a path or a tiling of the colour passes is asked for."""
-    if path == Q.PATH_FUSED:
-        return True
-    return path == Q.PATH_AUTO and bool(compressed) and not any(tiles.values())
-
-
 def roofline_of(results, lups_per_iteration, workload_key, iterations_per_launch=None):
     """Roofline object of the dominant SOR kernel from the run's own HIP-event
     timings: achieved = algorithmic bytes per launch / mean launch time.  With
-    iterations_per_launch = 2 (the march) a launch's 13 bytes per cell serve
+    iterations_per_launch = 2 (the march; qesmc_result.reserved) a launch's 13 bytes per cell serve
     two updates of it, 6.5 bytes each; where the arrays fit the Infinity
     Cache the march is bound by the caches and its vector ALUs."""
     last = results[-1]
@@ -851,7 +843,7 @@ def city400_leg(path, tiles, steps=5, warmup=1):
         grad_ms = min(ctx.velocity_gradient(uniform_z=False, copy=False)[1] for _ in range(3))
     its = results[-1]["iterations"]
     roof, ms_sor = roofline_of(results, city.interior_lups(), "city400x400x120",
-                               2 if marches(path, tiles, results[-1]["compressed"]) else None)
+                               results[-1]["reserved"] or None)
     return {"workload": desc, "steps": steps, "t_ref_ms": round(wall / steps * 1e3, 3), "sor_ms": round(ms_sor, 3),
             "glups": round(city.interior_lups() * its * steps / wall / 1e9, 3), "div_linf_ref_operator": div_ref,
             "velocity_gradient": {"ms": round(grad_ms, 4), "bytes_per_cell": 52,
@@ -933,7 +925,7 @@ def main():
     its = results[-1]["iterations"]
     last = results[-1]
     roof, ms_sor = roofline_of(results, lups_it, "city1000x1000x150",
-                               2 if marches(path, tiles, last["compressed"]) else None)
+                               last["reserved"] or None)
     glups = lups_it * its * a.steps / wall / 1e9
     out = {
         "metric": METRIC,
