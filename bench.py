@@ -953,7 +953,27 @@ def main():
     }
     print(f"headline: {out['value']} GLUPS, {out['ms_per_step']} ms per solve", file=sys.stderr, flush=True)
     run_legs(a, legs, out, path, tiles, (lups_it / (cpu["value"] * 1e6)) if cpu else None)
-    print(json.dumps(out))
+    print(bench_line(out))
+
+
+LEG_KEYS = ("city1000_tol", "city400", "time_to_tol", "batch")
+
+
+def bench_line(out):
+    """The line for the record: the headline whole, of each leg its numbers
+    and those of its parts.  The legs in full go to stderr, a line each: with
+    them the line is 11 KB and more, of which a log keeps the end."""
+    def numbers(d):
+        return {k: float("%.5g" % v) if isinstance(v, float) else v for k, v in d.items()
+                if isinstance(v, (bool, int, float))}
+
+    for key in LEG_KEYS:
+        if key in out:
+            leg = out[key]
+            print("leg %s: %s" % (key, json.dumps(leg)), file=sys.stderr, flush=True)
+            parts = {k: numbers(v) for k, v in leg.items() if isinstance(v, dict)}
+            out = dict(out, **{key: dict(numbers(leg), **{k: v for k, v in parts.items() if v})})
+    return json.dumps(out)
 
 
 def run_legs(a, legs, out, path, tiles, cpu_ms_per_it):
