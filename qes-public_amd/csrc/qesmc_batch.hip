@@ -393,7 +393,7 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
   // with the least expected time.
   struct Group {
     int begin, end;  // members
-    int shape[2], slots[2], which[2];
+    int shape[2], tiles[2], which[2];
     std::vector<MarchPlan> plans;  // for two iterations a launch
   };
   std::vector<Group> groups;
@@ -442,9 +442,9 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
           gr.which[T - 1] = (int)which.size();
           for (int i = 0; i < m; ++i) {
             MarchItem &it = mitems[(size_t)(T - 1) * n + gr.begin + i];
-            qesmc_march_item(ctxs[gr.begin + i], T == 1 ? single[(size_t)i] : gr.plans[(size_t)i], gr.slots[T - 1], it);
-            which.insert(which.end(), (size_t)it.slots, gr.begin + i);
-            gr.slots[T - 1] += it.slots;
+            qesmc_march_item(ctxs[gr.begin + i], T == 1 ? single[(size_t)i] : gr.plans[(size_t)i], gr.tiles[T - 1], it);
+            which.insert(which.end(), (size_t)it.ntiles, gr.begin + i);
+            gr.tiles[T - 1] += it.ntiles;
           }
         }
       }
@@ -506,7 +506,7 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
       }
     };
     auto launch_march = [&](const Group &gr, int iters, int t, int src, bool fix) -> hipError_t {
-      if (gr.slots[iters - 1] == 0) return hipSuccess;
+      if (gr.tiles[iters - 1] == 0) return hipSuccess;
       MarchRun run{};
       for (float &w : run.om) w = p.omega;
       run.tol = p.tol;
@@ -516,7 +516,7 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
       run.fix = fix ? 1 : 0;
       run.items = d_march + (size_t)(iters - 1) * n;
       run.which = reinterpret_cast<const int *>(d_march + 2 * (size_t)n) + gr.which[iters - 1];
-      return qesmc_launch_march_batch(bs, iters, gr.shape[iters - 1], gr.slots[iters - 1], run);
+      return qesmc_launch_march_batch(bs, iters, gr.shape[iters - 1], gr.tiles[iters - 1], run);
     };
     // iterations [t, t + count) by twos, reading buffer set src & 1 first
     auto march_chunk = [&](int t, int count, int src) -> hipError_t {

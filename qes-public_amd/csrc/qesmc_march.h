@@ -13,7 +13,7 @@ struct MarchItem {
   Dims d;
   int nq, nyt;  // x tiles, y tiles
   int ntiles;
-  int first, slots;     // its work-groups of the launch: slots (>= ntiles) from first, multiples of 8
+  int first;            // its work-groups of the launch: ntiles from here
   float2 *set0, *set1;  // lambda, the two buffer sets
   const float2 *R;
   const unsigned *mask;

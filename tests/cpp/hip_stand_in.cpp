@@ -17,7 +17,7 @@
 namespace {
 
 constexpr size_t kLargest = (size_t)64 << 20;  // copies and fills beyond this are left out
-constexpr int kNames = 1024, kLog = 1 << 20, kBlocks = 4096;
+constexpr int kNames = 1024, kLog = 1 << 20, kBlocks = 16384;
 
 struct Name {
   const void *host;
@@ -25,7 +25,11 @@ struct Name {
 };
 Name g_names[kNames];
 int g_nnames = 0;
-int g_log[kLog];
+struct Launch {
+  int name;
+  unsigned grid;
+};
+Launch g_log[kLog];
 int g_nlog = 0;
 struct Block {
   char *p;
@@ -144,8 +148,15 @@ void stand_in_cost(const char *kernel, double us)  // of a launch whose name hol
 int stand_in_launches(const char *kernel)
 {
   int n = 0;
-  for (int q = 0; q < g_nlog; ++q) n += std::strstr(g_names[g_log[q]].name, kernel) != nullptr;
+  for (int q = 0; q < g_nlog; ++q) n += std::strstr(g_names[g_log[q].name].name, kernel) != nullptr;
   return n;
+}
+
+int stand_in_grid(const char *kernel)  // work-groups along x of its last launch
+{
+  for (int q = g_nlog; q-- > 0;)
+    if (std::strstr(g_names[g_log[q].name].name, kernel)) return (int)g_log[q].grid;
+  return 0;
 }
 
 // ---- the runtime ------------------------------------------------------------
@@ -173,13 +184,13 @@ int __hipPopCallConfiguration(dim3s *g, dim3s *b, size_t *shm, void **stream)
   *stream = g_config.stream;
   return 0;
 }
-int hipLaunchKernel(const void *f, dim3s, dim3s, void **, size_t, void *)
+int hipLaunchKernel(const void *f, dim3s grid, dim3s, void **, size_t, void *)
 {
   std::lock_guard<std::recursive_mutex> lock(g_mu);
   for (int q = 0; q < g_nnames; ++q)
     if (g_names[q].host == f) {
       if (!g_capturing) {
-        if (g_nlog < kLog) g_log[g_nlog++] = q;
+        if (g_nlog < kLog) g_log[g_nlog++] = {q, grid.x};
         g_clock += g_slow && std::strstr(g_names[q].name, g_slow) ? g_slow_cost : 1.0;
       }
       return 0;

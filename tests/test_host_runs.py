@@ -32,6 +32,9 @@ class StandIn:
     def launches(self, kernel):
         return self.lib.stand_in_launches(kernel.encode())
 
+    def grid(self, kernel):
+        return self.lib.stand_in_grid(kernel.encode())
+
     def cost(self, kernel, us):
         self.lib.stand_in_cost(kernel.encode(), us)
 
@@ -272,6 +275,16 @@ def case_copies_of_memory_the_runtime_knows(Q, S):
         assert take((0, 1, 2)) == 3
         assert take(()) > 12
         assert 13 < take((1,))
+
+
+def case_small_members_fill_the_chip(Q, S):
+    """Work-groups go to the XCDs in turn: members of a few tiles follow each
+    other without gaps (padded to whole eighths, all went to one XCD)."""
+    ctxs = [flat_city(Q, 10, 10, 10) for _ in range(32)]
+    Q.run_batch(ctxs, itermax=16, check_every=16)
+    assert 32 <= S.grid("k_sor_march") < 8 * 32
+    for c in ctxs:
+        c.close()
 
 
 CASES = sorted(n for n in globals() if n.startswith("case_"))
