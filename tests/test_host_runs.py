@@ -287,6 +287,17 @@ def case_small_members_fill_the_chip(Q, S):
         c.close()
 
 
+def case_batch_replay_of_colour_passes(Q, S):
+    """use_graph replays the colour passes of a batch of wall-mask problems."""
+    ctxs = [flat_city(Q, 40 + q, 30, 20) for q in range(3)]
+    Q.run_batch(ctxs, itermax=8, check_every=8, use_graph=True, path=Q.PATH_SPLIT)
+    assert S.value("graph_launches") == 1 and S.launches("k_sor_batch") == 0
+    Q.run_batch(ctxs, itermax=8, check_every=8, use_graph=True)
+    assert S.value("graph_launches") == 1 and S.launches("k_sor_march") > 0
+    for c in ctxs:
+        c.close()
+
+
 CASES = sorted(n for n in globals() if n.startswith("case_"))
 
 
