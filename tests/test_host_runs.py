@@ -287,6 +287,18 @@ def case_small_members_fill_the_chip(Q, S):
         c.close()
 
 
+def case_batch_beyond_the_cache_is_taken_in_groups(Q, S):
+    """Each group has its own launches: two of two iterations, and the one that
+    redoes an end inside a launch."""
+    from test_gpu_batch_groups import GROUPS, SIZES
+
+    ctxs = [flat_city(Q, *s) for s in SIZES]
+    Q.run_batch(ctxs, itermax=4, check_every=4)
+    assert S.launches("k_sor_march") == 3 * GROUPS
+    for c in ctxs:
+        c.close()
+
+
 def case_batch_replay_of_colour_passes(Q, S):
     """use_graph replays the colour passes of a batch of wall-mask problems."""
     ctxs = [flat_city(Q, 40 + q, 30, 20) for q in range(3)]
