@@ -88,6 +88,13 @@ void dfree2(float **p)
   p[1] = nullptr;
 }
 
+// h_poll: two polling rows and status words, then room for the march's table
+// of highest walls (up to 1450 x 1450 cells; a pinned allocation costs 0.1 ms,
+// which every new domain would pay)
+constexpr int kPollWords = 2 * qesmc::kErrSlots + 8, kTopWords = 16384;
+
+int *own_top(const qesmc_ctx *x) { return reinterpret_cast<int *>(x->h_poll + kPollWords); }
+
 void free_march(qesmc_ctx *x)
 {
   dfree2(x->d_lc2);
@@ -95,7 +102,7 @@ void free_march(qesmc_ctx *x)
   dfree(x->d_canon8);
   dfree(x->d_mask2);
   dfree(x->d_top);
-  if (x->h_top) (void)hipHostFree(x->h_top);
+  if (x->h_top && x->h_top != own_top(x)) (void)hipHostFree(x->h_top);
   x->h_top = nullptr;
   x->pair_masks = false;
 }
@@ -110,7 +117,8 @@ hipError_t alloc_march(qesmc_ctx *x)
   if (e == hipSuccess) e = dalloc(&x->d_mask2, (long long)((d.NY + 1) / 2) * d.HP * d.NZ);
   const long long top = qesmc_march_top_words(d);
   if (e == hipSuccess) e = dalloc(&x->d_top, top);
-  if (e == hipSuccess) e = hipHostMalloc((void **)&x->h_top, sizeof(int) * (size_t)top, hipHostMallocDefault);
+  if (top <= kTopWords) x->h_top = own_top(x);
+  else if (e == hipSuccess) e = hipHostMalloc((void **)&x->h_top, sizeof(int) * (size_t)top, hipHostMallocDefault);
   if (e == hipSuccess) {
     try {
       x->march_cost.resize((size_t)d.NZ + 4);
@@ -319,7 +327,7 @@ int qesmc_create(qesmc_ctx **out, int device)
   // the no-allocation entry point's per-device scratch address (errors are
   // reported by qesmc_run_static itself, which repeats the lookup)
   (void)qesmc::static_scratch_init(device);
-  if (fail(hipHostMalloc((void **)&x->h_poll, (2 * qesmc::kErrSlots + 8) * sizeof(unsigned), hipHostMallocDefault))) goto bad;
+  if (fail(hipHostMalloc((void **)&x->h_poll, (kPollWords + kTopWords) * sizeof(unsigned), hipHostMallocDefault))) goto bad;
   if (fail(dalloc(&x->d_status, qesmc::kStatusWords))) goto bad;
   if (fail(dalloc(&x->d_norm, 1))) goto bad;
   *out = x;
