@@ -73,7 +73,8 @@ typedef struct qesmc_fields {
                                  tile fields tile the colour passes (where the
                                  colour arrays exceed the 256 MB Infinity Cache
                                  they do not apply, as on FUSED),
-                                 qesmc_autotune found these faster, or the
+                                 qesmc_autotune found these faster, the domain
+                                 is a thin tower of 1200 planes or more, or the
                                  march's buffers cannot be had (no memory, or
                                  not yet allocated in a qesmc_run_static call);
                                  else SPLIT.  Whole iterations per launch are

@@ -38,6 +38,7 @@ hipError_t qesmc_fused_prepare(qesmc_ctx *x);
 long long qesmc_march_top_words(const qesmc::Dims &d);
 void qesmc_march_costs(qesmc_ctx *x);
 void qesmc_march_choose(qesmc_ctx *x, int tile_k);
+bool qesmc_march_too_thin(const qesmc::Dims &d);
 
 namespace {
 
@@ -455,7 +456,8 @@ int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, BatchKind ba
   // The march (two iterations per launch) runs wherever it can: on every wall
   // mask below 2^31 half-cells whose planes its 32-bit byte offsets reach.
   // QESMC_PATH_AUTO takes it unless the caller tiles the colour passes, the
-  // autotuner found them faster, or a no-allocation run finds its buffers missing.  Where
+  // autotuner found them faster, a no-allocation run finds its buffers missing,
+  // or the domain is too thin a tower to gain.  Where
   // the colour arrays (lambda and R of both colours, the masks) exceed
   // MI355X's 256 MB Infinity Cache, AUTO is the fused path, as which it is
   // reported, and the tile fields of the colour passes do not apply to it.
@@ -469,7 +471,7 @@ int run_prepare(qesmc_ctx *x, const qesmc_params *pp, RunState &st, BatchKind ba
   const int march_tile_k = tuned ? 0 : p.tile_k;
   st.march = batch != BatchKind::colours && fits && x->d.splane < (1LL << 28) && x->d.NZ < 32768 &&
              (p.path == QESMC_PATH_FUSED || batch == BatchKind::march ||
-              (p.path == QESMC_PATH_AUTO && (beyond || untiled) && !x->colours_faster &&
+              (p.path == QESMC_PATH_AUTO && (beyond || (untiled && !qesmc_march_too_thin(x->d))) && !x->colours_faster &&
                (!x->no_alloc_run || march_ready(x))));
   if (st.march && !march_ready(x)) {
     const hipError_t e = alloc_march(x);

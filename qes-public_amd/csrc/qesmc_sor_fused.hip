@@ -701,6 +701,18 @@ void qesmc_march_choose(qesmc_ctx *x, int tile_k)
   }
 }
 
+// Whether the domain is a tower on one column of tiles that is too thin to
+// march: a plan has at most 127 segments, which then grow with the height.
+// March / colour passes in us per iteration: 12x12 cells 1200 high 8.9 / 8.4,
+// 2500 12.6 / 10.3, 8000 29 / 16; 20x20 1500 9.7 / 10.1, 2500 12.8 / 12.4,
+// 8000 32 / 17; 60x30 2500 16 / 21, 8000 39 / 42.
+bool qesmc_march_too_thin(const Dims &d)
+{
+  int nq, nyt;
+  march_columns(d, 2, kBatchShape, &nq, &nyt);
+  return nq * nyt == 1 && 5LL * (d.NZ - 700) > 16LL * d.NX * d.NY;
+}
+
 hipError_t qesmc_fused_prepare(qesmc_ctx *x)
 {
   hipLaunchKernelGGL(k_march_tables, dim3((unsigned)x->d.NZ), dim3(64), 0, x->stream, x->d.NZ, x->d_canon,

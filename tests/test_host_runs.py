@@ -310,6 +310,14 @@ def case_batch_replay_of_colour_passes(Q, S):
         c.close()
 
 
+def case_thin_towers_take_the_colour_passes(Q, S):
+    for dims, march in (((12, 12, 1000), True), ((12, 12, 1300), False), ((20, 20, 1900), True), ((20, 20, 2100), False),
+                        ((60, 30, 2500), True), ((100, 30, 2500), True)):
+        with flat_city(Q, *dims) as c:
+            assert c.run(itermax=4)["reserved"] == (2 if march else 0), dims
+            assert c.run(itermax=4, path=Q.PATH_FUSED)["reserved"] == 2
+
+
 CASES = sorted(n for n in globals() if n.startswith("case_"))
 
 
