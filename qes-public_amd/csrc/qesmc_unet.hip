@@ -494,6 +494,20 @@ __device__ __forceinline__ uint2 transpose16(uint2 raw, short4v ident)
   return r;
 }
 
+// One channel's operand: voxels x..x+3 and x+16..x+19 of a row of dx, moved
+// by `shift`; 0 outside it or without `in`.
+__device__ __forceinline__ bf16x8 gather16(const bf16_t *v, int ld, bool in, long long row, int x, int shift, int dx)
+{
+  unsigned w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int at = x + 16 * (e >> 2) + (e & 3), from = at + shift;
+    const unsigned h = in && at < dx && from >= 0 && from < dx ? v[(row + from) * ld] : 0u;
+    w[e >> 1] |= h << (16 * (e & 1));
+  }
+  return as_bf16x8(make_uint4(w[0], w[1], w[2], w[3]));
+}
+
 __global__ __launch_bounds__(256, 2) void k_conv_wgrad(ConvWgradArgs a)
 {
   __shared__ float sum[27 * 256];
@@ -577,6 +591,49 @@ __global__ __launch_bounds__(256, 2) void k_conv_wgrad(ConvWgradArgs a)
             acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(G[1 - oy][1 - oz], X[ox + 1], acc[t], 0, 0, 0);
           }
     }
+  }
+  // An infinity or a NaN makes the identity product's other terms NaN: it would
+  // reach all 16 channels of its tile.  Any in a strip has left a NaN in the
+  // wave's sums; the wave then takes its strips again with operands gathered a
+  // channel at a time (the same voxels in the same order), and with the products that
+  // a gradient at the border has with the zeros beyond it, which are then NaN.
+  // probe: 0, or NaN where any sum is not finite.
+  float probe = 0.f;
+#pragma unroll
+  for (int t = 0; t < 27; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) probe += 0.f * acc[t][i];
+  if (__builtin_amdgcn_ballot_w64(!(probe == 0.f)) != 0) {
+    // three taps at a time, so that little is held besides the sums
+#pragma unroll
+    for (int oz = -1; oz <= 1; ++oz)
+#pragma unroll
+      for (int oy = -1; oy <= 1; ++oy) {
+        f32x4 *const three = acc + (oz + 1) * 9 + (oy + 1) * 3;
+        three[0] = three[1] = three[2] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int strip = (int)blockIdx.x * 4 + wave; strip < strips; strip += (int)gridDim.x * 4) {
+          const int xt = strip % nxt, ys = strip / nxt % nys, z = strip / (nxt * nys);
+          const int x0 = 32 * xt, y0 = ys * a.ylen, y1 = y0 + a.ylen < a.dy ? y0 + a.ylen : a.dy;
+          // the strip's rows of X, and the rows of zeros beside them where it lies at the border
+          const int za = z == 0 ? -1 : z, zb = z == a.dz - 1 ? a.dz : z;
+          const int ya = y0 == 0 ? -1 : y0, yb = y1 == a.dy ? a.dy : y1 - 1;
+#pragma unroll 1
+          for (int row = 0; row < (zb - za + 1) * (yb - ya + 1); ++row) {
+            const int zz = za + row / (yb - ya + 1), yy = ya + row % (yb - ya + 1);
+            const int gz = zz - oz, gy = yy - oy;
+            if (gz < 0 || gz >= a.dz || gy < 0 || gy >= a.dy) continue;
+            const bool in = zz >= 0 && zz < a.dz && yy >= 0 && yy < a.dy && c0 + r < a.cin;
+            const bf16x8 G = gather16(a.g + n0 + r, a.ldg, true, ((long long)gz * a.dy + gy) * a.dx, x0 + 4 * oct, 0, a.dx);
+#pragma unroll
+            for (int ox = -1; ox <= 1; ++ox) {
+              const bf16x8 X = gather16(a.x + c0 + r, a.ldx, in, ((long long)zz * a.dy + yy) * a.dx, x0 + 4 * oct, ox, a.dx);
+              three[ox + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(G, X, three[ox + 1], 0, 0, 0);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          }
+        }
+      }
   }
   // lane holds D[n0 + 4*oct + i][c0 + r] of every tap
   for (int w = 0; w < 4; ++w) {
