@@ -1243,8 +1243,10 @@ hipError_t launch_conv_fwd(hipStream_t s, const ConvFwdArgs &a)
                        dim3(256), 0, s, a);
     return hipGetLastError();
   };
-  // a lane's offset within a brick's six planes has 31 bits in a buffer load
-  const bool wide = 12LL * a.dy * a.dx * a.ldx >= 0x7fffffffLL;
+  // A lane's offset from the halo's first voxel has 31 bits in a buffer load.
+  // The halo's last voxel is at most a row of it (kHaloX) beyond six planes, and 32
+  // bytes of it are read.
+  const bool wide = (6LL * a.dy * a.dx + kHaloX) * 2 * a.ldx + 32 > 0x7fffffffLL;
   switch (conv_kind(a.cin, a.dx, a.dy, a.dz)) {
   case ConvKind::chunks8: return wide ? chunks(k_conv_chunks<8, true>) : chunks(k_conv_chunks<8, false>);
   case ConvKind::chunks16: return wide ? chunks(k_conv_chunks<16, true>) : chunks(k_conv_chunks<16, false>);

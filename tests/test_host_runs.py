@@ -318,6 +318,18 @@ def case_thin_towers_take_the_colour_passes(Q, S):
             assert c.run(itermax=4, path=Q.PATH_FUSED)["reserved"] == 2
 
 
+def case_convolutions_at_31_bits(Q, S):
+    """A brick's last voxel lies up to 17 voxels beyond six planes: with 48
+    channels that passes 31 bits at 1864134 x 2 voxels, whose six planes
+    (2147482368 bytes) do not, and there the offsets have 64."""
+    for dx, wide in ((1864134, 1), (1864128, 0)):
+        S.reset()
+        net = Q.UNet(dx, 2, 6, levels=2, base_channels=16, seed=1)
+        net.forward(np.zeros((6, 2, dx, 8), np.float32))
+        assert S.launches("k_conv_chunksILi16ELb1E") == wide, (dx, S.launches("k_conv_chunks"))
+        net.close()
+
+
 CASES = sorted(n for n in globals() if n.startswith("case_"))
 
 
