@@ -283,7 +283,7 @@ int qesmc_run_batch(qesmc_ctx **ctxs, int n, const qesmc_params *params, qesmc_r
   }
   // The march (two iterations per launch) where no tiling of the colour passes
   // is asked for and every member has a wall-mask encoding: 16 cities of
-  // 64-256 cells a side (29.6 M cells) relax in 70 us per iteration instead of 112.
+  // 64-256 cells a side (29.6 M cells) relax in 67 us per iteration instead of 112.
   bool march = params->path == QESMC_PATH_AUTO && params->tile_k == 0 && params->tile_v == 0 && params->wg_per_cu == 0;
   if (!(params->flags & QESMC_RUN_REENCODE))
     for (int i = 0; i < n; ++i) march = march && ctxs[i]->compressible;

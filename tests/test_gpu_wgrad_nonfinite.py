@@ -54,6 +54,6 @@ def test_other_channels_are_untouched(qesmc, where, dims):
     others = [np.delete(a, Q, axis=axis) for a in out]
     assert np.isfinite(others[0]).all() and np.abs(others[0]).max() > 0
     assert not np.isfinite(np.take(infinite, Q, axis=axis)).any()
-    # at most 16 work-groups' sums in any order: their roundings, 2^-24 each
+    # up to 34 work-groups' sums in any order: their roundings, 2^-24 each in either run
     assert np.isfinite(others[1]).all()
-    assert np.abs(others[1] - others[0]).max() <= 16 * 2.0 ** -23 * np.abs(others[0]).max()
+    assert np.abs(others[1] - others[0]).max() <= 34 * 2.0 ** -23 * np.abs(others[0]).max()
