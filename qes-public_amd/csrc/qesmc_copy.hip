@@ -12,8 +12,10 @@
 // copies itself, at the link's rate: u, v, w of 400 x 400 x 120 cells into pinned
 // arrays take 4.15 ms so and 5.30 through the slots.
 //
-// The slots belong to the process: one set per device, made by the first large
-// copy, lent to one call at a time (a call that finds it lent takes the
+// The slots belong to the process: one set per device, made once the large
+// copies since they were last freed amount to 64 MiB (making and freeing them takes
+// 3.6 ms, which 13 MB of a context that then goes do not repay: set-up, run, copy and
+// close of 128 x 128 x 64 cells took 5.2 ms without them and 9.1 with), lent to one call at a time (a call that finds it lent takes the
 // runtime's copy) and freed with the device's last context.
 #include <atomic>
 #include <cstring>
@@ -36,12 +38,14 @@ constexpr size_t kLeastChunk = (size_t)1 << 20;
 // pages to fault in, reaches 31 GB/s.
 constexpr size_t kLeastToHost = (size_t)8 << 20;
 constexpr size_t kLeastToDevice = (size_t)128 << 20;
+constexpr size_t kRepay = (size_t)64 << 20;
 constexpr int kMaxDevices = 64;
 
 struct Slots {
   std::mutex mu;
   int contexts = 0;
   bool lent = false;
+  size_t without = 0;  // bytes of large copies made without the slots, while there are none
   void *pinned[kSlots] = {};
   hipEvent_t done[kSlots] = {};  // the slot's last copy over the link
   hipStream_t stream = nullptr;
@@ -59,13 +63,16 @@ void free_slots(Slots &s)
   }
   if (s.stream) (void)hipStreamDestroy(s.stream);
   s.stream = nullptr;
+  s.without = 0;
 }
 
-// The device's slots, made if need be; false if they are lent or cannot be had.
-bool borrow(Slots &s)
+// The device's slots for a copy of `bytes`, made if need be; false if they are
+// lent, do not repay yet or cannot be had.
+bool borrow(Slots &s, size_t bytes)
 {
   std::lock_guard<std::mutex> lock(s.mu);
   if (s.lent) return false;
+  if (!s.stream && (s.without += bytes) < kRepay) return false;
   bool ok = s.stream || hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) == hipSuccess;
   for (int q = 0; q < kSlots && ok; ++q) {
     ok = (s.pinned[q] || hipHostMalloc(&s.pinned[q], kSlotBytes, hipHostMallocDefault) == hipSuccess) &&
@@ -161,7 +168,7 @@ hipError_t host_copy(int device, hipStream_t st, const HostPiece *p, int n, bool
     return plain(st, p, n, to_device);
   }
   Slots &s = g_slots[device];
-  if (!borrow(s)) return plain(st, p, n, to_device);
+  if (!borrow(s, total)) return plain(st, p, n, to_device);
   hipError_t first = hipSuccess;
   for (int q = 0; q < n && first == hipSuccess; ++q)
     if (known(p[q].host)) first = queue(st, p[q], to_device);

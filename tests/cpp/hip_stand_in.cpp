@@ -40,7 +40,7 @@ Block g_blocks[kBlocks];
 std::recursive_mutex g_mu;
 
 long long g_fail_at = 0, g_fail_above = 0, g_fail_new = 0;  // 0: never
-long long g_device_allocs = 0, g_host_allocs = 0, g_live = 0;
+long long g_device_allocs = 0, g_host_allocs = 0, g_live = 0, g_host_live = 0;
 std::atomic<long long> g_news{0};
 thread_local bool g_count_news = false;
 long long g_syncs = 0, g_graph_launches = 0, g_copies = 0;
@@ -70,7 +70,7 @@ int allocate(void **p, size_t bytes, bool device)
     if (!b.p) {
       b = {(char *)std::calloc(bytes ? bytes : 1, 1), bytes, device};
       if (!b.p) return 2;
-      if (device) g_live += (long long)bytes;
+      (device ? g_live : g_host_live) += (long long)bytes;
       *p = b.p;
       return 0;
     }
@@ -83,7 +83,7 @@ int release(void *p)
   std::lock_guard<std::recursive_mutex> lock(g_mu);
   for (Block &b : g_blocks)
     if (b.p == p) {
-      if (b.device) g_live -= (long long)b.bytes;
+      (b.device ? g_live : g_host_live) -= (long long)b.bytes;
       std::free(b.p);
       b = {};
       return 0;
@@ -136,7 +136,7 @@ void stand_in_news(int count, long long fail_at)                  // this thread
 }
 long long stand_in_value(int what)
 {
-  const long long v[] = {g_device_allocs, g_host_allocs, g_live, g_news.load(), g_syncs, g_graph_launches, g_copies};
+  const long long v[] = {g_device_allocs, g_host_allocs, g_live, g_news.load(), g_syncs, g_graph_launches, g_copies, g_host_live};
   return v[what];
 }
 void stand_in_cost(const char *kernel, double us)  // of a launch whose name holds `kernel` (others 1)

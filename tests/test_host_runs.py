@@ -44,7 +44,7 @@ class StandIn:
 
     def value(self, what):
         return self.lib.stand_in_value(
-            ("device_allocs", "host_allocs", "live", "news", "syncs", "graph_launches", "copied").index(what))
+            ("device_allocs", "host_allocs", "live", "news", "syncs", "graph_launches", "copied", "host_live").index(what))
 
 
 def flat_city(Q, ncx, ncy, ncz):
@@ -257,7 +257,8 @@ def case_copies_of_memory_the_runtime_knows(Q, S):
     with flat_city(Q, 200, 200, 60) as c:
         c.run(itermax=2)
         n = c.city.nface
-        u, v, w = c.get_velocity()  # makes the slots
+        for _ in range(4):
+            c.get_velocity()  # makes the slots
 
         def take(pinned):
             out = [np.full(n, 7.0, np.float32) for _ in range(3)]
@@ -328,6 +329,36 @@ def case_convolutions_at_31_bits(Q, S):
         net.forward(np.zeros((6, 2, dx, 8), np.float32))
         assert S.launches("k_conv_chunksILi16ELb1E") == wide, (dx, S.launches("k_conv_chunks"))
         net.close()
+
+
+def case_slots_are_made_once_they_repay(Q, S):
+    """A context that copies little and goes is not worth the pinned slots; one
+    that copies on, or much, makes them, and the last to go frees them."""
+    slots = 12
+
+    def held():
+        return S.value("host_live")
+
+    for _ in range(8):  # 13 MB each, one context after another
+        with flat_city(Q, 128, 128, 64) as c:
+            before = held()
+            c.get_velocity()
+            assert held() == before
+    with flat_city(Q, 128, 128, 64) as c:
+        before = held()
+        made = []
+        for _ in range(8):
+            c.get_velocity()
+            made.append((held() - before) // (4 << 20))
+        assert made[0] == 0 and made[-1] == slots and sorted(made) == made, made
+        with flat_city(Q, 40, 30, 20):
+            pass
+        assert held() - before == slots * (4 << 20)
+    assert held() < 4 << 20
+    with flat_city(Q, 300, 300, 80) as c:  # 90 MB at once
+        before = held()
+        c.get_velocity()
+        assert held() - before == slots * (4 << 20)
 
 
 CASES = sorted(n for n in globals() if n.startswith("case_"))
