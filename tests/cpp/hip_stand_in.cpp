@@ -43,7 +43,8 @@ long long g_fail_at = 0, g_fail_above = 0, g_fail_new = 0;  // 0: never
 long long g_device_allocs = 0, g_host_allocs = 0, g_live = 0, g_host_live = 0;
 std::atomic<long long> g_news{0};
 thread_local bool g_count_news = false;
-long long g_syncs = 0, g_graph_launches = 0, g_copies = 0;
+std::atomic<long long> g_syncs{0}, g_copies{0};
+long long g_graph_launches = 0;
 bool g_capturing = false;
 double g_clock = 0.0;
 const char *g_slow = nullptr;
@@ -123,8 +124,8 @@ void stand_in_reset()
   std::lock_guard<std::recursive_mutex> lock(g_mu);
   g_nlog = 0;
   g_fail_at = g_fail_above = g_fail_new = 0;
-  g_device_allocs = g_host_allocs = g_syncs = g_graph_launches = 0;
-  g_news = 0;
+  g_device_allocs = g_host_allocs = g_graph_launches = 0;
+  g_news = g_syncs = 0;
 }
 void stand_in_fail_at(long long n) { g_fail_at = n; }             // the n-th device allocation from here
 void stand_in_fail_above(long long bytes) { g_fail_above = bytes; }  // device allocations beyond this size
@@ -136,7 +137,8 @@ void stand_in_news(int count, long long fail_at)                  // this thread
 }
 long long stand_in_value(int what)
 {
-  const long long v[] = {g_device_allocs, g_host_allocs, g_live, g_news.load(), g_syncs, g_graph_launches, g_copies, g_host_live};
+  const long long v[] = {g_device_allocs, g_host_allocs, g_live, g_news.load(), g_syncs.load(),
+                         g_graph_launches, g_copies.load(), g_host_live};
   return v[what];
 }
 void stand_in_cost(const char *kernel, double us)  // of a launch whose name holds `kernel` (others 1)
